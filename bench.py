@@ -13,8 +13,9 @@ with), then the W warm-up steps.
 
 Prints one JSON line.  `roofline` is computed for the fused stream-collide
 kernel from its average duration, measured with HIP events on the library's
-own stream; algorithmic bytes are 240 B per lattice update (15 x 8 B read +
-15 x 8 B written) in FP64 and 120 B in FP32-shifted storage.
+own stream; algorithmic bytes are 240 B per cell and launch (15 x 8 B read +
+15 x 8 B written) in FP64 and 120 B in FP32-shifted storage.  On lattices of
+this size a launch advances two steps (`updates_per_launch`).
 """
 import argparse
 import json
@@ -99,7 +100,15 @@ def measure(ctx, dims, mgs, tau, rho, u, precision, steps, warmup, keep_fields=F
     wall = t1 - t0
     avg_ms = kern_ms / launches if launches else float("nan")
     achieved = BYTES_PER_LU[precision] * cells / (avg_ms * 1e-3) / 1e9
+    storage = "double" if precision == lbx.LBX_FP64 else "float"
+    wall_arg = "" if all(periodic) else ", walls"
+    if launches and 2 * launches <= steps + 1 and steps > 1:
+        kernel = f"k_step_pair<{storage}{wall_arg}>"
+    else:
+        kernel = f"k_step_{'f64' if precision == lbx.LBX_FP64 else 'f32s'}<STEP_FUSED{wall_arg}>"
     return {
+        "kernel": kernel,
+        "updates_per_launch": steps / launches if launches else float("nan"),
         "boxes": len(boxes),
         "mlups": cells * steps / wall / 1e6,
         "ms_per_step": wall * 1e3 / steps,
@@ -530,7 +539,7 @@ def main():
             walls = {"workload": f"{n}^3, {rw['boxes']} boxes of {args.max_grid_size}^3, tau {tau}, halfway "
                                  "bounce-back walls on both z faces (x, y periodic)",
                      "periodic": [1, 1, 0], "steps": args.walls_steps, "mlups": rw["mlups"],
-                     "ms_per_step": rw["ms_per_step"], "kernel": "k_step_f64<STEP_FUSED, walls>",
+                     "ms_per_step": rw["ms_per_step"], "kernel": rw["kernel"], "updates_per_launch": rw["updates_per_launch"],
                      "kernel_avg_ms": rw["kernel_avg_ms"], "kernel_gbs": rw["kernel_gbs"],
                      "frac_of_hbm_peak": rw["kernel_gbs"] / HBM_PEAK_GBS,
                      "frac_of_copy_ceiling": rw["kernel_gbs"] / copy_gbs if copy_gbs else None,
@@ -619,7 +628,7 @@ def main():
                 f"({r32['kernel_gbs']:.0f} GB/s)")
 
     workload = f"{n}^3 periodic, {r64['boxes']} boxes of {args.max_grid_size}^3, tau {tau}"
-    kernel = "k_step_f64<STEP_FUSED>"
+    kernel = r64["kernel"]
     traffic = traffic_for(kernel, f"{n}^3")
     cells = n ** 3
     out = {
@@ -649,6 +658,7 @@ def main():
             "frac": round(r64["kernel_gbs"] / HBM_PEAK_GBS, 4),
             "traffic": traffic,
             "kernel": kernel,
+            "updates_per_launch": r64["updates_per_launch"],
             "kernel_avg_ms": round(r64["kernel_avg_ms"], 5),
             "algorithmic_bytes_per_launch": BYTES_PER_LU[lbx.LBX_FP64] * cells,
             "copy_ceiling_gbs": round(copy_gbs, 1) if copy_gbs else None,
@@ -664,8 +674,8 @@ def main():
             "speedup_vs_fp64": round(r32["mlups"] / r64["mlups"], 3),
             "roofline": {"bound": "hbm", "achieved": round(r32["kernel_gbs"], 1), "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": round(r32["kernel_gbs"] / HBM_PEAK_GBS, 4),
-                         "traffic": traffic_for("k_step_f32s<STEP_FUSED>", f"{n}^3"),
-                         "kernel": "k_step_f32s<STEP_FUSED>",
+                         "traffic": traffic_for(r32["kernel"], f"{n}^3"),
+                         "kernel": r32["kernel"], "updates_per_launch": r32["updates_per_launch"],
                          "kernel_avg_ms": round(r32["kernel_avg_ms"], 5),
                          "algorithmic_bytes_per_launch": BYTES_PER_LU[lbx.LBX_FP32_SHIFTED] * cells},
             "workgroup": {"bx": shape32[0], "by": shape32[1], "max_workgroups_per_cu": shape32[2]},

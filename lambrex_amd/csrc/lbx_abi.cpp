@@ -51,6 +51,7 @@ struct Level {
   int ratio = 2;         // refinement ratio to the parent (patched levels)
   std::vector<Box> boxes;
   Lattice lat{};         // level-array geometry (level 0)
+  lbx::PairShape pair{};  // two-step passes of a single-level simulation (tx = 0: none)
   void* buf[3] = {nullptr, nullptr, nullptr};  // state in buf[cur]; buf[2] scratch (patched)
   int cur = 0;
   // Level 0 of a single-level simulation between Iterate calls: buf[cur]
@@ -450,6 +451,19 @@ int launch_step(lbx_sim* sim, Level& L, lbx::StepKind kind) {
   return ps.close();
 }
 
+// Two fused steps of level 0 in one pass.
+int launch_pair(lbx_sim* sim, Level& L) {
+  lbx_ctx* ctx = sim->ctx;
+  const Relax r{L.omega_s, L.omega_b, sim->rho0};
+  ProfileScope ps(ctx, true);
+  if (ps.rc) return ps.rc;
+  const hipError_t e =
+      lbx::launch_step_pair(sim->precision, L.buf[L.cur], L.buf[1 - L.cur], L.lat, r, L.pair, ctx->stream);
+  if (e != hipSuccess) return hip_fail(ctx, e, "two-step launch");
+  L.cur = 1 - L.cur;
+  return ps.close();
+}
+
 // Bring level 0 back to the pre-collision populations f in place (the
 // stream-only pass) if it holds the post-collision state (Level::post).
 int materialise(lbx_sim* sim) {
@@ -751,6 +765,7 @@ int define_level0(lbx_sim* sim, const std::vector<Box>& boxes) {
   L.boxes = boxes;
   L.lat = lbx::make_lattice(sim->dims[0], sim->dims[1], sim->dims[2], (int)elem_size(sim->precision));
   L.lat.walls = sim->walls;
+  L.pair = lbx::pair_shape(L.lat, sim->precision);
   const size_t bytes = (size_t)L.lat.elems() * elem_size(sim->precision);
   for (int i = 0; i < 2; ++i) {
     hipError_t e = hipMalloc(&L.buf[i], bytes);
@@ -1596,17 +1611,20 @@ int lbx_iterate(lbx_sim* sim, int nsteps) {
   // Reference order per step is f <- S(C(f)).  Over n steps:
   //   f_n = S (C S)^(n-1) C f_0 = S g_n,  g_n = (C S)^(n-1) C f_0
   // so from f in place: one collide-only pass and n-1 fused pull+collide
-  // passes leave g_n (Level::post); from g: n fused passes.  The last S is
+  // steps leave g_n (Level::post); from g: n fused steps, two to a pass where
+  // the level has a pair shape.  The last S is
   // applied only when f is observed (a pull inside the readers, or the
   // stream-only pass of materialise()).  Per-cell arithmetic is unchanged,
   // so results are bit-identical to the reference order, and Iterate(a)
-  // then Iterate(b) is Iterate(a + b) pass for pass.
+  // then Iterate(b) is Iterate(a + b) step for step.
   int s = 0;
   if (!L.post) {
     if (int rc = launch_step(sim, L, lbx::STEP_COLLIDE)) return rc;
     L.post = true;
     s = 1;
   }
+  for (; L.pair.tx && s + 2 <= nsteps; s += 2)
+    if (int rc = launch_pair(sim, L)) return rc;
   for (; s < nsteps; ++s)
     if (int rc = launch_step(sim, L, lbx::STEP_FUSED)) return rc;
   return LBX_OK;

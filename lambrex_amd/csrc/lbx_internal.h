@@ -99,6 +99,18 @@ hipError_t launch_step_f64(StepKind kind, const double* src, double* dst, const 
 hipError_t launch_step_f32s(StepKind kind, const float* src, float* dst, const Lattice& L,
                             const Relax& r, LaunchShape s, hipStream_t st);
 
+// Two fused steps in one pass (k_step_pair): tx x ty columns of cells, each in
+// tz chunks of `depth` planes; tx = 0: not used for this lattice.
+struct PairShape {
+  int wide;  // columns of kPairWide cells, else kPairSquare
+  int tx, ty, tz, depth;
+};
+constexpr int kPairWide[2] = {64, 8};     // whole cache lines in x
+constexpr int kPairSquare[2] = {32, 16};  // smaller ring, less waste at ragged extents
+PairShape pair_shape(const Lattice& L, int precision);
+hipError_t launch_step_pair(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
+                            const PairShape& p, hipStream_t st);
+
 // Equilibrium of a region from device rho[nz][ny][nx], u[3][nz][ny][nx].
 hipError_t launch_equilibrium(int precision, void* f, const Lattice& L, const Region& R,
                               const double* rho, const double* u, double rho0, hipStream_t st);

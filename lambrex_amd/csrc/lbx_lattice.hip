@@ -69,7 +69,8 @@ __device__ constexpr int opposite(int q) {
 // Pull with halfway bounce-back: population q of cell (x, y, z) comes from
 // x - c_q, unless that crosses a wall face (an axis with its bit in
 // L.walls), where the cell's own opposite population, which left towards
-// the wall, returns instead.  Periodic axes wrap as in load_cell.
+// the wall, returns instead.  Periodic axes wrap as in load_cell.  ONCE: no
+// other workgroup reads the same elements (non-temporal loads).
 template <typename S>
 __device__ __forceinline__ void load_cell_walls(const S* __restrict__ src, const Lattice& L, int x, int y,
                                                 int z, long long selfz, int selfp, const Upstream& u, S* f) {
@@ -144,6 +145,156 @@ __global__ __launch_bounds__(512) void k_step_f32s(const float* __restrict__ src
   if (KIND != STEP_STREAM)
     collide_f32_shifted(f, float(r.rho0), float(r.omega_s), float(r.omega_b));
   store_cell<float>(dst, L, selfz, selfp, f);
+}
+
+// Two fused steps in one pass over the state: h'' = C(S(C(S(h)))).  One step
+// alone moves 240 B (FP64) per update and runs at the copy rate (256^3 FP64:
+// 652 us a step), so only a pass that keeps the state between two steps on
+// the chip is faster.  A workgroup owns a BX x BY column of cells and walks
+// its z-planes: it computes the first step of each plane over the column and
+// a ring of one cell (redundantly with its neighbours), hands the plane over
+// in LDS, and forms the second step of the plane below, whose populations
+// with c_z = -1 come from this plane, those with c_z = 0 and +1 from the two
+// planes before (carried in registers).  Two LDS planes alternate, so a
+// plane costs one barrier; the loads of the next plane are in flight while
+// this one is collided.  Each cell's arithmetic is that of two single
+// passes, so the results are the same bits.
+//
+// Bound: what the ring adds (64 x 8: 1.29 x the first-step collisions, but
+// only 1.07 x the reads beyond L2, the rest hits there since each XCD takes
+// a contiguous range of columns) and, with one workgroup of 11 waves per CU
+// (LDS, and ~150 VGPRs in FP64), the part of the collisions that the loads
+// do not cover; in FP32 the vector units are busy 90 % of the time.
+// Measured (us per step, single pass -> pair): 256^3 FP64 652 -> 445, FP32
+// 328 -> 264; 128^3 FP64 88 -> 52, FP32 42.5 -> 28.4.  Slower: 32 x 8 and
+// 64 x 4 columns with two workgroups per CU (540), separate waves for the
+// two steps (470), non-temporal loads (564, the ring misses L2).
+constexpr int pair_threads(int bx, int by) { return ((bx + 2) * (by + 2) + 63) / 64 * 64; }
+
+template <typename S>
+__device__ __forceinline__ void collide_any(S* f, const Relax& r) {
+  if constexpr (sizeof(S) == 8)
+    collide_f64(f, r.omega_s, r.omega_b);
+  else
+    collide_f32_shifted(f, float(r.rho0), float(r.omega_s), float(r.omega_b));
+}
+
+// The faces (x low, x high, y low, ...: bits 0 to 5) through which population
+// q can enter a cell.
+__device__ constexpr unsigned wall_faces(int q) {
+  unsigned m = 0;
+  for (int d = 0; d < 3; ++d) m |= kC[q][d] > 0 ? 1u << 2 * d : kC[q][d] < 0 ? 2u << 2 * d : 0u;
+  return m;
+}
+
+// The x and y faces with walls that cell (x, y, .) touches.
+__device__ __forceinline__ unsigned lateral_faces(int x, int y, const Lattice& L) {
+  unsigned m = 0;
+  if (L.walls & 1u) m |= (x == 0 ? 1u : 0u) | (x == L.nx - 1 ? 2u : 0u);
+  if (L.walls & 2u) m |= (y == 0 ? 4u : 0u) | (y == L.ny - 1 ? 8u : 0u);
+  return m;
+}
+
+template <typename S, int BX, int BY, bool WALLS>
+__global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __restrict__ src,
+                                                                    S* __restrict__ dst, Lattice L, Relax r,
+                                                                    PairShape p) {
+  constexpr int WX = BX + 2, NC = WX * (BY + 2);
+  __shared__ S ring[2][NV][NC];
+  // XCD k takes the k-th eighth of the columns (consecutive workgroups go
+  // to the 8 XCDs in turn; the grid is a multiple of 8)
+  const int w = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (w >= p.tx * p.ty * p.tz) return;
+  const int x0 = (w % p.tx) * BX, y0 = (w / p.tx % p.ty) * BY, z0 = w / (p.tx * p.ty) * p.depth;
+  const int z1 = min(z0 + p.depth, L.nz);
+  const int t = threadIdx.x;
+
+  // first step: cell t of the ring, its periodic image in the domain
+  const bool first = t < NC;
+  const int rx = (x0 - 1 + (first ? t % WX : 0) + L.nx) % L.nx, ry = (y0 - 1 + (first ? t / WX : 0) + L.ny) % L.ny;
+  const Upstream u = upstream(rx, ry, 0, L);
+  // second step: cell (ox, oy) of the column
+  const int ox = x0 + t % BX, oy = y0 + t / BX;
+  const bool second = t < BX * BY && ox < L.nx && oy < L.ny;
+  const int self = oy * L.nx + ox;
+  const int mid = (t / BX + 1) * WX + t % BX + 1;
+
+  // wall faces that a cell touches in x and y, and those that plane z lies on,
+  // as a mask of wall_faces(); a population that comes from behind one of
+  // them is the cell's own opposite population
+  const unsigned first_faces = WALLS ? lateral_faces(rx, ry, L) : 0, second_faces = WALLS ? lateral_faces(ox, oy, L) : 0;
+  auto z_faces = [&](int z) { return (L.walls & 4u) ? (z == 0 ? 16u : 0u) | (z == L.nz - 1 ? 32u : 0u) : 0u; };
+
+  auto load = [&](int z, S* f) {
+    z = z < 0 ? z + L.nz : z >= L.nz ? z - L.nz : z;
+    const S* zs[3] = {src + (z == L.nz - 1 ? 0 : z + 1) * L.zs, src + z * L.zs,
+                      src + (z == 0 ? L.nz - 1 : z - 1) * L.zs};
+    const unsigned faces = WALLS ? first_faces | z_faces(z) : 0;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      const S* from = zs[1 + kC[q][2]] + q * L.ps;
+      unsigned at = u.ys[1 + kC[q][1]] + u.xs[1 + kC[q][0]];
+      if (WALLS && (faces & wall_faces(q))) {
+        from = zs[1] + opposite(q) * L.ps;
+        at = u.ys[1] + u.xs[1];
+      }
+      f[q] = from[at];
+    }
+  };
+
+  S next[NV];   // first step's populations of the coming plane
+  S keep1[NV];  // second step of the coming plane: c_z = 0 and +1
+  S keep2[NV];  // ... of the plane after it: c_z = +1
+  S back[NV];   // walls: what the coming plane's c_z = -1 populations bounce to
+#pragma unroll
+  for (int q = 0; q < NV; ++q) next[q] = keep1[q] = keep2[q] = back[q] = S(0);
+  if (first) load(z0 - 1, next);
+  for (int z = z0 - 1; z <= z1; ++z) {
+    S(*plane)[NC] = ring[z & 1];
+    if (first) {
+      S f[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) f[q] = next[q];
+      if (z < z1) load(z + 1, next);
+      collide_any(f, r);
+#pragma unroll
+      for (int q = 0; q < NV; ++q) plane[q][t] = f[q];
+    }
+    __syncthreads();
+    if (second) {
+      S f[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) {
+        const S v = plane[q][mid - kC[q][1] * WX - kC[q][0]];
+        if (kC[q][2] < 0) {
+          f[q] = v;
+        } else {
+          f[q] = keep1[q];
+          keep1[q] = kC[q][2] == 0 ? v : keep2[q];
+          if (kC[q][2] > 0) keep2[q] = v;
+        }
+      }
+      if constexpr (WALLS) {
+        // the plane just formed is the own plane of the next second step:
+        // its bounced populations return from this cell
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+          if (kC[q][2] < 0) {
+            if ((second_faces | z_faces(z - 1)) & wall_faces(q)) f[q] = back[q];
+            back[q] = plane[opposite(q)][mid];
+          } else if ((second_faces | z_faces(z)) & wall_faces(q)) {
+            keep1[q] = plane[opposite(q)][mid];
+          }
+        }
+      }
+      if (z > z0) {
+        collide_any(f, r);
+        S* out = dst + (z - 1) * L.zs + self;
+#pragma unroll
+        for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], out + q * L.ps);
+      }
+    }
+  }
 }
 
 dim3 grid_of(const Lattice& L, LaunchShape s) {
@@ -453,6 +604,69 @@ hipError_t launch_step_f64(StepKind kind, const double* src, double* dst, const 
 hipError_t launch_step_f32s(StepKind kind, const float* src, float* dst, const Lattice& L,
                             const Relax& r, LaunchShape s, hipStream_t st) {
   LBX_STEP_LAUNCH(k_step_f32s, src, dst);
+}
+
+// Shape of the two-step pass for a lattice, or none (p.tx = 0) where two
+// single passes are the faster.  Every workgroup count that fills the device
+// for one or more rounds is a candidate: rounds x (planes of a workgroup + 2
+// of the ring + 1 to start) x the time of a plane, measured as 6.8 us (FP64)
+// and 4.1 us (FP32) at 256^3 and 4.4 and 2.8 us where both buffers stay in
+// the 256 MB MALL.  A single pass is taken at 5.3 TB/s.  At 64^3 the rule
+// takes the pair in FP64 (10.3 against 12.4 us a step) and not in FP32 (6.9
+// against 5.9); at 48^3 in neither (7.1 against 6.4, 5.6 against 4.7); at
+// 96x80x72 in both (19.5 against 25.7, 12.6 against 12.9).
+PairShape pair_shape(const Lattice& L, int precision) {
+  static const int cus = [] {
+    int dev = 0, n = 256;
+    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    return n < 1 ? 256 : n;
+  }();
+  PairShape best{};
+  const double bytes = double(L.elems()) * (precision == 0 ? 8 : 4);
+  const bool mall = 2 * bytes <= 256e6;
+  const double plane_us = precision == 0 ? (mall ? 4.4 : 6.8) : (mall ? 2.8 : 4.1);
+  double best_us = 2 * (2 * bytes / 5.3e6);  // two single passes
+  for (int wide = 1; wide >= 0; --wide) {
+    const int bx = wide ? kPairWide[0] : kPairSquare[0], by = wide ? kPairWide[1] : kPairSquare[1];
+    const long long tx = (L.nx + bx - 1) / bx, ty = (L.ny + by - 1) / by;
+    if (tx * ty > (1 << 20)) continue;
+    for (int chunks = 1; 2 * chunks <= L.nz || chunks == 1; ++chunks) {
+      const int depth = (L.nz + chunks - 1) / chunks;
+      const long long n = tx * ty * ((L.nz + depth - 1) / depth);
+      const long long rounds = (n + cus - 1) / cus;
+      const double us = double(rounds) * (depth + 3) * plane_us;
+      if (us < best_us) {
+        best_us = us;
+        best = PairShape{wide, (int)tx, (int)ty, (L.nz + depth - 1) / depth, depth};
+      }
+      if (rounds > 16) break;  // deeper splits only add ring planes
+    }
+  }
+  return best;
+}
+
+template <typename S>
+static hipError_t step_pair(const S* src, S* dst, const Lattice& L, const Relax& r, const PairShape& p,
+                            hipStream_t st) {
+  constexpr int wx = kPairWide[0], wy = kPairWide[1], qx = kPairSquare[0], qy = kPairSquare[1];
+  const unsigned grid = unsigned(((long long)p.tx * p.ty * p.tz + 7) / 8 * 8);
+  const bool walls = L.walls != 0;
+  if (p.wide && walls)
+    k_step_pair<S, wx, wy, true><<<grid, pair_threads(wx, wy), 0, st>>>(src, dst, L, r, p);
+  else if (p.wide)
+    k_step_pair<S, wx, wy, false><<<grid, pair_threads(wx, wy), 0, st>>>(src, dst, L, r, p);
+  else if (walls)
+    k_step_pair<S, qx, qy, true><<<grid, pair_threads(qx, qy), 0, st>>>(src, dst, L, r, p);
+  else
+    k_step_pair<S, qx, qy, false><<<grid, pair_threads(qx, qy), 0, st>>>(src, dst, L, r, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_step_pair(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
+                            const PairShape& p, hipStream_t st) {
+  if (p.tx < 1) return hipErrorInvalidValue;
+  if (precision == 0) return step_pair((const double*)src, (double*)dst, L, r, p, st);
+  return step_pair((const float*)src, (float*)dst, L, r, p, st);
 }
 
 hipError_t launch_equilibrium(int precision, void* f, const Lattice& L, const Region& R,
