@@ -52,7 +52,7 @@ struct Level {
   std::vector<Box> boxes;
   Lattice lat{};         // level-array geometry (level 0)
   lbx::PairShape pair{};  // two-step passes of a single-level simulation (tx = 0: none)
-  void* buf[3] = {nullptr, nullptr, nullptr};  // state in buf[cur]; buf[2] scratch (patched)
+  void* buf[3] = {nullptr, nullptr, nullptr};  // state in buf[cur]; buf[2] scratch (patched, ratio above 2)
   int cur = 0;
   // Level 0 of a single-level simulation between Iterate calls: buf[cur]
   // holds the post-collision state g of the last step, and the reference's
@@ -74,34 +74,32 @@ struct Level {
   // patched levels: ghost fill sources and the average-down contributions
   // into the parent; d_mask is then one byte per grown cell (the parent's
   // view of this level's own finer level)
-  long long* d_fill = nullptr;
+  long long* d_fill = nullptr;     // at ratio 2 in the form of lbx::FineStep::fill
+  unsigned* d_strides = nullptr;   // ... its strides, if they differ
   long long grown_cells = 0;        // length of the fill table
   long long* d_sum_cell = nullptr;  // level-array parent: its element per touched cell
   int* d_sum_start = nullptr;
   int* d_sum_contrib = nullptr;  // index into the block averages, per contribution
   int sum_ncell = 0;
-  // patched parent: touched-cell index per grown cell of the parent (-1 if
-  // none), for the parent's fused stream + sum
-  int* d_sum_slot = nullptr;
+  // patched parent: per grown cell of the parent, its contributions (the first
+  // in the high 32 bits, their number in the low ones; -1 if none)
+  long long* d_sum_span = nullptr;
   // Patches are stored in the buffers in `gdesc` order (box corners, x
-  // fastest), whatever order the caller gave the boxes in, and the finest
-  // level's substep pair runs over `groups` of consecutive ones there (about
-  // kFineGroupBytes of one buffer each), so a group is a compact set of
-  // neighbouring boxes.  gdesc holds copies of desc's entries in that order.
-  // With `regions` the array between the two substeps lives in one region of
-  // buf[2] per stream (region_span elements).
+  // fastest), whatever order the caller gave the boxes in, so consecutive
+  // ones are neighbours.  gdesc holds copies of desc's entries in that order.
+  // At ratio 2 a step is one launch over `tiles` of the patches; above it the
+  // passes of a step run over `groups` of consecutive patches (about
+  // kFineGroupBytes of one buffer each) and need buf[2] between them.
   std::vector<PatchDesc> gdesc;
   PatchDesc* d_gdesc = nullptr;
   std::vector<std::pair<int, int>> groups;  // (first position in gdesc, count)
-  long long region_span = 0;
-  bool regions = false;
+  lbx::FineTile* d_tiles = nullptr;
+  int ntiles = 0;
   double* d_avg = nullptr;       // 15 planes of avg_stride 2x2x2 block averages
   long long avg_stride = 0;
   int max_blocks = 0;            // largest (g/2)^3 of a patch
 };
 
-// One captured level-0 step of a hierarchy per (level-0 parity, finest-level
-// parity).
 // Captured level-0 steps, one per combination of the levels' buffer
 // parities at the start of the step (bit l = level l's `cur`).
 struct StepGraphs {
@@ -244,11 +242,13 @@ void free_level(Level& L) {
   if (L.d_desc) (void)hipFree(L.d_desc);
   if (L.d_mask) (void)hipFree(L.d_mask);
   if (L.d_fill) (void)hipFree(L.d_fill);
+  if (L.d_strides) (void)hipFree(L.d_strides);
   if (L.d_sum_cell) (void)hipFree(L.d_sum_cell);
   if (L.d_sum_start) (void)hipFree(L.d_sum_start);
   if (L.d_sum_contrib) (void)hipFree(L.d_sum_contrib);
-  if (L.d_sum_slot) (void)hipFree(L.d_sum_slot);
+  if (L.d_sum_span) (void)hipFree(L.d_sum_span);
   if (L.d_gdesc) (void)hipFree(L.d_gdesc);
+  if (L.d_tiles) (void)hipFree(L.d_tiles);
   if (L.d_avg) (void)hipFree(L.d_avg);
   L = Level{};
 }
@@ -485,165 +485,145 @@ void free_levels_from(lbx_sim* sim, int level) {
   for (int l = level; l < LBX_MAX_LEVELS; ++l) free_level(sim->lev[l]);
 }
 
-// The kernels of one level-0 step of the Rohde cycle (src/AmrSim.cpp:430-469)
-// for the current buffer parities.
-// The finest level's patches run in groups of about kFineGroupBytes of state
-// (one buffer), alternating over two streams: two groups' intermediate
-// arrays (≈ 2 x 2 x 48 MB) then stay in the 256 MB MALL.
+// Above ratio 2 a level's patches run in groups of about kFineGroupBytes of
+// state (one buffer), alternating over two streams: two groups' intermediate
+// arrays (~ 2 x 2 x 48 MB) then stay in the 256 MB MALL between the passes.
 constexpr long long kFineGroupBytes = 48ll << 20;
 
-// The finest level's substeps (two at ratio 2, r at ratio r), from its
-// parent's current state (level 0's `now`, or a middle level's state, which
-// its own step rewrites only after this).  Its block averages land in
-// F.d_avg.  par[l] is the buffer holding level l's state while the step is
-// enqueued; the finest level's flips.
-hipError_t enqueue_finest_pair(lbx_sim* sim, int f, int* par, hipStream_t st) {
-  Level& F = sim->lev[f];
-  const Level& C = sim->lev[f - 1];
-  const int prec = sim->precision;
-  const Relax rf{F.omega_s, F.omega_b, sim->rho0};
-  int& fpar = par[f];
-  const void* cnow = C.buf[par[f - 1]];
-  void* fnow = F.buf[fpar];
-  void* fnext = F.buf[1 - fpar];
-  void* ftmp = F.buf[2];
-  const PatchDesc* cpatches = C.patched ? C.d_desc : nullptr;
-  // The fine patches' two substeps depend on no other patch's substeps (the
-  // ghosts are filled once, from fnow and cnow), so they run in the level's
-  // groups of neighbouring patches, whose arrays stay in the MALL between
-  // the passes.  Groups write disjoint patches (and block sums), so
-  // consecutive groups alternate between the context's stream and its side
-  // stream, forked from and joined back to `st` around the loop; one group's
-  // launch ramp then overlaps the other's tail.  The array between the
-  // substeps is dead once its group ends: with F.regions each stream
-  // rewrites one region of buf[2] for it (the group's patches are
-  // contiguous, patch p at p.base - base(first)) while its lines are still
-  // in the MALL, instead of writing each group's back to HBM.  The groups
-  // run in storage order when fpar is 0 and in reverse order when it is 1,
-  // so each pair starts with the groups whose state the previous pair wrote
-  // last, while it may still be in the MALL.
-  lbx_ctx* ctx = sim->ctx;
-  const auto& groups = F.groups;
-  const size_t ng = groups.size();
-  const bool fork = ng > 1, rev = fpar == 1;
+// The arguments of level l's step at ratio 2 (launch_fine_step); the child's
+// block averages are added on a level that has one.  par[l] is the buffer
+// holding level l's state while the step is enqueued.
+lbx::FineStep fine_step_args(const lbx_sim* sim, int l, bool finest, bool average, const int* par) {
+  const Level& L = sim->lev[l];
+  const Level& P = sim->lev[l - 1];
+  lbx::FineStep a{};
+  a.finest = finest;
+  a.now = L.buf[par[l]];
+  a.next = L.buf[1 - par[l]];
+  a.parent = P.buf[par[l - 1]];
+  a.own = L.d_gdesc;
+  a.tiles = L.d_tiles;
+  a.ntiles = L.ntiles;
+  a.fill = (const unsigned long long*)L.d_fill;
+  a.strides = L.d_strides;
+  a.parent_stride = P.patched ? P.gdesc[0].qs : P.lat.ps;
+  a.mask = L.d_mask;
+  a.relax = Relax{L.omega_s, L.omega_b, sim->rho0};
+  if (average) {
+    a.avg = L.d_avg;
+    a.avg_stride = L.avg_stride;
+  }
+  if (!finest) {
+    const Level& F = sim->lev[l + 1];
+    a.spans = F.d_sum_span;
+    a.cavg = F.d_avg;
+    a.cavg_stride = F.avg_stride;
+    a.contrib = F.d_sum_contrib;
+  }
+  return a;
+}
+
+// Runs `pass(first, count, stream)` for each of a level's groups, alternating
+// between `st` and the context's side stream, which is forked from and joined
+// back to `st`: the groups write disjoint patches, so one group's launch ramp
+// overlaps the other's tail.
+template <typename Pass>
+hipError_t over_groups(lbx_ctx* ctx, const Level& L, hipStream_t st, Pass pass) {
+  const bool fork = L.groups.size() > 1;
   hipError_t e = hipSuccess;
   if (fork) {
     e = hipEventRecord(ctx->fork_ev, st);
     if (e == hipSuccess) e = hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0);
   }
-  for (size_t k = 0; k < ng && e == hipSuccess; ++k) {
-    const auto& grp = groups[rev ? ng - 1 - k : k];
-    const int first = grp.first, n = grp.second;
-    hipStream_t gs = (k & 1) ? ctx->side : st;
-    void* mid = ftmp;
-    long long shift = 0;
-    if (F.regions) {
-      mid = static_cast<char*>(ftmp) + (k & 1) * F.region_span * elem_size(prec);
-      shift = F.gdesc[first].base;
-    }
-    if (F.ratio == 2) {
-      e = lbx::launch_fine_fill_collide(prec, fnow, fnext, cnow, C.lat, cpatches, F.d_desc, F.d_gdesc, first, n,
-                                        F.max_cells, F.d_fill, nullptr, rf, gs);
-      if (e == hipSuccess)
-        e = lbx::launch_fine_stream_collide(prec, fnext, mid, shift, F.d_gdesc, first, n, F.max_cells, rf, gs);
-      if (e == hipSuccess)
-        e = lbx::launch_fine_stream_avg(prec, mid, shift, fnext, F.d_avg, F.avg_stride, F.d_gdesc, first, n,
-                                        F.max_blocks, sim->rho0, gs);
-    } else {
-      // ratio r > 2: r substeps, each a collide then a stream, chained
-      // through buf[2] (whole, no regions) and fnext so that the last one
-      // reads buf[2]: the fill-collide writes stage 1, the k-th
-      // stream-collide reads stage k and writes stage k+1, stage k in buf[2]
-      // when r - k is even; then the last stream into fnext and the
-      // average-down of its valid cells.
-      const int r = F.ratio;
-      auto stage = [&](int k) { return ((r - k) % 2 == 0) ? mid : fnext; };
-      e = lbx::launch_fine_fill_collide(prec, fnow, stage(1), cnow, C.lat, cpatches, F.d_desc, F.d_gdesc, first, n,
-                                        F.max_cells, F.d_fill, nullptr, rf, gs);
-      for (int k = 1; k < r && e == hipSuccess; ++k)
-        e = lbx::launch_fine_stream_collide(prec, stage(k), stage(k + 1), 0, F.d_gdesc, first, n, F.max_cells, rf, gs,
-                                            k > 1);
-      if (e == hipSuccess)
-        e = lbx::launch_fine_stream_valid(prec, mid, fnext, F.d_gdesc, first, n, F.max_cells, sim->rho0, gs);
-      if (e == hipSuccess)
-        e = lbx::launch_fine_avg_valid(prec, fnext, F.d_avg, F.avg_stride, F.d_gdesc, first, n, F.max_blocks, r,
-                                       sim->rho0, gs);
-    }
-  }
+  for (size_t k = 0; k < L.groups.size() && e == hipSuccess; ++k)
+    e = pass(L.groups[k].first, L.groups[k].second, (k & 1) ? ctx->side : st);
   if (fork) {  // join even after a failed launch, so a capture can end
     const hipError_t ej = hipEventRecord(ctx->join_ev, ctx->side);
     const hipError_t ew = ej == hipSuccess ? hipStreamWaitEvent(st, ctx->join_ev, 0) : ej;
     if (e == hipSuccess) e = ew;
   }
-  fpar = 1 - fpar;
+  return e;
+}
+
+// The finest level's substeps of one step of its parent (two at ratio 2, r at
+// ratio r), from its own and its parent's current states (level 0's `now`, or
+// a middle level's state, which its own step rewrites only after this).  Its
+// block averages land in F.d_avg; the level's buffer flips.
+hipError_t enqueue_finest(lbx_sim* sim, int f, int* par, hipStream_t st) {
+  Level& F = sim->lev[f];
+  const Level& C = sim->lev[f - 1];
+  const int prec = sim->precision, r = F.ratio;
+  hipError_t e;
+  if (r == 2) {
+    e = lbx::launch_fine_step(prec, fine_step_args(sim, f, true, true, par), st);
+  } else {
+    // r substeps, each a collide then a stream, chained through buf[2] and
+    // fnext so that the last one reads buf[2]: the fill-collide writes stage
+    // 1, the k-th stream-collide reads stage k and writes stage k+1, stage k
+    // in buf[2] when r - k is even; then the last stream into fnext and the
+    // average-down of its valid cells.
+    const Relax rf{F.omega_s, F.omega_b, sim->rho0};
+    const void* cnow = C.buf[par[f - 1]];
+    const PatchDesc* cpatches = C.patched ? C.d_desc : nullptr;
+    void* fnow = F.buf[par[f]];
+    void* fnext = F.buf[1 - par[f]];
+    void* mid = F.buf[2];
+    auto stage = [&](int k) { return ((r - k) % 2 == 0) ? mid : fnext; };
+    e = over_groups(sim->ctx, F, st, [&](int first, int n, hipStream_t gs) {
+      hipError_t g = lbx::launch_fine_fill_collide(prec, fnow, stage(1), cnow, C.lat, cpatches, F.d_desc, F.d_gdesc,
+                                                   first, n, F.max_cells, F.d_fill, nullptr, rf, gs);
+      for (int k = 1; k < r && g == hipSuccess; ++k)
+        g = lbx::launch_fine_stream_collide(prec, stage(k), stage(k + 1), F.d_gdesc, first, n, F.max_cells, rf, gs,
+                                            k > 1);
+      if (g == hipSuccess)
+        g = lbx::launch_fine_stream_valid(prec, mid, fnext, F.d_gdesc, first, n, F.max_cells, sim->rho0, gs);
+      if (g == hipSuccess)
+        g = lbx::launch_fine_avg_valid(prec, fnext, F.d_avg, F.avg_stride, F.d_gdesc, first, n, F.max_blocks, r,
+                                       sim->rho0, gs);
+      return g;
+    });
+  }
+  par[f] = 1 - par[f];
   return e;
 }
 
 hipError_t enqueue_children(lbx_sim* sim, int l, int finest, int* par, hipStream_t st);
 
 // One step of a middle level m (0 < m < finest), RohdeCycle(m): the finer
-// levels' steps, which read m's state; then, per group of m's patches, the
-// two-level fill from the parent with comp 0 zeroed on the outer layer and
-// the masked collide, and Stream + ZeroInvalidComponents with SumFromFine
-// added into the valid cells (one fused kernel) into m's other buffer,
-// which becomes its state.  The reference collides before the finer levels'
-// steps; the collide reads only m's and its parent's current states, which
-// those steps do not change, so it can follow them, and m's passes then run
-// in the same MALL-sized groups as the finest level's (the array between
-// the two in a group-sized region of buf[2] per stream, consecutive groups
-// on two streams): the fill of a group reads the neighbours' current state,
-// which no group overwrites.  In the last of its parent's r steps (`last`)
-// the block averages of the result for the parent are formed too: in the
-// same pass at ratio 2, where they include 2 fine ghost layers, or by a pass
-// over the valid cells above it (nGrow = 2 / r = 0).
+// levels' steps, which read m's state; then the two-level fill from the
+// parent with comp 0 zeroed on the outer layer, the masked collide, and
+// Stream + ZeroInvalidComponents with SumFromFine added into the valid cells,
+// into m's other buffer, which becomes its state.  The reference collides
+// before the finer levels' steps; the collide reads only m's and its parent's
+// current states, which those steps do not change, so it can follow them.  In
+// the last of its parent's r steps (`last`) the block averages of the result
+// for the parent are formed too: in the same pass at ratio 2, where they
+// include 2 fine ghost layers, or by a pass over the valid cells above it
+// (nGrow = 2 / r = 0).
 hipError_t enqueue_middle_step(lbx_sim* sim, int m, int finest, int* par, hipStream_t st, bool last) {
   Level& L = sim->lev[m];
   const Level& P = sim->lev[m - 1];
   const Level& F = sim->lev[m + 1];
   const int prec = sim->precision;
-  const Relax r{L.omega_s, L.omega_b, sim->rho0};
   hipError_t e = enqueue_children(sim, m, finest, par, st);
   if (e != hipSuccess) return e;
-  void* now = L.buf[par[m]];
-  void* next = L.buf[1 - par[m]];
-  const void* pnow = P.buf[par[m - 1]];
-  lbx_ctx* ctx = sim->ctx;
-  const auto& groups = L.groups;
-  const bool fork = groups.size() > 1;
-  if (fork) {
-    e = hipEventRecord(ctx->fork_ev, st);
-    if (e == hipSuccess) e = hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0);
-  }
-  for (size_t k = 0; k < groups.size() && e == hipSuccess; ++k) {
-    const int first = groups[k].first, n = groups[k].second;
-    hipStream_t gs = (k & 1) ? ctx->side : st;
-    void* mid = L.buf[2];
-    long long shift = 0;
-    if (L.regions) {
-      mid = static_cast<char*>(L.buf[2]) + (k & 1) * L.region_span * elem_size(prec);
-      shift = L.gdesc[first].base;
-    }
-    e = lbx::launch_fine_fill_collide(prec, now, mid, pnow, P.lat, P.patched ? P.d_desc : nullptr, L.d_desc,
-                                      L.d_gdesc, first, n, L.max_cells, L.d_fill, L.d_mask, r, gs, shift);
-    if (e == hipSuccess && last && L.ratio != 2) {
-      e = lbx::launch_fine_stream_zero(prec, mid, next, L.d_gdesc, first, n, L.max_cells, sim->rho0, F.d_sum_slot,
-                                       F.d_avg, F.avg_stride, F.d_sum_start, F.d_sum_contrib, gs, shift);
-      if (e == hipSuccess)
-        e = lbx::launch_fine_avg_valid(prec, next, L.d_avg, L.avg_stride, L.d_gdesc, first, n, L.max_blocks,
-                                       L.ratio, sim->rho0, gs);
-    } else if (e == hipSuccess && last) {  // the state the parent averages down: its block sums in the same pass
-      e = lbx::launch_middle_stream_avg(prec, mid, shift, next, L.d_avg, L.avg_stride, L.d_gdesc, first, n,
-                                        L.max_blocks, sim->rho0, F.d_sum_slot, F.d_avg, F.avg_stride, F.d_sum_start,
-                                        F.d_sum_contrib, gs);
-    } else if (e == hipSuccess) {
-      e = lbx::launch_fine_stream_zero(prec, mid, next, L.d_gdesc, first, n, L.max_cells, sim->rho0, F.d_sum_slot,
-                                       F.d_avg, F.avg_stride, F.d_sum_start, F.d_sum_contrib, gs, shift);
-    }
-  }
-  if (fork) {  // join even after a failed launch, so a capture can end
-    const hipError_t ej = hipEventRecord(ctx->join_ev, ctx->side);
-    const hipError_t ew = ej == hipSuccess ? hipStreamWaitEvent(st, ctx->join_ev, 0) : ej;
-    if (e == hipSuccess) e = ew;
+  if (L.ratio == 2) {
+    e = lbx::launch_fine_step(prec, fine_step_args(sim, m, false, last, par), st);
+  } else {
+    const Relax r{L.omega_s, L.omega_b, sim->rho0};
+    void* next = L.buf[1 - par[m]];
+    e = over_groups(sim->ctx, L, st, [&](int first, int n, hipStream_t gs) {
+      hipError_t g = lbx::launch_fine_fill_collide(prec, L.buf[par[m]], L.buf[2], P.buf[par[m - 1]], P.lat,
+                                                   P.patched ? P.d_desc : nullptr, L.d_desc, L.d_gdesc, first, n,
+                                                   L.max_cells, L.d_fill, L.d_mask, r, gs);
+      if (g == hipSuccess)
+        g = lbx::launch_fine_stream_zero(prec, L.buf[2], next, L.d_gdesc, first, n, L.max_cells, sim->rho0,
+                                         F.d_sum_span, F.d_avg, F.avg_stride, F.d_sum_contrib, gs);
+      if (g == hipSuccess && last)
+        g = lbx::launch_fine_avg_valid(prec, next, L.d_avg, L.avg_stride, L.d_gdesc, first, n, L.max_blocks, L.ratio,
+                                       sim->rho0, gs);
+      return g;
+    });
   }
   par[m] = 1 - par[m];
   return e;
@@ -654,13 +634,15 @@ hipError_t enqueue_middle_step(lbx_sim* sim, int m, int finest, int* par, hipStr
 // result (src/AmrSim.cpp:445-455).
 hipError_t enqueue_children(lbx_sim* sim, int l, int finest, int* par, hipStream_t st) {
   const int c = l + 1;
-  if (c == finest) return enqueue_finest_pair(sim, c, par, st);
+  if (c == finest) return enqueue_finest(sim, c, par, st);
   const int r = sim->lev[c].ratio;
   hipError_t e = hipSuccess;
   for (int k = 0; k < r && e == hipSuccess; ++k) e = enqueue_middle_step(sim, c, finest, par, st, k == r - 1);
   return e;
 }
 
+// The kernels of one level-0 step of the Rohde cycle (src/AmrSim.cpp:430-469)
+// for the current buffer parities.
 hipError_t enqueue_hierarchy_step(lbx_sim* sim, hipStream_t st) {
   Level& C = sim->lev[0];
   const Level& F = sim->lev[1];
@@ -825,6 +807,20 @@ long long grown_index(const PatchDesc& P, int x, int y, int z) {
   return ((long long)(z - P.lo[2] + 2) * P.g[1] + (y - P.lo[1] + 2)) * P.g[0] + (x - P.lo[0] + 2);
 }
 
+// Element of population 0 of grown cell `index` of patch P, which is stored.
+long long stored_element(const PatchDesc& P, long long index) {
+  const long long plane = (long long)P.g[0] * P.g[1];
+  return P.at((int)(index % P.g[0]), (int)(index % plane / P.g[0]), (int)(index / plane));
+}
+
+// A reference to a stored cell of level C from cell_ref's, as the remake
+// kernel takes it: elements from the patch's base instead of a grown index.
+long long stored_ref(const Level& C, long long ref) {
+  if (!C.patched) return ref;
+  const PatchDesc& P = C.desc[ref >> 32];
+  return (ref >> 32 << 32) | (stored_element(P, ref & 0xffffffffll) - P.base);
+}
+
 // Where a level keeps the valid cell at (x, y, z) of its own index space
 // (already wrapped into the domain): the element of population 0 in a level
 // array, or (patch << 32) | grown index on a patched level.  False if no
@@ -872,6 +868,98 @@ std::vector<unsigned char> patch_mask(const Level& C, const std::vector<Box>& ma
     }
   }
   return m;
+}
+
+// The k-th of n even-aligned parts of [0, g) (g even), as even as they can be.
+int part_begin(int g, int n, int k) { return 2 * (int)((long long)(g / 2) * k / n); }
+
+// Cuts patches into tiles for launch_fine_step.  Every patch is cut into parts
+// of at most `want` cells per direction; the target that costs least is taken:
+// rounds of workgroups over the CUs x planes a workgroup walks (its own and
+// up to 4 around them, and 2 of the pipeline) x time of a plane (2.5 us + 0.4
+// us per wave of its A plane, fitted to FP64 steps of 36^3 patches).  The
+// model only ranks the targets: of a sweep that forced each of them on 36^3
+// and 28^3 patches, none was faster than the one it takes by more than the
+// runs differed.
+std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches) {
+  std::map<std::tuple<int, int, int>, int> shapes;  // grown extents -> patches
+  int gmax[3] = {2, 2, 2};
+  for (const PatchDesc& p : patches) {
+    ++shapes[std::make_tuple(p.g[0], p.g[1], p.g[2])];
+    for (int d = 0; d < 3; ++d) gmax[d] = std::max(gmax[d], p.g[d]);
+  }
+  auto parts = [](int g, int want) { return (g + want - 1) / want; };
+  // the widest A extent of an axis cut into n parts
+  auto widest = [](int g, int n) {
+    int w = 0;
+    for (int k = 0; k < n; ++k)
+      w = std::max(w, std::min(part_begin(g, n, k + 1) + 2, g) - std::max(part_begin(g, n, k) - 2, 0));
+    return w;
+  };
+  int cus = 256, dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess)
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  int best[3] = {4, 4, gmax[2]};
+  double best_us = 1e300;
+  auto targets = [](int g) {
+    std::vector<int> t;
+    for (int n = 1; n <= 64; ++n) {
+      const int want = ((g + n - 1) / n + 1) / 2 * 2;
+      if (want >= 4 && (t.empty() || t.back() != want)) t.push_back(want);
+    }
+    if (t.empty()) t.push_back(g);
+    if (t.back() > 4) t.push_back(4);
+    return t;
+  };
+  const std::vector<int> tx = targets(gmax[0]), ty = targets(gmax[1]), tz = targets(gmax[2]);
+  for (int wx : tx)
+    for (int wy : ty) {
+      long long columns = 0;
+      int cells = 0;
+      for (const auto& s : shapes) {
+        const int gx = std::get<0>(s.first), gy = std::get<1>(s.first);
+        const int nx = parts(gx, wx), ny = parts(gy, wy);
+        cells = std::max(cells, widest(gx, nx) * widest(gy, ny));
+        columns += (long long)nx * ny * s.second;
+      }
+      if (cells > lbx::kFineTileCells || columns > (1 << 24)) continue;
+      const double plane_us = 2.5 + 0.4 * ((cells + 63) / 64);
+      for (int wz : tz) {
+        long long n = 0;
+        int planes = 0;
+        for (const auto& s : shapes) {
+          const int gz = std::get<2>(s.first), nz = parts(gz, wz);
+          n += (long long)parts(std::get<0>(s.first), wx) * parts(std::get<1>(s.first), wy) * nz * s.second;
+          planes = std::max(planes, widest(gz, nz) + 2);
+        }
+        const double us = (double)((n + cus - 1) / cus) * planes * plane_us;
+        if (n < (1 << 24) && us < best_us) {
+          best_us = us;
+          best[0] = wx;
+          best[1] = wy;
+          best[2] = wz;
+        }
+      }
+    }
+  std::vector<lbx::FineTile> tiles;
+  for (size_t p = 0; p < patches.size(); ++p) {
+    const int* g = patches[p].g;
+    int n[3];
+    for (int d = 0; d < 3; ++d) n[d] = parts(g[d], best[d]);
+    for (int c = 0; c < n[2]; ++c)
+      for (int b = 0; b < n[1]; ++b)
+        for (int a = 0; a < n[0]; ++a) {
+          lbx::FineTile t;
+          t.patch = (int)p;
+          const int at[3] = {a, b, c};
+          for (int d = 0; d < 3; ++d) {
+            t.lo[d] = part_begin(g[d], n[d], at[d]);
+            t.hi[d] = part_begin(g[d], n[d], at[d] + 1);
+          }
+          tiles.push_back(t);
+        }
+  }
+  return tiles;
 }
 
 // Level l >= 1: patches grown by 2; ghost-fill sources; average-down table
@@ -936,7 +1024,10 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
       return fail(ctx, LBX_E_ARG, "level-%d box too large", level);
     }
     d.cells = (int)cells;
-    d.qs = (cells + 63) / 64 * 64;
+    const bool packed = r == 2;
+    d.row = packed ? b.n(0) : d.g[0];
+    d.plane = packed ? b.n(0) * b.n(1) : d.g[0] * d.g[1];
+    d.qs = ((packed ? b.cells() : cells) + 63) / 64 * 64;
     d.fill_base = fill_base;
     d.avg_base = avg_base;
     const int blocks = (b.n(0) / r + 2 * ng) * (b.n(1) / r + 2 * ng) * (b.n(2) / r + 2 * ng);
@@ -961,12 +1052,14 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
       return std::make_tuple(A.lo[2], A.lo[1], A.lo[0]) < std::make_tuple(B.lo[2], B.lo[1], B.lo[0]);
     });
     for (int b : order) {
-      F.desc[b].base = base;
+      PatchDesc& d = F.desc[b];
+      d.base = base;
+      d.origin = r == 2 ? base - (2ll * d.plane + 2ll * d.row + 2) : base;
       base += F.desc[b].qs * lbx::NV_TOTAL;
     }
     for (int b : order) F.gdesc.push_back(F.desc[b]);
     const long long esz = (long long)elem_size(sim->precision);
-    for (size_t k = 0; k < F.gdesc.size();) {
+    for (size_t k = 0; r > 2 && k < F.gdesc.size();) {
       long long elems = 0;
       size_t n = 0;
       while (k + n < F.gdesc.size()) {
@@ -976,17 +1069,33 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
         ++n;
       }
       F.groups.push_back({(int)k, (int)n});
-      F.region_span = std::max(F.region_span, elems);
       k += n;
     }
-    // per-stream regions of buf[2] for the array between the two substeps;
-    // at a ratio above 2 the substeps chain through the whole buf[2]
-    F.regions = r == 2 && F.groups.size() > 1 && 2 * F.region_span <= base;  // base: one level buffer's elements
   }
+  std::vector<lbx::FineTile> tiles;
+  if (r == 2) tiles = plan_tiles(F.gdesc);
+  F.ntiles = (int)tiles.size();
   // Ghost fill sources (FillPatchTwoLevels with piecewise-constant
   // interpolation, src/AmrSim.cpp:373-388): the valid cell of this level
   // holding the periodic image if a box has it, else the coarse parent.
+  // At ratio 2 a source is an element and a stride (lbx::FineStep::fill); a
+  // level of fewer than 2^32 grown cells, and any level 0 that fits the
+  // device, has fewer than 2^40 elements, and the strides are at most one a box.
   std::vector<long long> fill((size_t)fill_base, 0);
+  std::vector<unsigned> strides;
+  bool same = true;  // one stride for this level's patches, one for the parent's
+  for (const PatchDesc& p : F.desc) same &= p.qs == F.desc[0].qs;
+  for (const PatchDesc& p : C.desc) same &= !C.patched || p.qs == C.desc[0].qs;
+  std::map<long long, unsigned> stride_ids;
+  auto packed_source = [&](unsigned long long parent, long long elem, long long qs) {
+    unsigned long long id = 0;
+    if (!same) {
+      const auto it = stride_ids.emplace(qs, (unsigned)stride_ids.size());
+      if (it.second) strides.push_back((unsigned)qs);
+      id = it.first->second;
+    }
+    return (long long)(parent | id << lbx::kFillStrideShift | (unsigned long long)elem);
+  };
   int hint = 0;
   for (size_t b = 0; b < boxes.size(); ++b) {
     const PatchDesc& P = F.desc[b];
@@ -1009,7 +1118,9 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
           long long d;
           if (src >= 0) {
             hint = src;
-            d = ((long long)src << 32) | grown_index(F.desc[src], wx, wy, wz);
+            const PatchDesc& Q = F.desc[src];
+            d = r == 2 ? packed_source(0, Q.at(wx - Q.lo[0] + 2, wy - Q.lo[1] + 2, wz - Q.lo[2] + 2), Q.qs)
+                       : ((long long)src << 32) | grown_index(Q, wx, wy, wz);
           } else {
             long long ref;
             if (!cell_ref(C, wx / r, wy / r, wz / r, &ref, chint)) {
@@ -1017,7 +1128,15 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
               return fail(ctx, LBX_E_ARG, "level-%d box %zu is not properly nested in level %d", level, b,
                           level - 1);
             }
-            d = -1 - ref;
+            if (r > 2) {
+              d = -1 - ref;
+            } else if (C.patched) {
+              const PatchDesc& Q = C.desc[ref >> 32];
+              d = packed_source(lbx::kFillParent,
+                                Q.at(wx / r - Q.lo[0] + 2, wy / r - Q.lo[1] + 2, wz / r - Q.lo[2] + 2), Q.qs);
+            } else {
+              d = packed_source(lbx::kFillParent, ref, C.lat.ps);
+            }
           }
           fill[P.fill_base + ((long long)gz * P.g[1] + gy) * P.g[0] + gx] = d;
         }
@@ -1061,11 +1180,12 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
   }
   start.push_back((int)list.size());
   F.sum_ncell = (int)cell.size();
-  std::vector<int> slot;
+  std::vector<long long> span;
   if (C.patched) {
-    slot.assign((size_t)C.grown_cells, -1);
+    span.assign((size_t)C.grown_cells, -1);
     for (size_t u = 0; u < cell.size(); ++u)
-      slot[C.desc[cell[u] >> 32].fill_base + (cell[u] & 0xffffffffll)] = (int)u;
+      span[C.desc[cell[u] >> 32].fill_base + (cell[u] & 0xffffffffll)] =
+          ((long long)start[u] << 32) | (start[u + 1] - start[u]);
   }
   F.avg_stride = (avg_base + 63) / 64 * 64;
   const size_t bytes = (size_t)base * elem_size(sim->precision);
@@ -1078,7 +1198,7 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
                   hipGetErrorString(e));
     }
   }
-  for (int i = 0; i < 3; ++i) {
+  for (int i = 0; i < (r == 2 ? 2 : 3); ++i) {
     hipError_t e = hipMalloc(&F.buf[i], bytes);
     if (e == hipSuccess) e = hipMemsetAsync(F.buf[i], 0, bytes, ctx->stream);
     if (e != hipSuccess) {
@@ -1089,11 +1209,13 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
   }
   hipError_t e = upload(&F.d_desc, F.desc, ctx->stream);
   if (e == hipSuccess) e = upload(&F.d_gdesc, F.gdesc, ctx->stream);
+  if (e == hipSuccess) e = upload(&F.d_tiles, tiles, ctx->stream);
   if (e == hipSuccess) e = upload(&F.d_fill, fill, ctx->stream);
+  if (e == hipSuccess) e = upload(&F.d_strides, strides, ctx->stream);
   if (e == hipSuccess && !C.patched) e = upload(&F.d_sum_cell, cell, ctx->stream);
   if (e == hipSuccess) e = upload(&F.d_sum_start, start, ctx->stream);
   if (e == hipSuccess) e = upload(&F.d_sum_contrib, contrib, ctx->stream);
-  if (e == hipSuccess && C.patched) e = upload(&F.d_sum_slot, slot, ctx->stream);
+  if (e == hipSuccess && C.patched) e = upload(&F.d_sum_span, span, ctx->stream);
   if (!C.patched) C.push_shape = lbx::default_shape(C.lat, sim->precision);
   if (e != hipSuccess) {
     free_level(F);
@@ -1152,7 +1274,7 @@ int remake_level(lbx_sim* sim, int level, const std::vector<Box>& boxes) {
         for (int x = P.lo[0]; x <= P.hi[0]; ++x) {
           long long ref = 0;
           (void)cell_ref(C, x / nf.ratio, y / nf.ratio, z / nf.ratio, &ref, chint);  // nesting checked by build_level
-          src[P.fill_base + grown_index(P, x, y, z)] = -1 - ref;
+          src[P.fill_base + grown_index(P, x, y, z)] = -1 - stored_ref(C, ref);
         }
     for (size_t o = 0; o < F.boxes.size(); ++o) {
       const PatchDesc& O = F.desc[o];
@@ -1167,7 +1289,7 @@ int remake_level(lbx_sim* sim, int level, const std::vector<Box>& boxes) {
       for (int z = lo[2]; z <= hi[2]; ++z)
         for (int y = lo[1]; y <= hi[1]; ++y)
           for (int x = lo[0]; x <= hi[0]; ++x)
-            src[P.fill_base + grown_index(P, x, y, z)] = ((long long)o << 32) | grown_index(O, x, y, z);
+            src[P.fill_base + grown_index(P, x, y, z)] = stored_ref(F, ((long long)o << 32) | grown_index(O, x, y, z));
     }
   }
   DeviceTemp t;
@@ -1207,7 +1329,7 @@ int fill_from_patched(lbx_sim* sim, int level) {
           long long ref;
           if (!cell_ref(C, x / F.ratio, y / F.ratio, z / F.ratio, &ref, chint))
             return fail(ctx, LBX_E_STATE, "level %d is not nested in level %d", level, level - 1);
-          src[P.fill_base + grown_index(P, x, y, z)] = -1 - ref;
+          src[P.fill_base + grown_index(P, x, y, z)] = -1 - stored_ref(C, ref);
         }
   }
   DeviceTemp t;
@@ -1518,7 +1640,7 @@ int lbx_fill_from_coarse(lbx_sim* sim, int level) {
   if (int rc = materialise(sim)) return rc;
   if (C.patched) return fill_from_patched(sim, level);
   LBX_HIP(ctx, lbx::launch_fine_from_coarse(sim->precision, F.buf[F.cur], C.buf[C.cur], C.lat, F.d_desc,
-                                            (int)F.boxes.size(), F.max_cells, sim->rho0, F.ratio, ctx->stream));
+                                            (int)F.boxes.size(), F.max_cells, F.ratio, ctx->stream));
   LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return LBX_OK;
 }

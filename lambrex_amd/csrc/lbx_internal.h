@@ -134,15 +134,20 @@ hipError_t launch_tag(int precision, bool pull, int criterion, const void* f, co
 hipError_t launch_conservation(int precision, bool pull, const void* f, const Lattice& L, double rho0,
                                double* partials, int nblocks, double* out, hipStream_t st);
 
-// A box stored on its own with 2 ghost layers (fine level), or a box of a
-// level array (coarse push: only lo/hi/cells used).  Population q of grown
-// local cell i is at base + q*qs + i.
+// A box of a patched level, which its step grows by 2 ghost layers, or a box
+// of a level array (only lo/hi/cells used).  Population q of grown local cell
+// (x, y, z) is at at(x, y, z) + q*qs: at refinement ratio 2 the valid cells
+// alone are stored, packed (whole cache lines are written, and a level buffer
+// of 32^3 boxes is 0.70 x the grown one); above it the grown box.
 struct PatchDesc {
   int lo[3], hi[3];  // valid box, level index space (inclusive)
   int g[3];          // grown extents (n + 4)
   int cells;         // grown cells (or valid cells for level-array boxes)
-  long long base;    // element offset of the patch in the level buffer
-  long long qs;      // population stride (cells rounded up to 64)
+  int row, plane;    // elements from a stored row and plane to the next
+  long long base;    // element of population 0 of the first stored cell
+  long long origin;  // ... of grown cell (0, 0, 0), stored or not
+  long long qs;      // population stride
+  LBX_IHD long long at(int x, int y, int z) const { return origin + (long long)z * plane + y * row + x; }
   long long fill_base;  // offset of this patch's rows in the fill table
   long long avg_base;   // offset of this patch's 2x2x2 block averages ((g/2)^3 per population)
 };
@@ -167,13 +172,10 @@ hipError_t launch_fine_fill_collide(int precision, const void* fnow, void* fnext
                                     const Lattice& clat, const PatchDesc* cpatches, const PatchDesc* patches,
                                     const PatchDesc* own, int first, int npatch, int max_cells,
                                     const long long* fill, const unsigned char* mask, const Relax& r,
-                                    hipStream_t st, long long oshift = 0);
-// out holds each patch at element P.base - oshift (0: a level buffer; the
-// group's first base: a group-sized scratch array); an input the same way
-// at P.base - ishift.
+                                    hipStream_t st);
 // inner: `in` is itself such an output (outer layer not stored, read as
 // zero), for the later substeps at a refinement ratio above 2.
-hipError_t launch_fine_stream_collide(int precision, const void* in, void* out, long long oshift,
+hipError_t launch_fine_stream_collide(int precision, const void* in, void* out,
                                       const PatchDesc* patches, int first, int npatch, int max_cells, const Relax& r,
                                       hipStream_t st, bool inner = false);
 // The finest level's last substep at a refinement ratio above 2: stream of
@@ -186,26 +188,53 @@ hipError_t launch_fine_avg_valid(int precision, const void* f, double* avg, long
                                  const PatchDesc* patches, int first, int npatch, int max_blocks, int ratio,
                                  double rho0, hipStream_t st);
 // Stream + ZeroInvalidComponents of a middle level (no collide), with the
-// child's block averages added into valid cells: slot[fill_base + i] is the
-// touched-cell index of grown cell i (-1 if none), start/contrib as in
-// launch_sum_apply.
+// child's block averages added into valid cells: spans[fill_base + i] names
+// the contributions of grown cell i in contrib (see launch_sum_apply): the
+// first in the high 32 bits, their number in the low ones; -1 if none.
 hipError_t launch_fine_stream_zero(int precision, const void* in, void* out, const PatchDesc* patches, int first,
-                                   int npatch, int max_cells, double rho0, const int* slot, const double* avg,
-                                   long long avg_stride, const int* start, const int* contrib, hipStream_t st,
-                                   long long ishift = 0);
-// avg holds 15 FP64 planes of avg_stride block averages; max_blocks = max (g/2)^3;
-// in holds each patch at element P.base - ishift.
-hipError_t launch_fine_stream_avg(int precision, const void* in, long long ishift, void* out, double* avg,
-                                  long long avg_stride, const PatchDesc* patches, int first, int npatch,
-                                  int max_blocks, double rho0, hipStream_t st);
-// A middle level's last step of its parent's step, all patches: the stream of
-// launch_fine_stream_zero (the child's block averages cavg added through
-// slot / start / contrib) fused with the level's own block averages of the
-// result into avg.
-hipError_t launch_middle_stream_avg(int precision, const void* in, long long ishift, void* out, double* avg,
-                                   long long avg_stride, const PatchDesc* patches, int first, int npatch,
-                                   int max_blocks, double rho0, const int* slot, const double* cavg,
-                                   long long cavg_stride, const int* start, const int* contrib, hipStream_t st);
+                                   int npatch, int max_cells, double rho0, const long long* spans,
+                                   const double* avg, long long avg_stride, const int* contrib, hipStream_t st);
+// A tile of a patch in k_fine_step: grown cells [lo, hi), even on both ends,
+// of patch `patch` (launch order).  With the 2 cells around it in x and y
+// (inside the patch) it holds at most kFineTileCells cells per plane.
+struct FineTile {
+  int patch;
+  int lo[3], hi[3];
+};
+constexpr int kFineTileCells = 512;
+
+constexpr unsigned long long kFillParent = 1ull << 63, kFillElement = (1ull << 40) - 1;
+constexpr int kFillStrideShift = 40;
+
+// One step of a patched level at ratio 2 (lbx_twolevel.hip): the finest
+// level's two substeps, or a middle level's step with its child's block
+// averages (spans, cavg, contrib) added; `avg` non-null: the level's
+// own block averages for its parent (always for the finest).
+struct FineStep {
+  bool finest;
+  const void* now;
+  void* next;
+  const void* parent;          // the parent's current state
+  const PatchDesc* own;        // the level's patches in launch order
+  const FineTile* tiles;
+  int ntiles;
+  // Per ghost cell of the level: the element of population 0 of its source,
+  // in the parent's state with kFillParent, else in the level's; the source's
+  // population stride is strides[bits from kFillStrideShift], or with strides
+  // null the patch's own (every patch has the same) or parent_stride.
+  const unsigned long long* fill;
+  const unsigned* strides;
+  long long parent_stride;
+  const unsigned char* mask;
+  Relax relax;
+  double* avg;
+  long long avg_stride;
+  const long long* spans;
+  const double* cavg;
+  long long cavg_stride;
+  const int* contrib;
+};
+hipError_t launch_fine_step(int precision, const FineStep& a, hipStream_t st);
 // flags: per coarse cell (x fastest), bits 0-5 = x+1, x-1, y+1, y-1, z+1,
 // z-1 leave the cell's box; bit 7 = masked by the fine level.
 hipError_t launch_coarse_push(int precision, const void* cnow, void* cnext, const Lattice& L,
@@ -217,11 +246,11 @@ hipError_t launch_sum_apply(int precision, const double* avg, long long avg_stri
                             const long long* cell, const int* start, const int* contrib, int ncell, double rho0,
                             hipStream_t st);
 hipError_t launch_fine_from_coarse(int precision, void* fnow, const void* cnow, const Lattice& clat,
-                                   const PatchDesc* patches, int npatch, int max_cells, double rho0, int ratio,
+                                   const PatchDesc* patches, int npatch, int max_cells, int ratio,
                                    hipStream_t st);
 // Valid cells of new patches from old patches or the coarse parent
-// (src per new grown cell: (old patch << 32) | old grown index, or a coarse
-// reference as above).
+// (src per new grown cell: (old patch << 32) | element from its base, or a
+// coarse reference likewise).
 hipError_t launch_fine_remake(int precision, void* fnew, const void* fold, const void* cnow, const Lattice& clat,
                               const PatchDesc* cpatches, const PatchDesc* patches, int npatch, int max_cells,
                               const PatchDesc* old_patches, const long long* src, hipStream_t st);

@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void k_patch_conservation(const S* __restrict_
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
     const int x = i % nx, t = i / nx, y = t % ny, z = t / ny;
-    const long long li = P.base + ((long long)(z + 2) * P.g[1] + (y + 2)) * P.g[0] + (x + 2);
+    const long long li = P.at(x + 2, y + 2, z + 2);
     double g[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) {

@@ -185,7 +185,7 @@ size_t esize(int precision) { return precision == LBX_FP64 ? 8 : 4; }
 
 long long cells_of(const lbx_request& q) { return (long long)q.dims[0] * q.dims[1] * q.dims[2]; }
 
-// Device memory a refined run's simulation allocates: two level-0 arrays
+// An upper bound of the device memory of a refined run: two level-0 arrays
 // and their flag bytes, four buffers of grown fine patches (2 ghost layers,
 // population stride rounded to 64) with their fill table, mask bytes and
 // block averages, and the parent's touched-cell slots; 1/8 more for the

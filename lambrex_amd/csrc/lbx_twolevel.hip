@@ -9,16 +9,12 @@
 // coarse step and never collided), so a cell seen as a ghost by one box and
 // as valid by its neighbour evolves differently in the two places.
 //
-// One coarse step, in the reference's order of effects:
-//   k_fine_fill_collide   FillPatchTwoLevels(fine next <- fine now | coarse
-//                         now, piecewise constant) + zero comp 0 on the outer
-//                         ghost layer + collide valid fine cells
-//   k_fine_stream_collide Stream(1) (valid + 1 ghost layer; outer layer of the
-//                         fresh array defined as 0, not stored) + collide
-//                         valid cells
-//   k_fine_stream_avg     Stream(1) + ZeroInvalidComponents(1), and the 1/8
-//                         weighted sum of every 2x2x2 block of the result;
-//                         valid cells stored (the next fill rewrites ghosts)
+// One coarse step at refinement ratio 2, in the reference's order of effects:
+//   k_fine_step           both fine substeps (FillPatchTwoLevels, collide,
+//                         Stream(1), collide, Stream(1),
+//                         ZeroInvalidComponents) in one pass from the current
+//                         state to the next, with the 1/8 weighted sum of
+//                         every 2x2x2 block of the result
 //   k_coarse_push         CoarseCollide(0) (masked cells -> 0) + Stream(0) in
 //                         push form; pulls across a box face read the
 //                         pre-collision ghost copies, as the reference's
@@ -27,16 +23,17 @@
 //   k_sum_apply           SumFromFine(0): ADD those block averages (fine valid
 //                         + ghosts) into coarse next, contributions to one
 //                         coarse cell in a fixed order
+// Only valid cells are stored, packed (PatchDesc): the ghosts live in the pass.
 //
-// Deeper hierarchies (RohdeCycle's recursion, src/AmrSim.cpp:453-455) reuse
-// these kernels on patched "middle" levels, which have both a parent and a
-// child: the fill-collide takes its coarse values from patches (PC) and
-// zeroes the cells under the child's mask (MASK); k_fine_stream_zero is the
-// middle level's stream of its valid cells with the child's block averages
-// added into them; and k_fine_stream_avg<S, true> is the same plus
-// ZeroInvalidComponents for the middle level's last step of its parent's
-// step, with the block averages of its result for the parent.  Every pass
-// stores valid cells only.
+// Deeper hierarchies (RohdeCycle's recursion, src/AmrSim.cpp:453-455) run the
+// same kernel on patched "middle" levels, which have both a parent and a
+// child: one step of them, with the cells under the child's mask zeroed
+// (MASK) and the child's block averages added into the valid cells (SUM).
+//
+// At ratios above 2 (r substeps, no fine ghosts in the average-down) a level's
+// patches are stored grown and a step is one pass per substep:
+// k_fine_fill_collide, k_fine_stream_collide, then k_fine_stream_valid and
+// k_fine_avg_valid on the finest level, k_fine_stream_zero on a middle one.
 //
 // Storage type S is double (FP64, bit-exact with the oracle) or float (the
 // shifted deviation d = f - w rho0 of the FP32 path).  Either way the block
@@ -131,12 +128,7 @@ __device__ __forceinline__ bool patch_outer(const PatchDesc& P, int gx, int gy, 
   return gx == 0 || gy == 0 || gz == 0 || gx == P.g[0] - 1 || gy == P.g[1] - 1 || gz == P.g[2] - 1;
 }
 
-// valid-region membership of absolute position p for patch P
-__device__ __forceinline__ bool in_valid(const PatchDesc& P, int x, int y, int z) {
-  return x >= P.lo[0] && x <= P.hi[0] && y >= P.lo[1] && y <= P.hi[1] && z >= P.lo[2] && z <= P.hi[2];
-}
-
-// Every lane first picks where its 15 populations come from (its own valid
+// Collide of a level at a ratio above 2.  Every lane first picks where its 15 populations come from (its own valid
 // cell, the fine valid cell holding its periodic image, or the coarse
 // parent) so the loads of valid and ghost lanes issue together; valid cells
 // are then collided.  Coarse sources are -1 - (element of population 0) in
@@ -151,7 +143,7 @@ __global__ __launch_bounds__(256) void k_fine_fill_collide(
     const S* __restrict__ fnow, S* __restrict__ fnext, const S* __restrict__ cnow, Lattice clat,
     const PatchDesc* __restrict__ cpatches, const PatchDesc* __restrict__ patches,
     const PatchDesc* __restrict__ own, int first, const long long* __restrict__ fill,
-    const unsigned char* __restrict__ mask, Relax r, long long oshift) {
+    const unsigned char* __restrict__ mask, Relax r) {
   // P is read in place: with a by-value copy the PC variants merged the
   // loads of base / qs from P, patches[s] and cpatches[] into one load through
   // a selected pointer, which kept the copy in 80 B of scratch per lane.
@@ -195,9 +187,8 @@ __global__ __launch_bounds__(256) void k_fine_fill_collide(
   } else if (patch_outer(P, gx, gy, gz)) {
     f[0] = zero_pop<S>(0, r.rho0);
   }
-  const long long ob = P.base - oshift;
 #pragma unroll
-  for (int q = 0; q < NV; ++q) fnext[ob + q * P.qs + i] = f[q];
+  for (int q = 0; q < NV; ++q) fnext[P.base + q * P.qs + i] = f[q];
 }
 
 // Pull of grown cell i over valid + 1 ghost layer, from the patch stored at
@@ -243,17 +234,15 @@ __device__ __forceinline__ bool fine_pull_inner(const PatchDesc& P, const S* __r
   return patch_valid(P, gx, gy, gz);
 }
 
-// First fine substep's stream + the second substep's collision: pull, then
-// collide valid cells.  `out` holds the patch at element P.base - oshift (a
-// group-sized scratch array when oshift is the group's first base).  The
-// outer ghost layer of the result is zero by definition (Stream's fresh
-// array) and is not stored: the next pass reads it as zero.  With INNER the
-// input is itself such a result (a later substep at a refinement ratio above
-// 2), whose outer layer is read as zero.
+// A fine substep's stream + the next one's collision (refinement ratios above
+// 2): pull, then collide valid cells.  The outer ghost layer of the result is
+// zero by definition (Stream's fresh array) and is not stored: the next pass
+// reads it as zero.  With INNER the input is itself such a result (a later
+// substep), whose outer layer is read as zero.
 template <typename S, bool INNER = false>
 __global__ __launch_bounds__(256) void k_fine_stream_collide(const S* __restrict__ in, S* __restrict__ out,
                                                              const PatchDesc* __restrict__ patches, int first,
-                                                             Relax r, long long oshift) {
+                                                             Relax r) {
   const PatchDesc P = patches[first + blockIdx.y];
   const int i = xcd_chunk() * 256 + threadIdx.x;
   if (i >= P.cells) return;
@@ -264,32 +253,22 @@ __global__ __launch_bounds__(256) void k_fine_stream_collide(const S* __restrict
   const bool valid = INNER ? fine_pull_inner(P, in, P.base, i, gx, gy, gz, r.rho0, f)
                            : fine_pull(P, in, P.base, i, gx, gy, gz, r.rho0, f);
   if (valid) collide_s(f, r);
-  const long long ob = P.base - oshift;
 #pragma unroll
-  for (int q = 0; q < NV; ++q) out[ob + q * P.qs + i] = f[q];
+  for (int q = 0; q < NV; ++q) out[P.base + q * P.qs + i] = f[q];
 }
 
-// ZeroInvalidComponents on a ghost cell at absolute (x, y, z): population m
-// survives only if pos - 2 c_m lies in the patch's valid box.
+// SumFromFine's addition into one valid cell of a patched level: `span` names
+// its contributions (the first in the high 32 bits, their number in the low
+// ones), the block averages avg[q * avg_stride + contrib[j]], added in FP64
+// in that order to the cell's streamed value.
 template <typename S>
-__device__ __forceinline__ void zero_invalid(const PatchDesc& P, int gx, int gy, int gz, double rho0, S* f) {
-  const int x = P.lo[0] - 2 + gx, y = P.lo[1] - 2 + gy, z = P.lo[2] - 2 + gz;
-#pragma unroll
-  for (int q = 0; q < NV; ++q)
-    if (!in_valid(P, x - 2 * kC[q][0], y - 2 * kC[q][1], z - 2 * kC[q][2])) f[q] = zero_pop<S>(q, rho0);
-}
-
-// SumFromFine's addition into one valid cell of a patched level: the block
-// averages avg[q * avg_stride + contrib[j]], j in [start[u], start[u+1]),
-// added in FP64 in that order to the cell's streamed value.
-template <typename S>
-__device__ __forceinline__ void add_block_sums(S* f, int u, const double* __restrict__ avg, long long avg_stride,
-                                               const int* __restrict__ start, const int* __restrict__ contrib,
-                                               double rho0) {
+__device__ __forceinline__ void add_block_sums(S* f, long long span, const double* __restrict__ avg,
+                                               long long avg_stride, const int* __restrict__ contrib, double rho0) {
   double acc[NV];
 #pragma unroll
   for (int q = 0; q < NV; ++q) acc[q] = to_f64(f[q], q, rho0);
-  for (int j = start[u]; j < start[u + 1]; ++j) {
+  const int first = int(span >> 32), n = int(span & 0xffffffffll);
+  for (int j = first; j < first + n; ++j) {
     const long long a = contrib[j];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] += avg[q * avg_stride + a];
@@ -305,18 +284,15 @@ __device__ __forceinline__ void add_block_sums(S* f, int u, const double* __rest
 // cells from its state (its next fill rewrites them, a finer level's fill
 // and every read-back take valid cells only).  Fused with the second half
 // of SumFromFine into this level (src/AmrSim.cpp:464-466, 592-602): a valid
-// cell whose slot (per grown cell, -1 if none) names a touched cell u adds
-// the child's block averages [start[u], start[u+1]) to its streamed value in
-// FP64, in the same order as k_sum_apply.  `in` holds each patch at element
-// P.base - ishift (a group-sized region when ishift is the group's first
-// base); `out` at P.base.
+// cell with a span (per grown cell, -1 if none) adds the child's block
+// averages it names to its streamed value in FP64, in the same order as
+// k_sum_apply.
 template <typename S>
 __global__ __launch_bounds__(256) void k_fine_stream_zero(const S* __restrict__ in, S* __restrict__ out,
                                                           const PatchDesc* __restrict__ patches, int first,
-                                                          double rho0, const int* __restrict__ slot,
+                                                          double rho0, const long long* __restrict__ spans,
                                                           const double* __restrict__ avg, long long avg_stride,
-                                                          const int* __restrict__ start,
-                                                          const int* __restrict__ contrib, long long ishift) {
+                                                          const int* __restrict__ contrib) {
   const PatchDesc P = patches[first + blockIdx.y];
   const int i = xcd_chunk() * 256 + threadIdx.x;
   if (i >= P.cells) return;
@@ -324,85 +300,366 @@ __global__ __launch_bounds__(256) void k_fine_stream_zero(const S* __restrict__ 
   patch_coords(P, i, gx, gy, gz);
   if (!patch_valid(P, gx, gy, gz)) return;
   S f[NV];
-  fine_pull(P, in, P.base - ishift, i, gx, gy, gz, rho0, f);
-  const int u = slot[P.fill_base + i];
-  if (u >= 0) add_block_sums(f, u, avg, avg_stride, start, contrib, rho0);
+  fine_pull(P, in, P.base, i, gx, gy, gz, rho0, f);
+  const long long span = spans[P.fill_base + i];
+  if (span >= 0) add_block_sums(f, span, avg, avg_stride, contrib, rho0);
 #pragma unroll
   for (int q = 0; q < NV; ++q) out[P.base + q * P.qs + i] = f[q];
 }
 
-// Second fine substep's stream + ZeroInvalidComponents(1), fused with the
-// first half of SumFromFine: the 1/8-weighted sum of each 2x2x2 block of the
-// grown patch (= one coarse cell of the coarsened box grown by 1), children
-// added in (k, j, i) order in FP64, to avg[q * avg_stride + avg_base + block].
-// A workgroup takes B = avg_blocks<S>() consecutive blocks; thread t
-// computes child t / B of block t % B, so each wavefront reads whole x-pairs
-// of its blocks.  The children meet in LDS for the ordered sums, as stored
-// values (S), and each child is converted to FP64 f as it is added (the
-// same bits as converting first).
-// With SUM (a middle level's
-// last step of its parent's step) the stream is k_fine_stream_zero's, the
-// child's block averages (slot, cavg, start, contrib) added into valid
-// cells, and the block sums are those of the level's resulting state, ghost
-// shell included.  Without SUM (the finest level's second substep) the
-// input's outer ghost layer is not stored and reads as zero.  Either way
-// only valid cells are stored: the ghost cells of a level's state are
-// rewritten by its next fill-collide before anything reads them.
-// Blocks per workgroup (8 threads each): 32 in FP64; 16 in FP32, whose
-// passes are shorter, so that a barrier spans two waves instead of four.
-template <typename S>
-constexpr int avg_blocks() { return sizeof(S) == 4 ? 16 : 32; }
+// One whole step of a patched level at ratio 2, from its parent's and its own
+// current states: with FINEST the finest level's two substeps of a step of
+// its parent, else one step of a level between level 0 and the finest.  In
+// the reference's terms, per grown cell:
+//   A  FillPatchTwoLevels, comp 0 zeroed on the outer ghost layer, collide of
+//      the valid cells (a cell under the child's mask is zeroed: MASK)
+//   B  (FINEST) Stream(1) over valid + 1 ghost layer of a fresh array, whose
+//      outer layer is zero, and the second substep's collide
+//   C  Stream(1); with SUM the child's block averages added into the valid
+//      cells (SumFromFine), ZeroInvalidComponents, the valid cells stored,
+//      and with AVG the 1/8-weighted sum of each 2x2x2 block of the grown
+//      patch for the parent (children in (k, j, i) order in FP64)
+// A patch's ghosts are filled once, so no patch's A, B or C depends on
+// another's, and nothing but the valid cells of C and the block averages has
+// to reach memory.  A workgroup takes a tile (FineTile: a range of grown
+// cells in x, y and z, even on both ends) and walks z: it forms plane k of A
+// over the tile and 2 cells around it, plane k - 1 of B over the tile and 1
+// cell around it, and plane k - 2 of C, each handed to the next through one
+// LDS plane; of the three planes a pull reads, the upper one is in LDS and
+// the populations with c_z = 0 and +1 of the other two are carried in
+// registers.  A wave holds whole 2x2 columns, so the 4 children of a block in
+// a plane meet in the wave's own part of the A plane, which is free by then,
+// without a barrier; its two halves hold a row each, so that its loads and
+// stores run along x (with the 4 children in neighbouring lanes a load took
+// 110 cycles to issue).  A
+// population that does not move (q = 0) stays in its lane.
+//
+// Bound: per plane two collisions of each cell (and the ring's) against one
+// read of the grown patch and one write of its valid cells.  The passes this
+// replaces (fill + collide, stream + collide, stream + average; each reading
+// and writing every patch, in groups kept in the MALL) moved 7.7 valid-cell
+// transfers per pair of substeps and ran at the fabric's rate.  128 patches of
+// 36^3 (64 of 32^3 valid cells each way), two substeps: FP64 750 us before,
+// 445 us so, of which a plane's two collisions and pulls are about 60 %; one
+// workgroup a CU (114 KB of LDS, 2 waves a SIMD at 256 registers).  Slower: 12
+// waves on tiles of 36 x 20 cells at 168 registers (484 us), the loads of a
+// plane in one piece or after the first barrier (503 to 627 us).
+constexpr int kFineThreads = 512;  // 8 waves
+constexpr int kFineCells = kFineTileCells;
 
-template <typename S, bool SUM = false>
-__global__ __launch_bounds__(256) void k_fine_stream_avg(const S* __restrict__ in, S* __restrict__ out,
-                                                         double* __restrict__ avg, long long avg_stride,
-                                                         const PatchDesc* __restrict__ patches, int first,
-                                                         double rho0, long long ishift,
-                                                         const int* __restrict__ slot = nullptr,
-                                                         const double* __restrict__ cavg = nullptr,
-                                                         long long cavg_stride = 0,
-                                                         const int* __restrict__ start = nullptr,
-                                                         const int* __restrict__ contrib = nullptr) {
-  constexpr int kAvgBlocks = avg_blocks<S>();
-  __shared__ S part[NV][8][kAvgBlocks];
-  const PatchDesc P = patches[first + blockIdx.y];
-  const int c0 = P.g[0] >> 1, c1 = P.g[1] >> 1, c2 = P.g[2] >> 1;
-  const int nblk = c0 * c1 * c2;
-  const int b0 = xcd_chunk() * kAvgBlocks;  // first block of this workgroup
-  if (b0 >= nblk) return;                  // uniform over the workgroup
-  const int child = threadIdx.x / kAvgBlocks, lb = threadIdx.x % kAvgBlocks;
-  const int u = b0 + lb;
-  if (u < nblk) {
-    const int di = child & 1, dj = (child >> 1) & 1, dk = child >> 2;
-    int cx, cy, cz;
-    split3(u, nblk, c0, c1, cx, cy, cz);
-    const int gx = 2 * cx + di, gy = 2 * cy + dj, gz = 2 * cz + dk;
-    const int i = (gz * P.g[1] + gy) * P.g[0] + gx;
-    S f[NV];
-    const bool valid = SUM ? fine_pull(P, in, P.base - ishift, i, gx, gy, gz, rho0, f)
-                           : fine_pull_inner(P, in, P.base - ishift, i, gx, gy, gz, rho0, f);
-    if (valid) {
-      if constexpr (SUM) {
-        const int su = slot[P.fill_base + i];
-        if (su >= 0) add_block_sums(f, su, cavg, cavg_stride, start, contrib, rho0);
-      }
-    } else if (!patch_outer(P, gx, gy, gz)) {
-      zero_invalid(P, gx, gy, gz, rho0, f);
+// Orders a wave's LDS accesses among its own lanes.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// to_f64 for a population known at run time only.
+template <typename S>
+__device__ __forceinline__ double to_f64_any(S v, int q, double rho0) {
+  if constexpr (sizeof(S) == 8)
+    return v;
+  else
+    return (q == 0 ? kT.W[0] : q <= 6 ? kT.W[1] : kT.W[7]) * rho0 + double(v);
+}
+
+// Number of a population's (c_x, c_y).
+__device__ constexpr int lateral(int q) { return (kC[q][1] + 1) * 3 + kC[q][0] + 1; }
+
+// First of the populations that share (c_x, c_y): 1 to 4, then 5, 7, 9, 11, 13.
+__device__ constexpr int pull_first(int c) { return c < 4 ? c + 1 : 2 * c - 3; }
+
+template <typename S, bool FINEST, bool MASK, bool SUM, bool AVG>
+__global__ __launch_bounds__(kFineThreads) void k_fine_step(
+    const S* __restrict__ fnow, S* __restrict__ fnext, const S* __restrict__ cnow,
+    const PatchDesc* __restrict__ own, const FineTile* __restrict__ tiles, int ntiles,
+    const unsigned long long* __restrict__ fill, const unsigned* __restrict__ strides, long long parent_stride,
+    const unsigned char* __restrict__ mask, Relax r, double* __restrict__ avg,
+    long long avg_stride, const long long* __restrict__ spans, const double* __restrict__ cavg, long long cavg_stride,
+    const int* __restrict__ contrib) {
+  // plane A of population q, then plane B of it
+  constexpr int kSets = FINEST ? 2 : 1;
+  __shared__ S planes[NV - 1][kSets][kFineCells];
+  constexpr int kB = kSets - 1;
+  constexpr int kCut1 = 5, kCut2 = 10;
+  const int w = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);  // an XCD takes neighbouring tiles
+  if (w >= ntiles) return;
+  const FineTile T = tiles[w];
+  const PatchDesc& P = own[T.patch];
+  const int gx = P.g[0], gy = P.g[1], gz = P.g[2];
+  // A region in x and y, and this thread's cell of it
+  const int ax = max(T.lo[0] - 2, 0), ay = max(T.lo[1] - 2, 0);
+  const int wb = (min(T.hi[0] + 2, gx) - ax) >> 1, hb = (min(T.hi[1] + 2, gy) - ay) >> 1;  // 2x2 columns
+  // A wave holds 16 consecutive 2x2 columns: its lower half their lower rows,
+  // its upper half the upper rows, each 32 cells along x.
+  const int t = threadIdx.x, col = (t >> 6) * 16 + ((t & 31) >> 1);
+  const bool on = col < wb * hb;
+  const int x = ax + 2 * (col % wb) + (t & 1), y = ay + 2 * (col / wb) + ((t >> 5) & 1);
+  const bool outer_xy = x == 0 || y == 0 || x == gx - 1 || y == gy - 1;
+  const bool valid_xy = on && x >= 2 && x < gx - 2 && y >= 2 && y < gy - 2;
+  const bool in_c = on && x >= T.lo[0] && x < T.hi[0] && y >= T.lo[1] && y < T.hi[1];
+  const bool in_b = on && x >= T.lo[0] - 1 && x <= T.hi[0] && y >= T.lo[1] - 1 && y <= T.hi[1];
+  // Where this lane pulls from: the cell at x - c_x, y - c_y of the same
+  // plane.  Every lane pulls, so that the carried populations see no branch;
+  // one whose neighbours lie outside the tile reads itself and is not used.
+  // One address serves the populations that differ in c_z only (5 and 6, 7
+  // and 8, ...) in both planes; kept opaque, or the compiler holds a sum per
+  // population in registers it does not have.
+  const bool inside = in_b && !outer_xy;
+  int from[9];
+#pragma unroll
+  for (int c = 0; c < 9; ++c) {
+    const int q = pull_first(c);
+    const int nx = x - ax - kC[q][0], ny = y - ay - kC[q][1];
+    const int ncol = (ny >> 1) * wb + (nx >> 1);
+    const int at = inside ? (ncol >> 4) * 64 + (ny & 1) * 32 + (ncol & 15) * 2 + (nx & 1) : t;
+    from[c] = ((q - 1) * kSets * kFineCells + at) * (int)sizeof(S);
+    asm volatile("" : "+v"(from[c]));
+  }
+  auto pulled = [&](int set, int q) {
+    const int c = q <= 4 ? q - 1 : 4 + (q - 5) / 2;
+    const int more = ((q - pull_first(c)) * kSets + set) * kFineCells * (int)sizeof(S);
+    return *(const S*)((const char*)&planes[0][0][0] + from[c] + more);
+  };
+  const int sz = gx * gy;
+  const unsigned stored = y * P.row + x;
+  const unsigned ixy = y * gx + x;  // 8 * ixy < 2^32: a patch has fewer than 2^31 cells and at least 6 planes
+  const int a0 = max(T.lo[2] - (FINEST ? 2 : 1), 0), a1 = min(T.hi[2] + (FINEST ? 2 : 1), gz);
+
+  // Ghost cells take their source from the fill table; the entry of a plane
+  // is loaded a plane ahead, so that its latency is not added to the data's.
+  auto load_fill = [&](int z) -> unsigned long long {
+    if (!on || z >= a1 || (valid_xy && z >= 2 && z < gz - 2)) return 0;
+    return *(const unsigned long long*)((const char*)(fill + (P.fill_base + (long long)z * sz)) + ixy * 8u);
+  };
+  auto source = [&](int z, unsigned long long d, const S*& src, long long& stride) {
+    src = (const S*)((const char*)(fnow + (P.origin + (long long)z * P.plane)) + stored * (unsigned)sizeof(S));
+    stride = P.qs;
+    if (!(valid_xy && z >= 2 && z < gz - 2)) {
+      src = ((long long)d < 0 ? cnow : fnow) + (d & kFillElement);
+      stride = strides ? strides[(d & ~kFillParent) >> kFillStrideShift]
+                       : ((long long)d < 0 ? parent_stride : P.qs);
     }
+  };
+  // Populations [q0, q1) from src on, which moves on to q1.
+  auto load_some = [&](int q0, int q1, const S*& src, long long stride, S* f) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q)
+      if (q >= q0 && q < q1) {
+        f[q] = *src;
+        src += stride;
+      }
+  };
+
+  // carried for B (FINEST) and for C: next plane's c_z = 0 and +1
+  // populations, and the c_z = +1 ones of the plane after it
+  S b1[NV], b2[NV], c1[NV], c2[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) b1[q] = b2[q] = c1[q] = c2[q] = S(0);
+  // pulls from the plane in LDS: f = the populations of the plane below it;
+  // `rest` is this lane's own q = 0 there
+  auto advance = [&](int set, S rest, S* p1, S* p2, S* f) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
-      if (valid) out[P.base + q * P.qs + i] = f[q];
-      part[q][child][lb] = f[q];
+      const S v = q == 0 ? rest : pulled(set, q);
+      if (kC[q][2] < 0) {
+        f[q] = v;
+      } else {
+        f[q] = p1[q];
+        p1[q] = kC[q][2] == 0 ? v : p2[q];
+        if (kC[q][2] > 0) p2[q] = v;
+      }
+    }
+  };
+
+  // bit lateral(q): the cell - 2 c_q is valid in x and y
+  int keep_xy = 0;
+  if constexpr (AVG) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      const int xq = x - 2 * kC[q][0], yq = y - 2 * kC[q][1];
+      if (xq >= 2 && xq < gx - 2 && yq >= 2 && yq < gy - 2) keep_xy |= 1 << lateral(q);
     }
   }
-  __syncthreads();
-  for (int task = threadIdx.x; task < NV * kAvgBlocks; task += 8 * kAvgBlocks) {
-    const int q = task / kAvgBlocks, b = task % kAvgBlocks;
-    if (b0 + b >= nblk) continue;
-    double sum = 0.0;
+  // this lane's column of the block sums
+  const int tc = (t >> 6) * 16 + (t & 15);
+  const int tx = ax + 2 * (tc % wb), ty = ay + 2 * (tc / wb);
+  const bool task = tc < wb * hb && tx >= T.lo[0] && tx < T.hi[0] && ty >= T.lo[1] && ty < T.hi[1];
+  const int task_block = (ty >> 1) * (gx >> 1) + (tx >> 1);
+
+  S next[NV];  // A's next plane, loading
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};  // this lane's block sums, between a block's two planes
+  const S* src = fnow;
+  long long stride = 0;
+  if (on) {
+    source(a0, load_fill(a0), src, stride);
+    load_some(0, NV, src, stride, next);
+  }
+  unsigned long long fill_next = load_fill(a0 + 1);
+  // MASK: this cell's byte; SUM: its span in C's plane; both a plane ahead
+  auto load_mask = [&](int z) -> int {
+    return MASK && valid_xy && z >= 2 && z < gz - 2 ? mask[P.fill_base + (long long)z * sz + ixy] : 0;
+  };
+  auto load_span = [&](int z) -> long long {
+    return SUM && in_c && valid_xy && z >= max(T.lo[2], 2) && z < min(T.hi[2], gz - 2)
+               ? spans[P.fill_base + (long long)z * sz + ixy]
+               : -1;
+  };
+  int mask_next = load_mask(a0);
+  long long span_next = load_span(a0 - 1);
+  if (FINEST && on) {  // B is zero on the outer layer, first and last planes included
 #pragma unroll
-    for (int c = 0; c < 8; ++c) sum += to_f64(part[q][c][b], q, rho0);
-    avg[q * avg_stride + P.avg_base + b0 + b] = sum * 0.125;
+    for (int q = 1; q < NV; ++q) planes[q - 1][kB][t] = zero_pop<S>(q, r.rho0);
+  }
+  const int steps_behind = FINEST ? 2 : 1;
+  for (int k = a0; k < T.hi[2] + steps_behind; ++k) {
+    const bool more = k + 1 < a1;
+    // A: plane k.  Valid and ghost lanes hand their values over separately:
+    // joining them first costs a copy of every population.
+    S f[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) f[q] = next[q];
+    // A's next plane is loaded in three parts, before each stage: a wave that
+    // issues all of it at once waits ~50 cycles per load for the ones before.
+    const bool load = on && more;
+    if (load) {
+      source(k + 1, fill_next, src, stride);
+      load_some(0, kCut1, src, stride, next);
+    }
+    fill_next = load_fill(k + 2);
+    const bool masked = mask_next;
+    long long span = span_next;
+    int block = 0;  // the span's first contribution
+    if constexpr (MASK) mask_next = load_mask(k + 1);
+    if constexpr (SUM) {
+      if (span >= 0) block = contrib[span >> 32];
+      span_next = load_span(k);
+    }
+    S rest = zero_pop<S>(0, r.rho0);
+    auto hand_over = [&](int set) {
+#pragma unroll
+      for (int q = 1; q < NV; ++q) planes[q - 1][set][t] = f[q];
+      rest = f[0];
+    };
+    if (on && k < a1) {
+      if (valid_xy && k >= 2 && k < gz - 2) {
+        if (MASK && masked) {
+#pragma unroll
+          for (int q = 0; q < NV; ++q) f[q] = zero_pop<S>(q, r.rho0);
+        } else {
+          collide_s(f, r);
+        }
+        hand_over(0);
+      } else {
+        if (outer_xy || k == 0 || k == gz - 1) f[0] = zero_pop<S>(0, r.rho0);
+        hand_over(0);
+      }
+    }
+    if (load) load_some(kCut1, kCut2, src, stride, next);
+    // SUM: the span's first block (most cells have no other), loading
+    double added[NV];
+    if constexpr (SUM) {
+      if (span >= 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) added[q] = cavg[q * cavg_stride + block];
+      }
+    }
+    __syncthreads();
+    const int zc = k - steps_behind;
+    if constexpr (FINEST) {
+      // B: plane k - 1
+      const int zb = k - 1;
+      advance(0, rest, b1, b2, f);
+      rest = zero_pop<S>(0, r.rho0);
+      if (inside) {
+        if (zb < 1 || zb >= gz - 1) {  // an outer layer
+          if (zb == gz - 1) {
+#pragma unroll
+            for (int q = 1; q < NV; ++q) planes[q - 1][kB][t] = zero_pop<S>(q, r.rho0);
+          }
+        } else if (valid_xy && zb >= 2 && zb < gz - 2) {
+          collide_s(f, r);
+          hand_over(kB);
+        } else {
+          hand_over(kB);
+        }
+      }
+      __syncthreads();
+    }
+    if (load) load_some(kCut2, NV, src, stride, next);
+    // C: plane zc
+    S g[NV];
+    advance(kB, rest, c1, c2, g);
+    if constexpr (!FINEST) __syncthreads();  // C has read the A plane
+    const bool valid_c = valid_xy & (zc >= 2) & (zc < gz - 2);
+    if constexpr (SUM) {
+      if (span >= 0) {
+        double acc[NV];
+#pragma unroll
+        for (int q = 0; q < NV; ++q) acc[q] = to_f64(g[q], q, r.rho0) + added[q];
+        const int first = int(span >> 32), n = int(span & 0xffffffffll);
+        for (int j = first + 1; j < first + n; ++j) {
+          const long long c = contrib[j];
+#pragma unroll
+          for (int q = 0; q < NV; ++q) acc[q] += cavg[q * cavg_stride + c];
+        }
+#pragma unroll
+        for (int q = 0; q < NV; ++q) g[q] = from_f64<S>(acc[q], q, r.rho0);
+      }
+    }
+    if constexpr (AVG) {
+      // The wave's 16 columns x 15 populations are 240 tasks: in round j lane
+      // l sums population 1 + 4 j + l / 16 of the wave's column l % 16 (0 for
+      // 15, which passes through the first plane once its population is done).
+      // The outer layer is zero; ZeroInvalidComponents: population q of
+      // another ghost cell survives only if the cell - 2 c_q is valid.
+      if (zc >= T.lo[2]) {
+        const bool outer = outer_xy | (zc <= 0) | (zc >= gz - 1);
+        auto meet = [&](int q, int at) {
+          const int zq = zc - 2 * kC[q][2];
+          const bool keep = valid_c | (!outer & ((keep_xy & 1 << lateral(q)) != 0) & (zq >= 2) & (zq < gz - 2));
+          if (in_c) {
+            planes[at][0][t] = g[q];
+            if (!keep) planes[at][0][t] = zero_pop<S>(q, r.rho0);
+          }
+        };
+        int lane = t;
+        asm volatile("" : "+v"(lane));  // no address per round held in registers
+        const int task_cell = (lane & ~63) + 2 * (lane & 15);
+        double* here = avg + P.avg_base + (long long)(zc >> 1) * ((gx >> 1) * (gy >> 1));
+#pragma unroll
+        for (int q = 1; q < NV; ++q) meet(q, q - 1);
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (j == 3) {
+            wave_sync();
+            meet(0, 0);
+            wave_sync();
+          }
+          const int q = 1 + 4 * j + (lane >> 4 & 3), qq = q < NV ? q : 0;
+          if (task && q <= NV) {
+            double s = (zc & 1) ? sum[j] : 0.0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              s += to_f64_any(planes[q < NV ? q - 1 : 0][0][task_cell + (c & 1) + 32 * (c >> 1)], qq, r.rho0);
+            sum[j] = s;
+            if (zc & 1) here[qq * avg_stride + task_block] = s * 0.125;
+          }
+        }
+      }
+    }
+    // The next plane's loads are waited for here, before the stores are
+    // issued: a wait after them would be for the stores as well.
+#pragma unroll
+    for (int q = 0; q < NV; ++q) asm volatile("" : "+v"(next[q]));
+    asm volatile("" : "+v"(fill_next));
+    if constexpr (MASK) asm volatile("" : "+v"(mask_next));
+    if constexpr (SUM) asm volatile("" : "+v"(span_next));
+    if (in_c & valid_c & (zc >= T.lo[2])) {
+      S* out = fnext + (P.origin + (long long)zc * P.plane);
+#pragma unroll
+      for (int q = 0; q < NV; ++q) *(S*)((char*)(out + q * P.qs) + stored * (unsigned)sizeof(S)) = g[q];
+    }
   }
 }
 
@@ -522,12 +779,11 @@ __global__ __launch_bounds__(256) void k_fine_avg_valid(const S* __restrict__ f,
 }
 
 // DistFnFillFromCoarse (src/AmrSim.cpp:393-411): valid fine cells take the
-// coarse value of their parent; ghosts are zeroed (they are rewritten before
-// they are read).
+// coarse value of their parent (ghosts are filled before they are read).
 template <typename S>
 __global__ __launch_bounds__(256) void k_fine_from_coarse(S* __restrict__ fnow, const S* __restrict__ cnow,
                                                           Lattice clat, const PatchDesc* __restrict__ patches,
-                                                          double rho0, int ratio) {
+                                                          int ratio) {
   const PatchDesc P = patches[blockIdx.y];
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= P.cells) return;
@@ -535,20 +791,17 @@ __global__ __launch_bounds__(256) void k_fine_from_coarse(S* __restrict__ fnow, 
   patch_coords(P, i, gx, gy, gz);
   if (patch_valid(P, gx, gy, gz)) {
     const int x = (P.lo[0] - 2 + gx) / ratio, y = (P.lo[1] - 2 + gy) / ratio, z = (P.lo[2] - 2 + gz) / ratio;
-    const long long c = clat.at(0, y * clat.nx + x, z);
+    const long long c = clat.at(0, y * clat.nx + x, z), to = P.at(gx, gy, gz);
 #pragma unroll
-    for (int q = 0; q < NV; ++q) fnow[P.base + q * P.qs + i] = cnow[c + q * clat.ps];
-  } else {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) fnow[P.base + q * P.qs + i] = zero_pop<S>(q, rho0);
+    for (int q = 0; q < NV; ++q) fnow[to + q * P.qs] = cnow[c + q * clat.ps];
   }
 }
 
 // RemakeLevel's fill (src/AmrSim.cpp:715-744 via DistFnFillPatch): each
 // valid cell of the new patches copies its populations from an old fine
-// patch (src >= 0: (old patch << 32) | old grown index) or from its coarse
-// parent (src < 0: -1 - coarse element of population 0, or with PC
-// -1 - ((coarse patch << 32) | grown index)).  With every source a parent it
+// patch (src >= 0: (old patch << 32) | element from its base) or from its
+// coarse parent (src < 0: -1 - coarse element of population 0, or with PC
+// -1 - ((coarse patch << 32) | element from its base)).  With every source a parent it
 // is DistFnFillFromCoarse on a level whose parent is patched.
 template <typename S, bool PC>
 __global__ __launch_bounds__(256) void k_fine_remake(S* __restrict__ fnew, const S* __restrict__ fold,
@@ -579,8 +832,9 @@ __global__ __launch_bounds__(256) void k_fine_remake(S* __restrict__ fnew, const
     from = cnow + (-1 - d);
     stride = clat.ps;
   }
+  const long long to = P.at(gx, gy, gz);
 #pragma unroll
-  for (int q = 0; q < NV; ++q) fnew[P.base + q * P.qs + i] = from[q * stride];
+  for (int q = 0; q < NV; ++q) fnew[to + q * P.qs] = from[q * stride];
 }
 
 // Valid cells of one patch <-> packed FP64 f [15][nz][ny][nx]; hydro of one
@@ -594,17 +848,17 @@ __global__ __launch_bounds__(256) void k_patch_io(S* __restrict__ f, const Patch
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const int x = i % nx, t = i / nx, y = t % ny, z = t / ny;
-  const long long li = ((long long)(z + 2) * P.g[1] + (y + 2)) * P.g[0] + (x + 2);
+  const long long li = P.at(x + 2, y + 2, z + 2);
   if (OP == 0) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) a[(long long)q * n + i] = to_f64(f[P.base + q * P.qs + li], q, rho0);
+    for (int q = 0; q < NV; ++q) a[(long long)q * n + i] = to_f64(f[li + q * P.qs], q, rho0);
   } else if (OP == 1) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) f[P.base + q * P.qs + li] = from_f64<S>(a[(long long)q * n + i], q, rho0);
+    for (int q = 0; q < NV; ++q) f[li + q * P.qs] = from_f64<S>(a[(long long)q * n + i], q, rho0);
   } else {
     double g[NV];
 #pragma unroll
-    for (int q = 0; q < NV; ++q) g[q] = to_f64(f[P.base + q * P.qs + li], q, rho0);
+    for (int q = 0; q < NV; ++q) g[q] = to_f64(f[li + q * P.qs], q, rho0);
     double rr, u0, u1, u2;
     hydro_f64(g, rr, u0, u1, u2);
     a[i] = rr;
@@ -632,19 +886,19 @@ hipError_t patch_io(int op, S* f, const PatchDesc* patches, int b, int valid_cel
 template <typename S>
 hipError_t fill_collide(const S* fnow, S* fnext, const S* cnow, const Lattice& clat, const PatchDesc* cpatches,
                         const PatchDesc* patches, const PatchDesc* own, int first, const long long* fill,
-                        const unsigned char* mask, const Relax& r, long long oshift, dim3 grid, hipStream_t st) {
+                        const unsigned char* mask, const Relax& r, dim3 grid, hipStream_t st) {
   if (cpatches && mask)
     k_fine_fill_collide<S, true, true><<<grid, 256, 0, st>>>(fnow, fnext, cnow, clat, cpatches, patches, own, first,
-                                                             fill, mask, r, oshift);
+                                                             fill, mask, r);
   else if (cpatches)
     k_fine_fill_collide<S, true, false><<<grid, 256, 0, st>>>(fnow, fnext, cnow, clat, cpatches, patches, own,
-                                                              first, fill, mask, r, oshift);
+                                                              first, fill, mask, r);
   else if (mask)
     k_fine_fill_collide<S, false, true><<<grid, 256, 0, st>>>(fnow, fnext, cnow, clat, cpatches, patches, own,
-                                                              first, fill, mask, r, oshift);
+                                                              first, fill, mask, r);
   else
     k_fine_fill_collide<S, false, false><<<grid, 256, 0, st>>>(fnow, fnext, cnow, clat, cpatches, patches, own,
-                                                               first, fill, mask, r, oshift);
+                                                               first, fill, mask, r);
   return hipGetLastError();
 }
 
@@ -652,7 +906,7 @@ hipError_t launch_fine_fill_collide(int precision, const void* fnow, void* fnext
                                     const Lattice& clat, const PatchDesc* cpatches, const PatchDesc* patches,
                                     const PatchDesc* own, int first, int npatch, int max_cells,
                                     const long long* fill, const unsigned char* mask, const Relax& r,
-                                    hipStream_t st, long long oshift) {
+                                    hipStream_t st) {
   // A multiple of 8 workgroups per patch, so that xcd_chunk() gives each XCD
   // the same slab of every patch: the rows whose first or last two cells an
   // x-neighbour's ghost fill reads (and the rows a y-neighbour's reads) are
@@ -661,74 +915,57 @@ hipError_t launch_fine_fill_collide(int precision, const void* fnow, void* fnext
   const dim3 grid(((max_cells + 255) / 256 + 7) / 8 * 8, npatch);
   if (precision == 0)
     return fill_collide((const double*)fnow, (double*)fnext, (const double*)cnow, clat, cpatches, patches, own,
-                        first, fill, mask, r, oshift, grid, st);
+                        first, fill, mask, r, grid, st);
   return fill_collide((const float*)fnow, (float*)fnext, (const float*)cnow, clat, cpatches, patches, own, first,
-                      fill, mask, r, oshift, grid, st);
+                      fill, mask, r, grid, st);
 }
 
 hipError_t launch_fine_stream_zero(int precision, const void* in, void* out, const PatchDesc* patches, int first,
-                                   int npatch, int max_cells, double rho0, const int* slot, const double* avg,
-                                   long long avg_stride, const int* start, const int* contrib, hipStream_t st,
-                                   long long ishift) {
+                                   int npatch, int max_cells, double rho0, const long long* spans,
+                                   const double* avg, long long avg_stride, const int* contrib, hipStream_t st) {
   const dim3 grid(((max_cells + 255) / 256 + 7) / 8 * 8, npatch);  // for xcd_chunk()
   if (precision == 0)
-    k_fine_stream_zero<double><<<grid, 256, 0, st>>>((const double*)in, (double*)out, patches, first, rho0, slot,
-                                                     avg, avg_stride, start, contrib, ishift);
+    k_fine_stream_zero<double><<<grid, 256, 0, st>>>((const double*)in, (double*)out, patches, first, rho0, spans,
+                                                     avg, avg_stride, contrib);
   else
-    k_fine_stream_zero<float><<<grid, 256, 0, st>>>((const float*)in, (float*)out, patches, first, rho0, slot, avg,
-                                                    avg_stride, start, contrib, ishift);
+    k_fine_stream_zero<float><<<grid, 256, 0, st>>>((const float*)in, (float*)out, patches, first, rho0, spans, avg,
+                                                    avg_stride, contrib);
   return hipGetLastError();
 }
 
-// Grid of k_fine_stream_avg<S>: a multiple of 8 workgroups per patch, for
-// xcd_chunk(); each workgroup has 8 avg_blocks<S>() threads.
 template <typename S>
-dim3 avg_grid(int max_blocks, int npatch) {
-  constexpr int ab = avg_blocks<S>();
-  return dim3(((max_blocks + ab - 1) / ab + 7) / 8 * 8, npatch);
-}
-
-hipError_t launch_middle_stream_avg(int precision, const void* in, long long ishift, void* out, double* avg,
-                                   long long avg_stride, const PatchDesc* patches, int first, int npatch,
-                                   int max_blocks, double rho0, const int* slot, const double* cavg,
-                                   long long cavg_stride, const int* start, const int* contrib, hipStream_t st) {
-  if (precision == 0)
-    k_fine_stream_avg<double, true><<<avg_grid<double>(max_blocks, npatch), 8 * avg_blocks<double>(), 0, st>>>(
-        (const double*)in, (double*)out, avg, avg_stride, patches, first, rho0, ishift, slot, cavg, cavg_stride,
-        start, contrib);
+static hipError_t fine_step(const FineStep& a, dim3 grid, hipStream_t st) {
+#define LBX_FINE_STEP(FINEST, MIDDLE, AVG)                                                                     \
+  k_fine_step<S, FINEST, MIDDLE, MIDDLE, AVG><<<grid, kFineThreads, 0, st>>>(                                   \
+      (const S*)a.now, (S*)a.next, (const S*)a.parent, a.own, a.tiles, a.ntiles, a.fill, a.strides,             \
+      a.parent_stride, a.mask, a.relax, a.avg, a.avg_stride, a.spans, a.cavg, a.cavg_stride, a.contrib)
+  if (a.finest)
+    LBX_FINE_STEP(true, false, true);
+  else if (a.avg)
+    LBX_FINE_STEP(false, true, true);
   else
-    k_fine_stream_avg<float, true><<<avg_grid<float>(max_blocks, npatch), 8 * avg_blocks<float>(), 0, st>>>(
-        (const float*)in, (float*)out, avg, avg_stride, patches, first, rho0, ishift, slot, cavg, cavg_stride, start,
-        contrib);
+    LBX_FINE_STEP(false, true, false);
+#undef LBX_FINE_STEP
   return hipGetLastError();
 }
 
-hipError_t launch_fine_stream_collide(int precision, const void* in, void* out, long long oshift,
+hipError_t launch_fine_step(int precision, const FineStep& a, hipStream_t st) {
+  const dim3 grid((a.ntiles + 7) / 8 * 8);
+  return precision == 0 ? fine_step<double>(a, grid, st) : fine_step<float>(a, grid, st);
+}
+
+hipError_t launch_fine_stream_collide(int precision, const void* in, void* out,
                                       const PatchDesc* patches, int first, int npatch, int max_cells, const Relax& r,
                                       hipStream_t st, bool inner) {
   const dim3 grid(((max_cells + 255) / 256 + 7) / 8 * 8, npatch);  // for xcd_chunk()
   if (precision == 0 && inner)
-    k_fine_stream_collide<double, true><<<grid, 256, 0, st>>>((const double*)in, (double*)out, patches, first, r,
-                                                              oshift);
+    k_fine_stream_collide<double, true><<<grid, 256, 0, st>>>((const double*)in, (double*)out, patches, first, r);
   else if (precision == 0)
-    k_fine_stream_collide<double><<<grid, 256, 0, st>>>((const double*)in, (double*)out, patches, first, r, oshift);
+    k_fine_stream_collide<double><<<grid, 256, 0, st>>>((const double*)in, (double*)out, patches, first, r);
   else if (inner)
-    k_fine_stream_collide<float, true><<<grid, 256, 0, st>>>((const float*)in, (float*)out, patches, first, r,
-                                                             oshift);
+    k_fine_stream_collide<float, true><<<grid, 256, 0, st>>>((const float*)in, (float*)out, patches, first, r);
   else
-    k_fine_stream_collide<float><<<grid, 256, 0, st>>>((const float*)in, (float*)out, patches, first, r, oshift);
-  return hipGetLastError();
-}
-
-hipError_t launch_fine_stream_avg(int precision, const void* in, long long ishift, void* out, double* avg,
-                                  long long avg_stride, const PatchDesc* patches, int first, int npatch,
-                                  int max_blocks, double rho0, hipStream_t st) {
-  if (precision == 0)
-    k_fine_stream_avg<double><<<avg_grid<double>(max_blocks, npatch), 8 * avg_blocks<double>(), 0, st>>>(
-        (const double*)in, (double*)out, avg, avg_stride, patches, first, rho0, ishift);
-  else
-    k_fine_stream_avg<float><<<avg_grid<float>(max_blocks, npatch), 8 * avg_blocks<float>(), 0, st>>>(
-        (const float*)in, (float*)out, avg, avg_stride, patches, first, rho0, ishift);
+    k_fine_stream_collide<float><<<grid, 256, 0, st>>>((const float*)in, (float*)out, patches, first, r);
   return hipGetLastError();
 }
 
@@ -758,13 +995,13 @@ hipError_t launch_sum_apply(int precision, const double* avg, long long avg_stri
 }
 
 hipError_t launch_fine_from_coarse(int precision, void* fnow, const void* cnow, const Lattice& clat,
-                                   const PatchDesc* patches, int npatch, int max_cells, double rho0, int ratio,
+                                   const PatchDesc* patches, int npatch, int max_cells, int ratio,
                                    hipStream_t st) {
   const dim3 grid((max_cells + 255) / 256, npatch);
   if (precision == 0)
-    k_fine_from_coarse<double><<<grid, 256, 0, st>>>((double*)fnow, (const double*)cnow, clat, patches, rho0, ratio);
+    k_fine_from_coarse<double><<<grid, 256, 0, st>>>((double*)fnow, (const double*)cnow, clat, patches, ratio);
   else
-    k_fine_from_coarse<float><<<grid, 256, 0, st>>>((float*)fnow, (const float*)cnow, clat, patches, rho0, ratio);
+    k_fine_from_coarse<float><<<grid, 256, 0, st>>>((float*)fnow, (const float*)cnow, clat, patches, ratio);
   return hipGetLastError();
 }
 
