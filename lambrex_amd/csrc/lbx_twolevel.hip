@@ -339,8 +339,8 @@ __global__ __launch_bounds__(256) void k_fine_stream_zero(const S* __restrict__ 
 // replaces (fill + collide, stream + collide, stream + average; each reading
 // and writing every patch, in groups kept in the MALL) moved 7.7 valid-cell
 // transfers per pair of substeps and ran at the fabric's rate.  128 patches of
-// 36^3 (64 of 32^3 valid cells each way), two substeps: FP64 750 us before,
-// 445 us so, of which a plane's two collisions and pulls are about 60 %; one
+// 36^3 grown cells (64x256x256 in boxes of 32^3), two substeps: FP64 750 us
+// before, 437 us so, of which a plane's two collisions and pulls are about 60 %; one
 // workgroup a CU (114 KB of LDS, 2 waves a SIMD at 256 registers).  Slower: 12
 // waves on tiles of 36 x 20 cells at 168 registers (484 us), the loads of a
 // plane in one piece or after the first barrier (503 to 627 us).
