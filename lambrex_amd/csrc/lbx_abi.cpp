@@ -19,12 +19,14 @@
 #include <tuple>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <new>
 #include <string>
 #include <vector>
 
 #include "../../include/lbx.h"
 #include "lbx_internal.h"
+#include "lbx_readback.h"
 
 using lbx::Lattice;
 using lbx::LaunchShape;
@@ -139,6 +141,7 @@ struct lbx_ctx {
   // every call that uses it synchronises before returning)
   void* stage = nullptr;
   size_t stage_bytes = 0;
+  lbx::ReadBack readback;  // its ring is kept until destroy
   // profiling of stream-collide launches
   bool prof = false;
   std::vector<hipEvent_t> ev_pool;
@@ -301,6 +304,10 @@ hipError_t stage_buffer(lbx_ctx* ctx, size_t bytes, void** out) {
   }
   *out = ctx->stage;
   return hipSuccess;
+}
+
+hipError_t read_back(lbx_ctx* ctx, std::initializer_list<lbx::ReadBack::Part> parts) {
+  return ctx->readback.copy(ctx->device, parts.begin(), (int)parts.size(), ctx->stream);
 }
 
 // Fold recorded event pairs into the running total.
@@ -1407,6 +1414,7 @@ hipError_t scratch_setup(int device) {
 
 int lbx::ctx_device(const lbx_ctx* ctx) { return ctx->device; }
 hipStream_t lbx::ctx_stream(const lbx_ctx* ctx) { return ctx->stream; }
+lbx::ReadBack& lbx::ctx_readback(lbx_ctx* ctx) { return ctx->readback; }
 
 extern "C" {
 
@@ -1462,6 +1470,7 @@ int lbx_ctx_destroy(lbx_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->push);
   if (ctx->sums) (void)hipFree(ctx->sums);
   if (ctx->stage) (void)hipFree(ctx->stage);
+  ctx->readback.release();
   (void)hipEventDestroy(ctx->join_ev);
   (void)hipEventDestroy(ctx->fork_ev);
   (void)hipStreamDestroy(ctx->side);
@@ -1567,8 +1576,7 @@ int lbx_tag_cells(lbx_sim* sim, int level, int criterion, double threshold, uint
   LBX_HIP(ctx, stage_buffer(ctx, n, &t));
   LBX_HIP(ctx, lbx::launch_tag(sim->precision, L.post, criterion, L.buf[L.cur], L.lat, sim->rho0,
                                threshold * threshold, (unsigned char*)t, ctx->stream));
-  LBX_HIP(ctx, hipMemcpyAsync(tags, t, n, hipMemcpyDeviceToHost, ctx->stream));
-  LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  LBX_HIP(ctx, read_back(ctx, {{tags, t, n}}));
   return LBX_OK;
 }
 
@@ -1708,8 +1716,7 @@ int lbx_download_f(lbx_sim* sim, int level, int box, double* f) {
   else
     LBX_HIP(ctx, lbx::launch_pack_f(sim->precision, L.post, L.buf[L.cur], L.lat, region_of(L.boxes[box]),
                                     (double*)t, sim->rho0, ctx->stream));
-  LBX_HIP(ctx, hipMemcpyAsync(f, t, n * lbx::NV_TOTAL * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  LBX_HIP(ctx, read_back(ctx, {{f, t, n * lbx::NV_TOTAL * sizeof(double)}}));
   return LBX_OK;
 }
 
@@ -1770,9 +1777,7 @@ int lbx_hydro(lbx_sim* sim, int level, int box, double* rho, double* u) {
   else
     LBX_HIP(ctx, lbx::launch_hydro(sim->precision, L.post, L.buf[L.cur], L.lat, region_of(L.boxes[box]), drho,
                                    du, sim->rho0, ctx->stream));
-  LBX_HIP(ctx, hipMemcpyAsync(rho, drho, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  LBX_HIP(ctx, hipMemcpyAsync(u, du, 3 * n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  LBX_HIP(ctx, read_back(ctx, {{rho, drho, n * sizeof(double)}, {u, du, 3 * n * sizeof(double)}}));
   return LBX_OK;
 }
 
@@ -1801,9 +1806,7 @@ int lbx_hydro_level(lbx_sim* sim, int level, double* rho, double* u) {
                                      drho + off, du + 3 * off, sim->rho0, ctx->stream));
     off += n;
   }
-  LBX_HIP(ctx, hipMemcpyAsync(rho, drho, total * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  LBX_HIP(ctx, hipMemcpyAsync(u, du, 3 * total * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  LBX_HIP(ctx, read_back(ctx, {{rho, drho, total * sizeof(double)}, {u, du, 3 * total * sizeof(double)}}));
   return LBX_OK;
 }
 

@@ -41,6 +41,7 @@
 
 #include "../../include/lbx.h"
 #include "lbx_internal.h"
+#include "lbx_readback.h"
 
 using lbx::ServeBatch;
 using lbx::ServeRun;
@@ -135,6 +136,7 @@ struct lbx_server {
   lbx_ctx* ctx = nullptr;
   int device = 0;
   hipStream_t stream = nullptr;
+  hipStream_t out = nullptr;  // fields of finished runs
   int precision = LBX_FP32_SHIFTED;
   double rho0 = 1.0;
   int max_active = lbx::kServeMaxRuns;
@@ -467,8 +469,8 @@ int deliver_refined(lbx_server* s, Run& r) {
 }
 
 // Deliver runs whose sums have reached the host; optional field outputs are
-// copied synchronously (the run's arena space is still intact), then the
-// arena space and the slot are released.
+// copied (the call waits for them), then the arena space and the slot are
+// released.
 int collect(lbx_server* s, bool wait) {
   for (size_t i = 0; i < s->active.size();) {
     Run& r = s->active[i];
@@ -503,20 +505,21 @@ int collect(lbx_server* s, bool wait) {
     res.t_submit = r.r.t_submit;
     res.t_admit = r.t_admit;
     res.t_done = now_s();
+    // The run's last state is complete and stays until its arena space is
+    // released: its outputs go by a stream of their own, beside the steps
+    // already queued for the other runs.
     if (rq.out_rho || rq.out_u) {
-      SRV_HIP(s, lbx::launch_hydro(s->precision, false, fin, L, R, s->staging, s->staging + n, s->rho0, s->stream));
-      if (rq.out_rho)
-        SRV_HIP(s, hipMemcpyAsync(rq.out_rho, s->staging, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-      if (rq.out_u)
-        SRV_HIP(s, hipMemcpyAsync(rq.out_u, s->staging + n, 3 * n * sizeof(double), hipMemcpyDeviceToHost,
-                                  s->stream));
-      SRV_HIP(s, hipStreamSynchronize(s->stream));
+      SRV_HIP(s, lbx::launch_hydro(s->precision, false, fin, L, R, s->staging, s->staging + n, s->rho0, s->out));
+      lbx::ReadBack::Part parts[2];
+      int k = 0;
+      if (rq.out_rho) parts[k++] = {rq.out_rho, s->staging, n * sizeof(double)};
+      if (rq.out_u) parts[k++] = {rq.out_u, s->staging + n, 3 * n * sizeof(double)};
+      SRV_HIP(s, lbx::ctx_readback(s->ctx).copy(s->device, parts, k, s->out));
     }
     if (rq.out_f) {
-      SRV_HIP(s, lbx::launch_pack_f(s->precision, false, fin, L, R, s->staging, s->rho0, s->stream));
-      SRV_HIP(s, hipMemcpyAsync(rq.out_f, s->staging, lbx::NV_TOTAL * n * sizeof(double),
-                                hipMemcpyDeviceToHost, s->stream));
-      SRV_HIP(s, hipStreamSynchronize(s->stream));
+      SRV_HIP(s, lbx::launch_pack_f(s->precision, false, fin, L, R, s->staging, s->rho0, s->out));
+      const lbx::ReadBack::Part part{rq.out_f, s->staging, lbx::NV_TOTAL * n * sizeof(double)};
+      SRV_HIP(s, lbx::ctx_readback(s->ctx).copy(s->device, &part, 1, s->out));
     }
     s->lattice_updates += n * (int64_t)rq.steps;
     s->arena.release(r.off, r.bytes);
@@ -615,6 +618,7 @@ int lbx_serve_create(lbx_ctx* ctx, int precision, double rho0, size_t arena_byte
   // bounded for very long lists.
   s->grid = std::max(1, cus) * 4096;
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->out, hipStreamNonBlocking);
   if (e == hipSuccess && arena_bytes == 0) {
     size_t fr = 0, tot = 0;
     e = hipMemGetInfo(&fr, &tot);
@@ -668,6 +672,7 @@ int lbx_serve_destroy(lbx_server* s) {
   for (int k = 0; k < lbx::kServeMaxRuns; ++k)
     if (s->slot_ev[k]) (void)hipEventDestroy(s->slot_ev[k]);
   if (s->stream) (void)hipStreamDestroy(s->stream);
+  if (s->out) (void)hipStreamDestroy(s->out);
   delete s;
   return LBX_OK;
 }
