@@ -414,6 +414,12 @@ __global__ __launch_bounds__(256) void k_hydro(const S* __restrict__ f, Lattice 
   u[2 * n + i] = u2;
 }
 
+constexpr int kTagX = 32, kTagY = 16;  // k_tag_gradient's tile
+constexpr int kTagGroups = 1024;       // and the workgroups it cuts z for
+// Cells from which a tile pays: k_tag against it, 32^3 6.4 and 8.8 us (FP32
+// 6.8 and 8.2), 48^3 13.4 and 10.7 (9.7 and 8.2).
+constexpr long long kTagTiled = 64000;
+
 // ErrorEst on device data: tag[c] = 1 (c = (z*ny + y)*nx + x) where
 // CRIT 0: |grad rho|^2 > thr2, central differences with periodic wrap;
 // CRIT 1: |u|^2 > thr2.  rho and u are exactly what k_hydro returns.
@@ -448,6 +454,58 @@ __global__ __launch_bounds__(256) void k_tag(const S* __restrict__ f, Lattice L,
     s = u0 * u0 + u1 * u1 + u2 * u2;
   }
   tag[c] = s > thr2 ? 1 : 0;
+}
+
+// k_tag's criterion 0 with each density formed once per tile instead of six
+// times: a workgroup marches a tile of kTagX x kTagY cells, its outer ring
+// included, through `depth` planes of z; the densities of the plane below and
+// above are the lane's own, those beside it come through LDS.  Bound by the
+// cells' one read: 192x160x128 after a step 354 -> 123 us (FP32 190 -> 90),
+// 256^3 1495 -> 605 us (788 -> 370); 178 us with the tiles dealt to the XCDs in
+// turn, 156 and 149 us with tiles of 64x16 and 64x8.
+template <typename S, bool PULL>
+__global__ __launch_bounds__(kTagX* kTagY) void k_tag_gradient(const S* __restrict__ f, Lattice L, double rho0,
+                                                               double thr2, int tx, int ty,
+                                                               int groups, int depth,
+                                                               unsigned char* __restrict__ tag) {
+  __shared__ double plane[2][kTagY][kTagX];
+  const int lx = threadIdx.x, ly = threadIdx.y;
+  const int w = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);  // an XCD takes neighbouring tiles
+  if (w >= groups) return;
+  const int x = (w % tx) * (kTagX - 2) + lx - 1, y = (w / tx % ty) * (kTagY - 2) + ly - 1;
+  const int z0 = w / (tx * ty) * depth, z1 = min(z0 + depth, L.nz);
+  const bool on = x <= L.nx && y <= L.ny;
+  const bool inner = lx > 0 && lx < kTagX - 1 && ly > 0 && ly < kTagY - 1 && x < L.nx && y < L.ny;
+  const int wx = x < 0 ? L.nx - 1 : x == L.nx ? 0 : x, wy = y < 0 ? L.ny - 1 : y == L.ny ? 0 : y;
+  auto density = [&](int z) {
+    double g[NV], r, u0, u1, u2;
+    cell_at<S, PULL>(f, L, wx, wy, z < 0 ? L.nz - 1 : z == L.nz ? 0 : z, rho0, g);
+    hydro_f64(g, r, u0, u1, u2);
+    return r;
+  };
+  double below = 0.0, here = 0.0, above = 0.0;
+  if (on) {
+    below = density(z0 - 1);
+    here = density(z0);
+    plane[z0 & 1][ly][lx] = here;
+  }
+  for (int z = z0; z < z1; ++z) {
+    __syncthreads();  // plane z is there, and the one it replaces has been read
+    if (on) {
+      above = density(z + 1);
+      plane[(z + 1) & 1][ly][lx] = above;
+    }
+    if (inner) {
+      const double(&p)[kTagY][kTagX] = plane[z & 1];
+      const double gx = (p[ly][lx + 1] - p[ly][lx - 1]) * 0.5;
+      const double gy = (p[ly + 1][lx] - p[ly - 1][lx]) * 0.5;
+      const double gz = (above - below) * 0.5;
+      const double s = gx * gx + gy * gy + gz * gz;
+      tag[((long long)z * L.ny + y) * L.nx + x] = s > thr2 ? 1 : 0;
+    }
+    below = here;
+    here = above;
+  }
 }
 
 // Block sum of 4 doubles in a fixed order: wavefront butterfly, then the
@@ -719,10 +777,18 @@ hipError_t launch_hydro(int precision, bool pull, const void* f, const Lattice& 
 template <typename S, bool PULL>
 static void tag_launch(int criterion, const S* f, const Lattice& L, double rho0, double thr2, unsigned char* tag,
                 int blocks, hipStream_t st) {
-  if (criterion == 0)
-    k_tag<S, 0, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
-  else
-    k_tag<S, 1, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
+  if (criterion == 1)
+    return k_tag<S, 1, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
+  if ((long long)L.nx * L.ny * L.nz < kTagTiled)
+    return k_tag<S, 0, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
+  const int tx = (L.nx + kTagX - 3) / (kTagX - 2), ty = (L.ny + kTagY - 3) / (kTagY - 2);
+  const long long columns = (long long)tx * ty;
+  const long long want = columns * L.nz / kTagGroups;  // planes per workgroup that leave kTagGroups of them
+  const int depth = want < 2 ? 2 : want > 32 ? 32 : (int)want;
+  const int tz = (L.nz + depth - 1) / depth;
+  const int groups = tx * ty * tz;
+  k_tag_gradient<S, PULL><<<(groups + 7) / 8 * 8, dim3(kTagX, kTagY), 0, st>>>(f, L, rho0, thr2, tx, ty, groups, depth,
+                                                                              tag);
 }
 
 hipError_t launch_tag(int precision, bool pull, int criterion, const void* f, const Lattice& L, double rho0,
