@@ -257,8 +257,8 @@ int lbx_bench_copy(lbx_ctx* ctx, size_t bytes, int reps, double* gbs);
  * 2,236,962 cells; 128^3 fits), or, with fine boxes, a two-level run
  * (ratio 2) stepped by the Rohde cycle (src/AmrSim.cpp:430-469).
  * Single-level requests are admitted while the server's device arena has
- * room and advance together, one patch-list kernel launch per step over the
- * work items of every active run; a refined run is admitted while the
+ * room and advance together, one patch-list kernel launch per step (or per two,
+ * where that is faster) over the work items of every active run; a refined run is admitted while the
  * device has memory for its levels, is held in a simulation of its own on
  * the context (one captured level-0 step per server step, on the context's
  * stream, overlapping the patch-list launches on the server's stream) and

@@ -262,22 +262,29 @@ hipError_t launch_patch_io(int precision, int op, void* f, const PatchDesc* patc
 // Serving: one active run of the batch, passed by value in the kernel
 // arguments (kServeMaxRuns * sizeof(ServeRun) stays under 4 KB).
 struct ServeRun {
-  void* buf[2];      // state buffers (pass p reads buf[p & 1])
+  const void* src;   // state buffers of this launch
+  void* dst;
   int n[3];          // lattice extents
-  int item_begin;    // first work item (256 cells, x fastest) of this run in the batch
-  int steps;         // LB steps of the run (passes 0..steps)
-  long long start;   // global step of pass 0
+  int item_begin;    // first work item of this run in the batch
+  int kind;          // one pass: a StepKind; two: ServePair bits
+  short bx, by;      // two passes: a work item is a column of bx x by cells ...
+  int depth;         // ... through `depth` planes; one: 256 cells, x fastest
   long long ps;      // population-plane stride of the run's lattice (zs = 15 ps)
   double omega_s, omega_b, rho0;
 };
+// The two passes of a launch in one: C and S of the first, C of the second
+// (which always streams): collide + fused, two fused, fused + stream, or, with
+// none, the stream-only pass alone.
+enum ServePair { PAIR_PULL = 1, PAIR_COLLIDE1 = 2, PAIR_COLLIDE2 = 4 };
+constexpr int kServePairCells = 640;  // cells of a column and the ring around it
 constexpr int kServeMaxRuns = 44;
 struct ServeBatch {
   ServeRun run[kServeMaxRuns];
   int nruns;
   int total_items;
 };
-hipError_t launch_serve_step(int precision, const ServeBatch& b, long long step, int grid,
-                             hipStream_t st);
+hipError_t launch_serve_step(int precision, const ServeBatch& b, int grid, hipStream_t st);
+hipError_t launch_serve_pair(int precision, const ServeBatch& b, hipStream_t st);
 hipError_t launch_serve_init_pulse(int precision, void* f, const Lattice& L, int axis, int plane,
                                    double amplitude, double rho0, hipStream_t st);
 

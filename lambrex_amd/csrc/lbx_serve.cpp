@@ -8,8 +8,9 @@
 // does not fit; LBX_SERVE_SHORTEST_FIRST admits the queued requests in order
 // of their work (cells x steps, ties by arrival), skipping any that do not
 // fit yet.  All
-// active runs advance together: one patch-list kernel launch per global step
-// walks the patch list of every active run.  At most kInFlight steps are
+// active runs advance together: one patch-list kernel launch per global step, or
+// per two of them where that is faster, walks the patch list of every active
+// run.  At most kInFlight steps are
 // queued ahead of the GPU, so admission and completion are observed within a
 // few steps.  A run finishes with its stream-only pass; once the GPU has
 // executed it, its FP64 sums (reduced on the stream right behind its final
@@ -50,6 +51,11 @@ namespace {
 
 constexpr int kInFlight = 4;
 constexpr size_t kAlign = 256;
+// Launches of two steps from this many cells in all active single-level runs
+// on.  Us per step, one and two at a time: FP32 2 x 64^3 17.0 and 18.9, 16 x
+// 32^3 19.4 and 19.0, 96^3 24.6 and 20.4, 30 runs of 32^3 to 128^3 414 and 335;
+// FP64 27.6 and 27.3, 29.9 and 27.3, 41.8 and 29.9, 823 and 563.
+constexpr long long kPairCells = 640 << 10;
 // device memory left free when a refined run is admitted
 constexpr size_t kRefinedReserve = (size_t)512 << 20;
 
@@ -119,7 +125,9 @@ struct Run {
   Request r;
   size_t off = 0, bytes = 0;
   lbx::Lattice lat{};    // the run's level-array geometry
-  long long start = 0;  // global step of pass 0
+  int passes = 0;        // passes launched, of steps + 1: collide, steps - 1 fused, stream
+  int cur = 0;           // buffer that holds the state after them
+  short bx = 0, by = 0;  // column of cells of a work item of two passes
   double t_admit = 0.0;
   bool launched_last = false;
   long long last_step = 0;
@@ -143,6 +151,7 @@ struct lbx_server {
   int policy = LBX_SERVE_FIFO;
   double max_wait_s = 0.0;  // shortest-first: runs queued longer go first (0 = no limit)
   int grid = 2048;
+  int cus = 256;
   Arena arena;
   void* arena_mem = nullptr;
   double* staging = nullptr;  // device: hydro and packed populations of a finishing run
@@ -282,6 +291,66 @@ void reject_refined(lbx_server* s, Run& r, int rc) {
   s->free_slots.push_back(r.slot);
 }
 
+// Two passes at once (k_serve_pair): the column of cells of a run's work
+// items, the one that covers its x-y plane in the fewest, rows whole or in
+// pieces of whole cache lines.
+void pair_column(Run& r) {
+  const int nx = r.r.req.dims[0], ny = r.r.req.dims[1];
+  long long best = -1;
+  for (int bx = std::min(nx, 208); bx >= 1; --bx) {
+    if (bx != nx && bx % 16) continue;
+    const int rows = lbx::kServePairCells / (bx + 2) - 2;
+    if (rows < 1) continue;
+    const long long tx = (nx + bx - 1) / bx, ty = (ny + rows - 1) / rows;
+    if (best < 0 || tx * ty < best) {
+      best = tx * ty;
+      r.bx = (short)bx;
+      r.by = (short)((ny + ty - 1) / ty);
+    }
+  }
+}
+
+long long columns(const Run& r) {
+  return (long long)((r.r.req.dims[0] + r.bx - 1) / r.bx) * ((r.r.req.dims[1] + r.by - 1) / r.by);
+}
+
+// Planes per work item, from the cost of a launch: rounds of items over the
+// CUs (a second one per CU in FP32 shares the vector units) x planes an item
+// walks.  200 steps of 8 runs of 64^3 in FP32 take 44, 38 and 63 us a step at
+// 8, 16 and 32 planes, 4 of 96^3 76, 74 and 72, 8 of 128^3 298, 284 and 278
+// (not less at 64 or 128); this takes the fastest of the three in 16 of 18
+// mixes tried, both precisions, and loses 5 % in the others (12 of 96^3).
+int pair_depth(const lbx_server* s) {
+  long long best = 0;
+  int best_depth = 8;
+  for (int depth = 8; depth <= 32; depth *= 2) {
+    long long items = 0;
+    for (const Run& r : s->active)
+      if (!r.sim && !r.launched_last) items += columns(r) * ((r.r.req.dims[2] + depth - 1) / depth);
+    const long long cost = (items + s->cus - 1) / s->cus * (depth + 3);
+    if (depth == 8 || cost < best) {
+      best = cost;
+      best_depth = depth;
+    }
+  }
+  return best_depth;
+}
+
+// Whether the next launch advances the active runs by two steps: enough cells
+// (kPairCells), in lattices whose columns keep most lanes busy (a cube's do to
+// 2/3 and more; a row of cells is better off as 256 cells per item).
+bool pairs_pay(const lbx_server* s) {
+  long long cells = 0, lanes = 0, left = 0;
+  for (const Run& r : s->active) {
+    if (r.launched_last) continue;
+    left = std::max(left, r.sim ? (long long)r.r.req.steps - r.steps_done : (long long)r.r.req.steps + 1 - r.passes);
+    if (r.sim) continue;
+    cells += cells_of(r.r.req);
+    lanes += columns(r) * lbx::kServePairCells * r.r.req.dims[2];
+  }
+  return left > 1 && cells >= kPairCells && lanes <= 2 * cells;
+}
+
 // Admission: move queued requests into the active set while they fit, in
 // arrival order (FIFO, stopping at the first that does not fit) or in order
 // of work (shortest first, skipping those that do not fit yet).
@@ -356,7 +425,7 @@ int admit(lbx_server* s) {
     r.off = off;
     r.bytes = bytes;
     r.lat = L;
-    r.start = s->step;
+    pair_column(r);
     r.t_admit = now_s();
     char* b0 = s->arena.base + off;
     const lbx_request& rq = r.r.req;
@@ -386,9 +455,8 @@ int admit(lbx_server* s) {
 // Enqueue a finished run's FP64 sums right behind its final pass: reduce
 // into the run's slot, copy to pinned host memory, record the slot event.
 int queue_finish(lbx_server* s, Run& r) {
-  const lbx_request& rq = r.r.req;
   const lbx::Lattice& L = r.lat;
-  char* fin = s->arena.base + r.off + (size_t)((rq.steps + 1) & 1) * L.elems() * esize(s->precision);
+  char* fin = s->arena.base + r.off + (size_t)r.cur * L.elems() * esize(s->precision);
   double* out = s->sums + 1024 + 4 * r.slot;
   SRV_HIP(s, lbx::launch_conservation(s->precision, false, fin, L, s->rho0, s->sums, 256, out, s->stream));
   SRV_HIP(s, hipMemcpyAsync(s->pinned + 4 * r.slot, out, 4 * sizeof(double), hipMemcpyDeviceToHost,
@@ -494,7 +562,7 @@ int collect(lbx_server* s, bool wait) {
     const long long n = cells_of(rq);
     const lbx::Lattice& L = r.lat;
     lbx::Region R{{0, 0, 0}, {rq.dims[0], rq.dims[1], rq.dims[2]}};
-    char* fin = s->arena.base + r.off + (size_t)((rq.steps + 1) & 1) * L.elems() * esize(s->precision);
+    char* fin = s->arena.base + r.off + (size_t)r.cur * L.elems() * esize(s->precision);
     lbx_result res{};
     res.id = r.r.id;
     res.status = LBX_OK;
@@ -530,8 +598,9 @@ int collect(lbx_server* s, bool wait) {
   return LBX_OK;
 }
 
-int launch_step(lbx_server* s) {
-  // refined runs: one level-0 step each on the context's stream, at most
+// Enqueues the next `width` (1 or 2) steps of every active run.
+int launch_steps(lbx_server* s, int width) {
+  // refined runs: their level-0 steps on the context's stream, at most
   // kInFlight steps ahead of the GPU
   bool stepped = false;
   for (Run& r : s->active) {
@@ -540,9 +609,11 @@ int launch_step(lbx_server* s) {
       const int k = int(s->step % kInFlight);
       if (s->rev_step[k] >= 0) SRV_HIP(s, hipEventSynchronize(s->rev[k]));
     }
-    if (int rc = lbx_iterate(r.sim, 1)) return sfail(s, rc, "refined run: %s", lbx_last_error(s->ctx));
+    const int n = std::min(width, r.r.req.steps - r.steps_done);
+    if (int rc = lbx_iterate(r.sim, n)) return sfail(s, rc, "refined run: %s", lbx_last_error(s->ctx));
     stepped = true;
-    if (++r.steps_done == r.r.req.steps) {
+    r.steps_done += n;
+    if (r.steps_done == r.r.req.steps) {
       r.launched_last = true;
       r.last_step = s->step;
       SRV_HIP(s, hipEventRecord(s->slot_ev[r.slot], lbx::ctx_stream(s->ctx)));
@@ -556,40 +627,61 @@ int launch_step(lbx_server* s) {
   }
   ServeBatch b{};
   int items = 0;
+  const int depth = width == 2 ? pair_depth(s) : 0;
   for (Run& r : s->active) {
     if (r.sim || r.launched_last) continue;
     ServeRun& d = b.run[b.nruns++];
-    d.buf[0] = s->arena.base + r.off;
-    d.buf[1] = s->arena.base + r.off + (size_t)r.lat.elems() * esize(s->precision);
+    char* base = s->arena.base + r.off;
+    const size_t one = (size_t)r.lat.elems() * esize(s->precision);
+    d.src = base + r.cur * one;
+    d.dst = base + (1 - r.cur) * one;
     for (int k = 0; k < 3; ++k) d.n[k] = r.r.req.dims[k];
     d.item_begin = items;
-    d.steps = r.r.req.steps;
-    d.start = r.start;
     d.ps = r.lat.ps;
     d.omega_s = 1.0 / (r.r.req.tau_s + 0.5);
     d.omega_b = 1.0 / (r.r.req.tau_b + 0.5);
     d.rho0 = s->rho0;
-    items += (int)((r.lat.nx * (long long)r.lat.ny * r.lat.nz + 255) / 256);
-    if (s->step - r.start == r.r.req.steps) {
+    const int last = r.r.req.steps;  // number of the stream-only pass
+    if (width == 2) {
+      const bool alone = r.passes == last;
+      d.kind = alone ? 0
+                     : (r.passes ? lbx::PAIR_PULL : 0) | lbx::PAIR_COLLIDE1 |
+                           (r.passes + 1 < last ? lbx::PAIR_COLLIDE2 : 0);
+      d.bx = r.bx;
+      d.by = r.by;
+      const int chunks = (d.n[2] + depth - 1) / depth;
+      d.depth = (d.n[2] + chunks - 1) / chunks;
+      items += (int)(columns(r) * ((d.n[2] + d.depth - 1) / d.depth));
+      r.passes += alone ? 1 : 2;
+    } else {
+      d.kind = r.passes == 0 ? lbx::STEP_COLLIDE : r.passes == last ? lbx::STEP_STREAM : lbx::STEP_FUSED;
+      items += (int)((r.lat.nx * (long long)r.lat.ny * r.lat.nz + 255) / 256);
+      ++r.passes;
+    }
+    r.cur ^= 1;
+    if (r.passes > last) {
       r.launched_last = true;
       r.last_step = s->step;
     }
   }
   b.total_items = items;
   if (b.nruns == 0) {
-    if (stepped) ++s->step;
+    if (stepped) s->step += width;
     return LBX_OK;
   }
   // reuse the event slot of step - kInFlight once the GPU has passed it
   const int k = int(s->step % kInFlight);
   if (s->ev_step[k] >= 0) SRV_HIP(s, hipEventSynchronize(s->ev[k]));
-  SRV_HIP(s, lbx::launch_serve_step(s->precision, b, s->step, s->grid, s->stream));
+  if (width == 2)
+    SRV_HIP(s, lbx::launch_serve_pair(s->precision, b, s->stream));
+  else
+    SRV_HIP(s, lbx::launch_serve_step(s->precision, b, s->grid, s->stream));
   SRV_HIP(s, hipEventRecord(s->ev[k], s->stream));
   s->ev_step[k] = s->step;
   for (Run& r : s->active)
     if (r.launched_last && !r.finish_queued && r.last_step == s->step)
       if (int rc = queue_finish(s, r)) return rc;
-  ++s->step;
+  s->step += width;
   return LBX_OK;
 }
 
@@ -616,7 +708,8 @@ int lbx_serve_create(lbx_ctx* ctx, int precision, double rho0, size_t arena_byte
   // One workgroup per work item (the hardware refills CUs as items finish;
   // a persistent grid of 4 per CU walking the list measured 16 % slower),
   // bounded for very long lists.
-  s->grid = std::max(1, cus) * 4096;
+  s->cus = std::max(1, cus);
+  s->grid = s->cus * 4096;
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->out, hipStreamNonBlocking);
   if (e == hipSuccess && arena_bytes == 0) {
@@ -734,13 +827,15 @@ int lbx_serve_submit(lbx_server* s, const lbx_request* req, uint64_t* id) {
 int lbx_serve_progress(lbx_server* s, int max_steps, int* active, int* queued) {
   if (!s) return LBX_E_ARG;
   SRV_HIP(s, hipSetDevice(s->device));
-  for (int it = 0; it < std::max(max_steps, 1); ++it) {
+  for (int it = 0; it < std::max(max_steps, 1);) {
     if (int rc = collect(s, false)) return rc;
     if (int rc = admit(s)) return rc;
     bool pending = false;
     for (const Run& r : s->active) pending |= !r.launched_last;
     if (!pending) break;
-    if (int rc = launch_step(s)) return rc;
+    const int width = max_steps - it > 1 && pairs_pay(s) ? 2 : 1;
+    if (int rc = launch_steps(s, width)) return rc;
+    it += width;
   }
   if (int rc = collect(s, false)) return rc;
   if (active) *active = (int)s->active.size();

@@ -7,13 +7,12 @@
 // The launch normally has one workgroup per item, with resident workgroups
 // per CU capped as for the stream-collide kernels; the loop below walks
 // further items with a static stride when the grid is smaller than the list,
-// so every workgroup ends after a bounded number of items.  Each run's pass kind
-// follows from the global step: pass p = step - start is collide-only for
-// p = 0, fused pull + collide for 0 < p < steps, stream-only for p = steps
-// (the same S (C S)^(n-1) C association as lbx_iterate), reading buffer
-// p & 1 and writing the other one.  The per-cell arithmetic does not depend
-// on which other runs share the launch, so a run's result is the same alone
-// and in any mix, bit for bit.
+// so every workgroup ends after a bounded number of items.  A run of n steps
+// takes n + 1 passes: collide-only, n - 1 fused pull + collide, stream-only
+// (the same S (C S)^(n-1) C association as lbx_iterate); a launch of two steps
+// (k_serve_pair) takes two of them at once.  The per-cell arithmetic does not
+// depend on which other runs share the launch nor on how passes are paired, so
+// a run's result is the same alone and in any mix, bit for bit.
 #include <hip/hip_runtime.h>
 
 #include "d3q15.h"
@@ -59,27 +58,123 @@ __device__ __forceinline__ void serve_cell(const ServeRun& R, int kind, const S*
   for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], dst + selfz + q * R.ps + selfp);
 }
 
+// The run holding a work item: the last r with item_begin <= item.
+__device__ __forceinline__ int run_of(const ServeBatch& B, int item) {
+  int lo = 0, hi = B.nruns - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (B.run[mid].item_begin <= item) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
 template <typename S>
-__global__ __launch_bounds__(256) void k_serve_step(ServeBatch B, long long step) {
+__global__ __launch_bounds__(256) void k_serve_step(ServeBatch B) {
   for (int item = blockIdx.x; item < B.total_items; item += gridDim.x) {
-    // run holding this item: last r with item_begin <= item
-    int lo = 0, hi = B.nruns - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (B.run[mid].item_begin <= item) lo = mid; else hi = mid - 1;
-    }
-    const ServeRun& R = B.run[lo];
-    const long long p = step - R.start;
-    if (p < 0 || p > R.steps) continue;  // not active at this step
-    const int kind = (p == 0) ? STEP_COLLIDE : (p == R.steps ? STEP_STREAM : STEP_FUSED);
-    const S* src = (const S*)R.buf[p & 1];
-    S* dst = (S*)R.buf[(p + 1) & 1];
+    const ServeRun& R = B.run[run_of(B, item)];
+    const S* src = (const S*)R.src;
+    S* dst = (S*)R.dst;
     const int plane = R.n[0] * R.n[1];
     const long long c = (long long)(item - R.item_begin) * 256 + threadIdx.x;
     if (c < (long long)plane * R.n[2]) {
       const int z = int(c / plane), r = int(c - (long long)z * plane);
       const int y = r / R.n[0], x = r - y * R.n[0];
-      serve_cell<S>(R, kind, src, dst, x, y, z);
+      serve_cell<S>(R, R.kind, src, dst, x, y, z);
+    }
+  }
+}
+
+// Two passes of every run in one pass over its state, as k_step_pair does for
+// one lattice: a work item is a column of cells and the ring around it, walked
+// through `depth` planes of z, the first pass of a plane handed over in LDS to
+// the second pass of the plane below.  The column is the run's own (rows of 32
+// cells and 16 of them on cubes of 32, 64, 96 and 128; 48 x 10 on 48^3), so a
+// small run wastes few lanes.  Bound like k_step_pair: by the collisions (the
+// ring repeats a fifth of the first ones) with one workgroup of 10 waves per CU
+// in FP64, by the reads and writes beside them in FP32 with two.  30 runs of
+// 32^3 to 128^3, us per step: FP32 414 -> 335, FP64 823 -> 563; 8 runs of 64^3
+// 48 -> 38 and 88 -> 63.
+template <typename S>
+__global__ __launch_bounds__(kServePairCells, sizeof(S) == 4 ? 5 : 3) void k_serve_pair(ServeBatch B) {
+  __shared__ S ring[2][NV][kServePairCells];
+  const int w = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);  // an XCD takes neighbouring columns
+  if (w >= B.total_items) return;
+  const ServeRun& R = B.run[run_of(B, w)];
+  const int nx = R.n[0], ny = R.n[1], nz = R.n[2], bx = R.bx, by = R.by, kind = R.kind;
+  const int item = w - R.item_begin, tx = (nx + bx - 1) / bx, ty = (ny + by - 1) / by;
+  const int x0 = item % tx * bx, y0 = item / tx % ty * by, z0 = item / (tx * ty) * R.depth;
+  const int z1 = min(z0 + R.depth, nz);
+  const int wx = bx + 2, t = threadIdx.x;
+  const S* __restrict__ src = (const S*)R.src;
+  S* __restrict__ dst = (S*)R.dst;
+  const long long ps = R.ps, zst = NV * ps;
+  const bool pull = kind & PAIR_PULL;
+
+  // first pass: cell t of the ring, its periodic image in the domain, and
+  // where its populations come from
+  const bool first = t < wx * (by + 2);
+  const int rx = (x0 - 1 + (first ? t % wx : 0) + nx) % nx, ry = (y0 - 1 + (first ? t / wx : 0) + ny) % ny;
+  unsigned xs[3], ys[3];
+  xs[1] = rx;
+  xs[0] = !pull ? rx : rx == nx - 1 ? 0 : rx + 1;
+  xs[2] = !pull ? rx : rx == 0 ? nx - 1 : rx - 1;
+  ys[1] = ry * nx;
+  ys[0] = (!pull ? ry : ry == ny - 1 ? 0 : ry + 1) * nx;
+  ys[2] = (!pull ? ry : ry == 0 ? ny - 1 : ry - 1) * nx;
+  // second pass: a cell of the column
+  const int cx = t % bx, cy = t / bx, ox = x0 + cx, oy = y0 + cy;
+  const bool second = cy < by && ox < nx && oy < ny;
+  const int self = oy * nx + ox, mid = second ? (cy + 1) * wx + cx + 1 : wx + 1;
+
+  auto load = [&](int z, S* f) {
+    z = z < 0 ? z + nz : z >= nz ? z - nz : z;
+    const S* zs[3] = {src + (!pull ? z : z == nz - 1 ? 0 : z + 1) * zst, src + z * zst,
+                      src + (!pull ? z : z == 0 ? nz - 1 : z - 1) * zst};
+#pragma unroll
+    for (int q = 0; q < NV; ++q) f[q] = (zs[1 + kC[q][2]] + q * ps)[ys[1 + kC[q][1]] + xs[1 + kC[q][0]]];
+  };
+  auto collide = [&](S* f) {
+    if constexpr (sizeof(S) == 8)
+      collide_f64(f, R.omega_s, R.omega_b);
+    else
+      collide_f32_shifted(f, float(R.rho0), float(R.omega_s), float(R.omega_b));
+  };
+
+  S next[NV], keep1[NV], keep2[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) next[q] = keep1[q] = keep2[q] = S(0);
+  if (first) load(z0 - 1, next);
+  for (int z = z0 - 1; z <= z1; ++z) {
+    S(*plane)[kServePairCells] = ring[z & 1];
+    if (first) {
+      S f[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) f[q] = next[q];
+      if (z < z1) load(z + 1, next);
+      if (kind & PAIR_COLLIDE1) collide(f);
+#pragma unroll
+      for (int q = 0; q < NV; ++q) plane[q][t] = f[q];
+    }
+    __syncthreads();
+    if (second) {
+      S f[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) {
+        const S v = plane[q][mid - kC[q][1] * wx - kC[q][0]];
+        if (kC[q][2] < 0) {
+          f[q] = v;
+        } else {
+          f[q] = keep1[q];
+          keep1[q] = kC[q][2] == 0 ? v : keep2[q];
+          if (kC[q][2] > 0) keep2[q] = v;
+        }
+      }
+      if (z > z0) {
+        if (kind & PAIR_COLLIDE2) collide(f);
+        S* out = dst + (z - 1) * zst + self;
+#pragma unroll
+        for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], out + q * ps);
+      }
     }
   }
 }
@@ -111,16 +206,25 @@ __global__ __launch_bounds__(256) void k_serve_init_pulse(S* __restrict__ f, Lat
 
 }  // namespace
 
-hipError_t launch_serve_step(int precision, const ServeBatch& b, long long step, int grid,
-                             hipStream_t st) {
+hipError_t launch_serve_step(int precision, const ServeBatch& b, int grid, hipStream_t st) {
   if (b.total_items <= 0) return hipSuccess;
   const int blocks = b.total_items < grid ? b.total_items : grid;
   // resident workgroups per CU capped like the stream-collide launches
   const int lds = lds_bytes_for_cap(precision == 0 ? 3 : 4);
   if (precision == 0)
-    k_serve_step<double><<<blocks, 256, lds > 0 ? lds : 0, st>>>(b, step);
+    k_serve_step<double><<<blocks, 256, lds > 0 ? lds : 0, st>>>(b);
   else
-    k_serve_step<float><<<blocks, 256, lds > 0 ? lds : 0, st>>>(b, step);
+    k_serve_step<float><<<blocks, 256, lds > 0 ? lds : 0, st>>>(b);
+  return hipGetLastError();
+}
+
+hipError_t launch_serve_pair(int precision, const ServeBatch& b, hipStream_t st) {
+  if (b.total_items <= 0) return hipSuccess;
+  const int blocks = (b.total_items + 7) / 8 * 8;
+  if (precision == 0)
+    k_serve_pair<double><<<blocks, kServePairCells, 0, st>>>(b);
+  else
+    k_serve_pair<float><<<blocks, kServePairCells, 0, st>>>(b);
   return hipGetLastError();
 }
 
