@@ -224,7 +224,8 @@ int lbx_conservation_noalloc(lbx_sim* sim, int level, double* d_out);
 /* Timing of the stream-collide kernel with HIP events recorded on the
  * context's stream around every launch while enabled.  *ms is the summed
  * kernel time, *launches the number of timed launches since the last
- * reset (on larger lattices one launch advances two steps). */
+ * reset (a launch advances two steps on larger lattices, up to three on
+ * small ones). */
 int lbx_profile_enable(lbx_ctx* ctx, int enable);
 int lbx_profile_read(lbx_ctx* ctx, double* ms, int64_t* launches);
 
@@ -234,7 +235,7 @@ int lbx_profile_read(lbx_ctx* ctx, double* ms, int64_t* launches);
  * While enabled, the first launch for a new (nx, ny, precision) times every
  * candidate on a small proxy lattice with the same rows and keeps the
  * fastest for the context's lifetime; shapes never change results.  Passes
- * that advance two steps in one launch have a shape of their own.  No
+ * that advance several steps in one launch have a shape of their own.  No
  * reference counterpart.  lbx_tuned_shape reports the shape launches of
  * that geometry use: the tuned choice and its time per proxy launch, or the
  * default shape (time 0) if the geometry was never tuned. */

@@ -53,7 +53,10 @@ struct Level {
   int ratio = 2;         // refinement ratio to the parent (patched levels)
   std::vector<Box> boxes;
   Lattice lat{};         // level-array geometry (level 0)
-  lbx::PairShape pair{};  // two-step passes of a single-level simulation (tx = 0: none)
+  // passes of several steps of a single-level simulation: of two (tx = 0:
+  // none), of a small lattice (steps = 0: none)
+  lbx::PairShape pair{};
+  lbx::BlockShape block{};
   void* buf[3] = {nullptr, nullptr, nullptr};  // state in buf[cur]; buf[2] scratch (patched, ratio above 2)
   int cur = 0;
   // Level 0 of a single-level simulation between Iterate calls: buf[cur]
@@ -471,6 +474,18 @@ int launch_pair(lbx_sim* sim, Level& L) {
   return ps.close();
 }
 
+int launch_block(lbx_sim* sim, Level& L, int steps) {
+  lbx_ctx* ctx = sim->ctx;
+  const Relax r{L.omega_s, L.omega_b, sim->rho0};
+  ProfileScope ps(ctx, true);
+  if (ps.rc) return ps.rc;
+  const hipError_t e = lbx::launch_step_block(sim->precision, L.buf[L.cur], L.buf[1 - L.cur], L.lat, r, L.block, steps,
+                                              ctx->stream);
+  if (e != hipSuccess) return hip_fail(ctx, e, "fused-steps launch");
+  L.cur = 1 - L.cur;
+  return ps.close();
+}
+
 // Bring level 0 back to the pre-collision populations f in place (the
 // stream-only pass) if it holds the post-collision state (Level::post).
 int materialise(lbx_sim* sim) {
@@ -754,7 +769,8 @@ int define_level0(lbx_sim* sim, const std::vector<Box>& boxes) {
   L.boxes = boxes;
   L.lat = lbx::make_lattice(sim->dims[0], sim->dims[1], sim->dims[2], (int)elem_size(sim->precision));
   L.lat.walls = sim->walls;
-  L.pair = lbx::pair_shape(L.lat, sim->precision);
+  L.block = lbx::block_shape(L.lat);
+  L.pair = L.block.steps ? lbx::PairShape{} : lbx::pair_shape(L.lat, sim->precision);
   const size_t bytes = (size_t)L.lat.elems() * elem_size(sim->precision);
   for (int i = 0; i < 2; ++i) {
     hipError_t e = hipMalloc(&L.buf[i], bytes);
@@ -1740,8 +1756,8 @@ int lbx_iterate(lbx_sim* sim, int nsteps) {
   // Reference order per step is f <- S(C(f)).  Over n steps:
   //   f_n = S (C S)^(n-1) C f_0 = S g_n,  g_n = (C S)^(n-1) C f_0
   // so from f in place: one collide-only pass and n-1 fused pull+collide
-  // steps leave g_n (Level::post); from g: n fused steps, two to a pass where
-  // the level has a pair shape.  The last S is
+  // steps leave g_n (Level::post); from g: n fused steps, several to a pass where
+  // the level has a block or pair shape.  The last S is
   // applied only when f is observed (a pull inside the readers, or the
   // stream-only pass of materialise()).  Per-cell arithmetic is unchanged,
   // so results are bit-identical to the reference order, and Iterate(a)
@@ -1751,6 +1767,11 @@ int lbx_iterate(lbx_sim* sim, int nsteps) {
     if (int rc = launch_step(sim, L, lbx::STEP_COLLIDE)) return rc;
     L.post = true;
     s = 1;
+  }
+  while (L.block.steps && s + 2 <= nsteps) {
+    const int left = nsteps - s, steps = left == 4 ? 2 : std::min(left, L.block.steps);
+    if (int rc = launch_block(sim, L, steps)) return rc;
+    s += steps;
   }
   for (; L.pair.tx && s + 2 <= nsteps; s += 2)
     if (int rc = launch_pair(sim, L)) return rc;

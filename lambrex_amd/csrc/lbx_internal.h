@@ -111,6 +111,18 @@ PairShape pair_shape(const Lattice& L, int precision);
 hipError_t launch_step_pair(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
                             const PairShape& p, hipStream_t st);
 
+// Several fused steps of a small lattice in one pass (k_step_block): n[d]
+// blocks of b[d] cells in each direction, up to `steps` steps a pass; steps =
+// 0: not used for this lattice.
+struct BlockShape {
+  int steps;
+  int b[3], n[3];
+};
+constexpr int kBlockCells = 768;  // of a block and its ring, at most
+BlockShape block_shape(const Lattice& L);
+hipError_t launch_step_block(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
+                             const BlockShape& b, int steps, hipStream_t st);
+
 // Equilibrium of a region from device rho[nz][ny][nx], u[3][nz][ny][nx].
 hipError_t launch_equilibrium(int precision, void* f, const Lattice& L, const Region& R,
                               const double* rho, const double* u, double rho0, hipStream_t st);

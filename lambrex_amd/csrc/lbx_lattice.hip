@@ -297,6 +297,73 @@ __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __r
   }
 }
 
+// T fused steps of a small lattice in one pass.  Such a lattice leaves a pass
+// nothing to do but wait: a launch, the loads' way to memory and back and one
+// collision take 4 us whether it has 500 cells or 10000.  A workgroup takes a
+// block of cells and a ring of T - 1 around it, a cell per lane: every lane
+// takes its cell's first step, the lanes one in from the edge the second, and
+// so on, the populations between them in LDS (one at rest stays in its lane).
+// The ring repeats work (4x4x4 cells of 3 steps: 8 x the first collision), on
+// CUs that have nothing else to do as long as the blocks fit them in one
+// round.  Us per step, one pass a step -> so: 10x10x50 FP64 4.1 -> 2.75, FP32
+// 4.0 -> 2.3; 32^3 5.2 -> 3.6 and 4.0 -> 2.9; 40^3 5.7 -> 5.0 and 5.0 -> 3.9.
+template <typename S, bool WALLS, int T>
+__global__ __launch_bounds__(kBlockCells) void k_step_block(const S* __restrict__ src, S* __restrict__ dst, Lattice L,
+                                                            Relax r, BlockShape b) {
+  __shared__ S moved[NV - 1][kBlockCells];
+  const int w = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);  // an XCD takes neighbouring blocks
+  if (w >= b.n[0] * b.n[1] * b.n[2]) return;
+  constexpr int R = T - 1;
+  const int ex = b.b[0] + 2 * R, ey = b.b[1] + 2 * R, ez = b.b[2] + 2 * R, t = threadIdx.x;
+  const int lx = t % ex, ly = t / ex % ey, lz = t / (ex * ey);
+  const bool on = lz < ez;
+  const int x = w % b.n[0] * b.b[0] + lx - R, y = w / b.n[0] % b.n[1] * b.b[1] + ly - R;
+  const int z = w / (b.n[0] * b.n[1]) * b.b[2] + lz - R;
+  auto wrapped = [](int v, int n) { return (v % n + n) % n; };
+  const int wx = wrapped(x, L.nx), wy = wrapped(y, L.ny), wz = on ? wrapped(z, L.nz) : 0;
+  unsigned faces = 0;
+  if (WALLS) {
+    faces = lateral_faces(wx, wy, L);
+    if (L.walls & 4u) faces |= (wz == 0 ? 16u : 0u) | (wz == L.nz - 1 ? 32u : 0u);
+  }
+  S f[NV];
+  if (on) {
+    const Upstream u = upstream(wx, wy, wz, L);
+    const long long own = L.at(0, wy * L.nx + wx, wz);
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      long long at = u.zo[1 + kC[q][2]] + u.ys[1 + kC[q][1]] + u.xs[1 + kC[q][0]] + q * L.ps;
+      if (WALLS && (faces & wall_faces(q))) at = own + opposite(q) * L.ps;
+      f[q] = src[at];
+    }
+    collide_any(f, r);
+  }
+#pragma unroll
+  for (int s = 1; s < T; ++s) {
+    if (s > 1) __syncthreads();
+    if (on) {
+#pragma unroll
+      for (int q = 1; q < NV; ++q) moved[q - 1][t] = f[q];
+    }
+    __syncthreads();
+    if (lx >= s && lx < ex - s && ly >= s && ly < ey - s && lz >= s && lz < ez - s) {
+#pragma unroll
+      for (int q = 1; q < NV; ++q) {
+        if (WALLS && (faces & wall_faces(q)))
+          f[q] = moved[opposite(q) - 1][t];
+        else
+          f[q] = moved[q - 1][t - (kC[q][2] * ey + kC[q][1]) * ex - kC[q][0]];
+      }
+      collide_any(f, r);
+    }
+  }
+  if (lx >= R && lx < ex - R && ly >= R && ly < ey - R && lz >= R && lz < ez - R && x < L.nx && y < L.ny && z < L.nz) {
+    const long long own = L.at(0, y * L.nx + x, z);
+#pragma unroll
+    for (int q = 0; q < NV; ++q) dst[own + q * L.ps] = f[q];
+  }
+}
+
 dim3 grid_of(const Lattice& L, LaunchShape s) {
   return dim3((L.nx + s.bx - 1) / s.bx, (L.ny + s.by - 1) / s.by, L.nz);
 }
@@ -664,6 +731,39 @@ hipError_t launch_step_f32s(StepKind kind, const float* src, float* dst, const L
   LBX_STEP_LAUNCH(k_step_f32s, src, dst);
 }
 
+static int compute_units() {
+  static const int cus = [] {
+    int dev = 0, n = 256;
+    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    return n < 1 ? 256 : n;
+  }();
+  return cus;
+}
+
+// Blocks of k_step_block for a lattice, or none (steps = 0): the first of
+// three shapes whose blocks fit the CUs in one round.  In one round a launch
+// takes 7 to 10 us (FP64) whatever the lattice; a second round loses what the
+// fused steps save (48^3 FP64 6.8 to 7.5 us a step in two rounds, 6.2 in
+// single passes).  Of 15 shapes swept at 16^3 to 40^3 and 10x10x50 these are
+// the fastest: 4x4x4 of 3 steps at 24^3 (3.15 us, the 2-step blocks 3.2 and
+// more), 8x4x4 of 2 at 32^3 (3.6; 4x4x8 of 3 steps 4.0), 8x8x4 at 40^3.
+BlockShape block_shape(const Lattice& L) {
+  static constexpr int kShapes[3][4] = {{3, 4, 4, 4}, {2, 8, 4, 4}, {2, 8, 8, 4}};
+  const long long n[3] = {L.nx, L.ny, L.nz};
+  for (const int(&c)[4] : kShapes) {
+    BlockShape b{};
+    b.steps = c[0];
+    long long blocks = 1;
+    for (int d = 0; d < 3; ++d) {
+      b.b[d] = c[1 + d];
+      b.n[d] = int((n[d] + c[1 + d] - 1) / c[1 + d]);
+      blocks = blocks > compute_units() ? blocks : blocks * b.n[d];
+    }
+    if (blocks <= compute_units()) return b;
+  }
+  return BlockShape{};
+}
+
 // Shape of the two-step pass for a lattice, or none (p.tx = 0) where two
 // single passes are the faster.  Every workgroup count that fills the device
 // for one or more rounds is a candidate: rounds x (planes of a workgroup + 2
@@ -674,11 +774,7 @@ hipError_t launch_step_f32s(StepKind kind, const float* src, float* dst, const L
 // against 5.9); at 48^3 in neither (7.1 against 6.4, 5.6 against 4.7); at
 // 96x80x72 in both (19.5 against 25.7, 12.6 against 12.9).
 PairShape pair_shape(const Lattice& L, int precision) {
-  static const int cus = [] {
-    int dev = 0, n = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    return n < 1 ? 256 : n;
-  }();
+  const int cus = compute_units();
   PairShape best{};
   const double bytes = double(L.elems()) * (precision == 0 ? 8 : 4);
   const bool mall = 2 * bytes <= 256e6;
@@ -718,6 +814,29 @@ static hipError_t step_pair(const S* src, S* dst, const Lattice& L, const Relax&
   else
     k_step_pair<S, qx, qy, false><<<grid, pair_threads(qx, qy), 0, st>>>(src, dst, L, r, p);
   return hipGetLastError();
+}
+
+template <typename S>
+static hipError_t step_block(const S* src, S* dst, const Lattice& L, const Relax& r, const BlockShape& b, int steps,
+                             hipStream_t st) {
+  const int grid = (b.n[0] * b.n[1] * b.n[2] + 7) / 8 * 8, ring = 2 * (steps - 1);
+  const int threads = ((b.b[0] + ring) * (b.b[1] + ring) * (b.b[2] + ring) + 63) / 64 * 64;
+  if (steps == 3 && L.walls)
+    k_step_block<S, true, 3><<<grid, threads, 0, st>>>(src, dst, L, r, b);
+  else if (steps == 3)
+    k_step_block<S, false, 3><<<grid, threads, 0, st>>>(src, dst, L, r, b);
+  else if (L.walls)
+    k_step_block<S, true, 2><<<grid, threads, 0, st>>>(src, dst, L, r, b);
+  else
+    k_step_block<S, false, 2><<<grid, threads, 0, st>>>(src, dst, L, r, b);
+  return hipGetLastError();
+}
+
+hipError_t launch_step_block(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
+                             const BlockShape& b, int steps, hipStream_t st) {
+  if (steps < 2 || steps > b.steps) return hipErrorInvalidValue;
+  if (precision == 0) return step_block((const double*)src, (double*)dst, L, r, b, steps, st);
+  return step_block((const float*)src, (float*)dst, L, r, b, steps, st);
 }
 
 hipError_t launch_step_pair(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,

@@ -1,0 +1,72 @@
+"""Passes of several steps of a small lattice (k_step_block) against single
+passes and the CPU oracle.
+
+Iterate(1) always runs single passes, Iterate(n) passes of two or three steps
+on lattices small enough; both form the same bits.  Sizes: below one block,
+whole blocks, remainders in every direction for each block shape, extents of 1
+to 3 cells (a ring that wraps more than once), walls on every axis, every
+remainder of the step count."""
+import numpy as np
+import pytest
+
+from lambrex_amd import lbx, workloads
+from oracle import oracle as orc
+from test_gpu_pair import start
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # dims, periodic
+    ((1, 1, 1), (1, 1, 1)),
+    ((2, 3, 1), (1, 1, 1)),
+    ((10, 10, 50), (1, 1, 1)),
+    ((5, 4, 9), (0, 0, 0)),
+    ((24, 24, 24), (1, 1, 0)),
+    ((32, 32, 32), (1, 1, 1)),
+    ((33, 29, 30), (0, 1, 1)),
+    ((40, 40, 40), (1, 1, 1)),
+    ((39, 33, 37), (0, 0, 1)),
+    ((250, 2, 3), (1, 0, 1)),
+    ((3, 2, 1000), (1, 1, 1)),
+]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with lbx.Context(0) as c:
+        yield c
+
+
+@pytest.mark.parametrize("precision", [lbx.LBX_FP64, lbx.LBX_FP32_SHIFTED])
+@pytest.mark.parametrize("dims,periodic", CASES)
+def test_blocks_equal_single_passes(ctx, dims, periodic, precision):
+    rho, u = workloads.random_state(dims, 5, 1e-2, 0.03)
+    a, b = (start(ctx, dims, periodic, precision, rho, u) for _ in range(2))
+    a.iterate(1)
+    ctx.profile_enable()
+    for n in (2, 3, 4, 5, 6, 7):
+        a.iterate(n)
+    launches = ctx.profile_read()[1]
+    ctx.profile_enable(False)
+    assert launches < 20  # of 27 steps: this size takes the path under test
+    for _ in range(28):
+        b.iterate(1)
+    fa, fb = a.get_f(), b.get_f()
+    a.close()
+    b.close()
+    assert np.array_equal(fa.view(np.uint64), fb.view(np.uint64))
+
+
+@pytest.mark.parametrize("dims", [(10, 10, 50), (34, 30, 31), (40, 37, 38)])
+def test_blocks_equal_oracle(ctx, dims):
+    rho, u = workloads.random_state(dims, 8, 1e-2, 0.03)
+    sim = start(ctx, dims, (1, 1, 1), lbx.LBX_FP64, rho, u)
+    sim.iterate(9)
+    f = sim.get_f()
+    sim.close()
+    o = orc.Sim(*dims, 0.7, 0.9, boxes=[(list(a), list(b)) for a, b in workloads.chop(dims, 64)])
+    o.init(np.ascontiguousarray(rho.transpose(2, 1, 0)).reshape(-1),
+           np.ascontiguousarray(u.transpose(3, 2, 1, 0)).reshape(-1))
+    o.iterate(9)
+    ref = o.get_f()
+    o.close()
+    assert np.array_equal(f.view(np.uint64), ref.view(np.uint64))
