@@ -296,8 +296,8 @@ def two_level_geometry():
 
 
 def two_level(ctx, steps, warmup, precision=lbx.LBX_FP64):
-    """The two-level configuration on the GPU (one coarse step = one replay
-    of the captured HIP graph).  Also returns the final density and velocity
+    """The two-level configuration on the GPU (one coarse step = three
+    launches).  Also returns the final density and velocity
     of both levels (for the FP32 vs FP64 comparison).  Its timed region
     (hundreds of coarse steps) is long enough that the GPU's clock ramp after
     idling does not matter, so there is no clock warm-up."""
@@ -327,7 +327,6 @@ def two_level(ctx, steps, warmup, precision=lbx.LBX_FP64):
                         f"ratio 2, 2 fine substeps per coarse step, {name}",
             "coarse_steps": steps, "warmup_steps": warmup, "mlups": lu / (t1 - t0) / 1e6,
             "ms_per_coarse_step": (t1 - t0) * 1e3 / steps,
-            "graph": "one coarse step captured as a HIP graph",
             "traffic_per_step": traffic,
             "roofline": hierarchy_roofline(lu / (t1 - t0) / 1e6, (t1 - t0) * 1e3 / steps, precision, traffic)}, fields
 
@@ -353,8 +352,7 @@ def three_level_geometry():
 
 
 def three_level(ctx, steps, warmup, precision=lbx.LBX_FP64):
-    """The three-level configuration on the GPU (one level-0 step = one
-    replay of the captured HIP graph)."""
+    """The three-level configuration on the GPU ."""
     dims, levels, masks, rho, u, lu_per_step = three_level_geometry()
     sim = lbx.Sim(ctx, dims, precision=precision, rho0=1.0)
     try:
@@ -385,7 +383,6 @@ def three_level(ctx, steps, warmup, precision=lbx.LBX_FP64):
                         f"32x512x512 (256 boxes of 32^3), ratio 2, {name}",
             "coarse_steps": steps, "warmup_steps": warmup, "mlups": lu / (t1 - t0) / 1e6,
             "ms_per_coarse_step": (t1 - t0) * 1e3 / steps,
-            "graph": "one level-0 step captured as a HIP graph",
             "traffic_per_step": traffic,
             "roofline": hierarchy_roofline(lu / (t1 - t0) / 1e6, (t1 - t0) * 1e3 / steps, precision, traffic),
             "final_rho_range_per_level": [[float(np.min(r)), float(np.max(r))] for r in rhos]}, rhos

@@ -8,7 +8,7 @@
 // grown by 2 ghost layers; the tables that drive its ghost fill (from its own
 // patches or its parent) and its average-down into the parent are built here
 // on the host once per level definition.  One level-0 step of a hierarchy is
-// the recursive Rohde cycle, captured as one HIP graph per buffer parity.
+// the recursive Rohde cycle, enqueued launch by launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -105,19 +105,6 @@ struct Level {
   int max_blocks = 0;            // largest (g/2)^3 of a patch
 };
 
-// Captured level-0 steps, one per combination of the levels' buffer
-// parities at the start of the step (bit l = level l's `cur`).
-struct StepGraphs {
-  hipGraphExec_t exec[1 << LBX_MAX_LEVELS] = {};
-  void clear() {
-    for (auto& e : exec)
-      if (e) {
-        (void)hipGraphExecDestroy(e);
-        e = nullptr;
-      }
-  }
-};
-
 // Conservation sums: a level array is reduced by kLatticePartials
 // workgroups; a patched level by patch_chunks(n) workgroups per patch.  The
 // context's scratch holds kPartials partials (4 doubles each) + 4 results.
@@ -167,8 +154,6 @@ struct lbx_sim {
   // every level)
   int ratio = 2;
   Level lev[LBX_MAX_LEVELS];
-  StepGraphs graphs;
-  bool use_graphs = true;
 };
 
 namespace {
@@ -559,7 +544,7 @@ hipError_t over_groups(lbx_ctx* ctx, const Level& L, hipStream_t st, Pass pass) 
   }
   for (size_t k = 0; k < L.groups.size() && e == hipSuccess; ++k)
     e = pass(L.groups[k].first, L.groups[k].second, (k & 1) ? ctx->side : st);
-  if (fork) {  // join even after a failed launch, so a capture can end
+  if (fork) {  // join even after a failed launch
     const hipError_t ej = hipEventRecord(ctx->join_ev, ctx->side);
     const hipError_t ew = ej == hipSuccess ? hipStreamWaitEvent(st, ctx->join_ev, 0) : ej;
     if (e == hipSuccess) e = ew;
@@ -674,63 +659,51 @@ hipError_t enqueue_hierarchy_step(lbx_sim* sim, hipStream_t st) {
   void* cnext = C.buf[1 - C.cur];
   int par[LBX_MAX_LEVELS];
   for (int l = 0; l < LBX_MAX_LEVELS; ++l) par[l] = sim->lev[l].cur;
-  // CoarseCollide + Stream(0) read level 0's `now` and write its `next`;
-  // the finer levels only read `now` (their parent fills), so the push runs
+  // CoarseCollide + Stream(0) read level 0's `now` and write its `next`, and
+  // the finer levels only read `now` (their parent fills), so the push can run
   // on its own stream beside them, and SumFromFine(0) into `next` waits for
-  // both.
+  // both.  It does where level 0 is worth the fork (8 us) and its two buffers
+  // stay in the 256 MB MALL; beyond it the push slows the finer levels for as
+  // long as it takes alone.  Us per step, in one stream and two: 64^3 FP32 74
+  // and 76, FP64 99 and 98; 96^3 FP32 210 and 202, FP64 294 and 277; 128^3 FP32
+  // 390 and 375, FP64 563 and 574.
   lbx_ctx* ctx = sim->ctx;
-  hipError_t e = hipEventRecord(ctx->push_fork_ev, st);
-  if (e == hipSuccess) e = hipStreamWaitEvent(ctx->push, ctx->push_fork_ev, 0);
-  if (e != hipSuccess) return e;
+  const double bytes = 2.0 * double(C.lat.elems()) * double(elem_size(sim->precision));
+  const bool fork = bytes > 64e6 && bytes <= 256e6;
+  hipError_t e = hipSuccess;
+  if (fork) {
+    e = hipEventRecord(ctx->push_fork_ev, st);
+    if (e == hipSuccess) e = hipStreamWaitEvent(ctx->push, ctx->push_fork_ev, 0);
+    if (e != hipSuccess) return e;
+  }
   const hipError_t ep = lbx::launch_coarse_push(sim->precision, cnow, cnext, C.lat, C.d_mask, rc, C.push_shape,
-                                                ctx->push);
+                                                fork ? ctx->push : st);
   e = enqueue_children(sim, 0, finest, par, st);
-  // join even after a failed launch, so a capture can end
-  const hipError_t ej = hipEventRecord(ctx->push_join_ev, ctx->push);
-  const hipError_t ew = ej == hipSuccess ? hipStreamWaitEvent(st, ctx->push_join_ev, 0) : ej;
+  if (fork) {  // join even after a failed launch
+    const hipError_t ej = hipEventRecord(ctx->push_join_ev, ctx->push);
+    const hipError_t ew = ej == hipSuccess ? hipStreamWaitEvent(st, ctx->push_join_ev, 0) : ej;
+    if (e == hipSuccess) e = ew;
+  }
   if (e == hipSuccess) e = ep;
-  if (e == hipSuccess) e = ew;
   if (e == hipSuccess)
     e = lbx::launch_sum_apply(sim->precision, F.d_avg, F.avg_stride, cnext, C.lat, F.d_sum_cell,
                               F.d_sum_start, F.d_sum_contrib, F.sum_ncell, sim->rho0, st);
   return e;
 }
 
-// One level-0 step: replayed from a captured graph, or launched eagerly
-// while profiling (event records cannot sit inside the capture).
+// One level-0 step.  Enqueued as it is: a HIP graph of it left the device idle
+// for 5 us between steps and 10 us at a join, and the host keeps ahead of the
+// launches (us per step, graph -> so: 24^3 with a 16^3-wide level FP64 57 -> 43,
+// 64^3 FP32 86 -> 74, 72x60x48 at ratio 3, 32 launches, 614 -> 564).
 int launch_hierarchy_step(lbx_sim* sim) {
   lbx_ctx* ctx = sim->ctx;
   Level& C = sim->lev[0];
   const int finest = finest_level(sim);
   Level& F = sim->lev[finest];
-  if (sim->use_graphs && !ctx->prof) {
-    unsigned key = 0;
-    for (int l = 0; l <= finest; ++l) key |= (unsigned)sim->lev[l].cur << l;
-    hipGraphExec_t& ex = sim->graphs.exec[key];
-    if (!ex) {
-      hipGraph_t g = nullptr;
-      LBX_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-      const hipError_t ek = enqueue_hierarchy_step(sim, ctx->stream);
-      const hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
-      if (ek != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return hip_fail(ctx, ek, "hierarchy step capture");
-      }
-      if (ec != hipSuccess) return hip_fail(ctx, ec, "hipStreamEndCapture");
-      const hipError_t ei = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (ei != hipSuccess) {
-        ex = nullptr;
-        return hip_fail(ctx, ei, "hipGraphInstantiate");
-      }
-    }
-    LBX_HIP(ctx, hipGraphLaunch(ex, ctx->stream));
-  } else {
-    ProfileScope ps(ctx, true);
-    if (ps.rc) return ps.rc;
-    LBX_HIP(ctx, enqueue_hierarchy_step(sim, ctx->stream));
-    if (int rc = ps.close()) return rc;
-  }
+  ProfileScope ps(ctx, true);
+  if (ps.rc) return ps.rc;
+  LBX_HIP(ctx, enqueue_hierarchy_step(sim, ctx->stream));
+  if (int rc = ps.close()) return rc;
   // every step of a middle level flips its buffer, and level l takes the
   // product of the ratios of levels 1..l steps per level-0 step; the finest
   // level's substeps run (and flip its buffer) once per step of its parent
@@ -1542,7 +1515,6 @@ int lbx_sim_destroy(lbx_sim* sim) {
   if (!sim) return LBX_OK;
   (void)hipSetDevice(sim->ctx->device);
   (void)hipStreamSynchronize(sim->ctx->stream);
-  sim->graphs.clear();
   for (Level& L : sim->lev) free_level(L);
   delete sim;
   return LBX_OK;
@@ -1557,7 +1529,6 @@ int lbx_level_define(lbx_sim* sim, int level, int n_boxes, const int32_t* lohi) 
   LBX_HIP(ctx, hipSetDevice(ctx->device));
   LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const std::vector<Box> boxes = read_boxes(n_boxes, lohi);
-  sim->graphs.clear();
   if (level == 0) return define_level0(sim, boxes);
   if (int rc = materialise(sim)) return rc;  // the Rohde cycle keeps level 0 pre-collision
   return define_level(sim, level, boxes);
@@ -1571,7 +1542,6 @@ int lbx_level_remake(lbx_sim* sim, int level, int n_boxes, const int32_t* lohi) 
   LBX_HIP(ctx, hipSetDevice(ctx->device));
   LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const std::vector<Box> boxes = read_boxes(n_boxes, lohi);
-  sim->graphs.clear();
   if (int rc = materialise(sim)) return rc;
   return remake_level(sim, level, boxes);
 }
@@ -1601,7 +1571,6 @@ int lbx_level_clear(lbx_sim* sim, int level) {
   if (level < 0 || level >= LBX_MAX_LEVELS) return fail(sim->ctx, LBX_E_ARG, "level %d out of range", level);
   LBX_HIP(sim->ctx, hipSetDevice(sim->ctx->device));
   (void)hipStreamSynchronize(sim->ctx->stream);
-  sim->graphs.clear();
   free_levels_from(sim, level);
   // the new finest level has no finer level to mask for
   return level > 0 ? unmask_level(sim, level - 1) : LBX_OK;
@@ -1624,7 +1593,6 @@ int lbx_set_relax(lbx_sim* sim, int level, double omega_s, double omega_b) {
   sim->lev[level].omega_s = omega_s;
   sim->lev[level].omega_b = omega_b;
   sim->lev[level].relax_set = true;
-  sim->graphs.clear();
   return LBX_OK;
 }
 
@@ -1640,7 +1608,6 @@ int lbx_set_level_mask(lbx_sim* sim, int level, int n_boxes, const int32_t* lohi
   LBX_HIP(ctx, hipSetDevice(ctx->device));
   LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   if (!C.d_mask) {
-    sim->graphs.clear();  // captured steps hold the mask's address
     LBX_HIP(ctx, hipMalloc(&C.d_mask, bytes.size()));
   }
   LBX_HIP(ctx, hipMemcpyAsync(C.d_mask, bytes.data(), bytes.size(), hipMemcpyHostToDevice, ctx->stream));
