@@ -165,10 +165,13 @@ __global__ __launch_bounds__(512) void k_step_f32s(const float* __restrict__ src
 // a contiguous range of columns) and, with one workgroup of 11 waves per CU
 // (LDS, and ~150 VGPRs in FP64), the part of the collisions that the loads
 // do not cover; in FP32 the vector units are busy 90 % of the time.
-// Measured (us per step, single pass -> pair): 256^3 FP64 652 -> 445, FP32
-// 328 -> 264; 128^3 FP64 88 -> 52, FP32 42.5 -> 28.4.  Slower: 32 x 8 and
-// 64 x 4 columns with two workgroups per CU (540), separate waves for the
-// two steps (470), non-temporal loads (564, the ring misses L2).
+// Measured (us per step, single pass -> pair): 256^3 FP64 652 -> 397, FP32
+// 328 -> 208 (5.2 and 5.0 TB/s, of a copy's 6.5); 128^3 FP64 88 -> 57, FP32
+// 42.5 -> 30.  FP64 409 and FP32 219 with the next plane's loads waited for
+// before the second step.  Slower: 32 x 8 and 64 x 4 columns with two
+// workgroups per CU, separate waves for the two steps, non-temporal loads (the
+// ring misses L2); in FP32 32 x 16 (221), 64 x 12 (229), 128 x 5 (226) and 64 x
+// 7 with two workgroups (238).
 constexpr int pair_threads(int bx, int by) { return ((bx + 2) * (by + 2) + 63) / 64 * 64; }
 
 template <typename S>
@@ -217,7 +220,7 @@ __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __r
   const int ox = x0 + t % BX, oy = y0 + t / BX;
   const bool second = t < BX * BY && ox < L.nx && oy < L.ny;
   const int self = oy * L.nx + ox;
-  const int mid = (t / BX + 1) * WX + t % BX + 1;
+  const int mid = WALLS || t < BX * BY ? (t / BX + 1) * WX + t % BX + 1 : WX + 1;
 
   // wall faces that a cell touches in x and y, and those that plane z lies on,
   // as a mask of wall_faces(); a population that comes from behind one of
@@ -248,33 +251,41 @@ __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __r
   S back[NV];   // walls: what the coming plane's c_z = -1 populations bounce to
 #pragma unroll
   for (int q = 0; q < NV; ++q) next[q] = keep1[q] = keep2[q] = back[q] = S(0);
-  if (first) load(z0 - 1, next);
-  for (int z = z0 - 1; z <= z1; ++z) {
-    S(*plane)[NC] = ring[z & 1];
-    if (first) {
-      S f[NV];
+  auto pull = [&](const S(*plane)[NC], S* f) {
 #pragma unroll
-      for (int q = 0; q < NV; ++q) f[q] = next[q];
-      if (z < z1) load(z + 1, next);
-      collide_any(f, r);
-#pragma unroll
-      for (int q = 0; q < NV; ++q) plane[q][t] = f[q];
-    }
-    __syncthreads();
-    if (second) {
-      S f[NV];
-#pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        const S v = plane[q][mid - kC[q][1] * WX - kC[q][0]];
-        if (kC[q][2] < 0) {
-          f[q] = v;
-        } else {
-          f[q] = keep1[q];
-          keep1[q] = kC[q][2] == 0 ? v : keep2[q];
-          if (kC[q][2] > 0) keep2[q] = v;
-        }
+    for (int q = 0; q < NV; ++q) {
+      const S v = plane[q][mid - kC[q][1] * WX - kC[q][0]];
+      if (kC[q][2] < 0) {
+        f[q] = v;
+      } else {
+        f[q] = keep1[q];
+        keep1[q] = kC[q][2] == 0 ? v : keep2[q];
+        if (kC[q][2] > 0) keep2[q] = v;
       }
-      if constexpr (WALLS) {
+    }
+  };
+  auto store = [&](int z, const S* f) {
+    S* out = dst + z * L.zs + self;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], out + q * L.ps);
+  };
+  if constexpr (WALLS) {
+    if (first) load(z0 - 1, next);
+    for (int z = z0 - 1; z <= z1; ++z) {
+      S(*plane)[NC] = ring[z & 1];
+      if (first) {
+        S f[NV];
+#pragma unroll
+        for (int q = 0; q < NV; ++q) f[q] = next[q];
+        if (z < z1) load(z + 1, next);
+        collide_any(f, r);
+#pragma unroll
+        for (int q = 0; q < NV; ++q) plane[q][t] = f[q];
+      }
+      __syncthreads();
+      if (second) {
+        S f[NV];
+        pull(plane, f);
         // the plane just formed is the own plane of the next second step:
         // its bounced populations return from this cell
 #pragma unroll
@@ -286,14 +297,45 @@ __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __r
             keep1[q] = plane[opposite(q)][mid];
           }
         }
-      }
-      if (z > z0) {
-        collide_any(f, r);
-        S* out = dst + (z - 1) * L.zs + self;
-#pragma unroll
-        for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], out + q * L.ps);
+        if (z > z0) {
+          collide_any(f, r);
+          store(z - 1, f);
+        }
       }
     }
+  } else {
+    // Every lane loads and pulls (one without a cell, another's): behind a
+    // branch, as with walls, the loaded values are copied where it joins and
+    // so waited for there, before the second step.  They are waited for after
+    // it, but before the stores are issued, or the wait would be for those as
+    // well.  (With walls the registers do not suffice for this in FP64, and it
+    // gained nothing in FP32.)
+    auto arrived = [&] {
+#pragma unroll
+      for (int q = 0; q < NV; ++q) asm volatile("" : "+v"(next[q]));
+    };
+    load(z0 - 1, next);
+    arrived();
+    auto walk = [&](int z, bool more) {
+      S(*plane)[NC] = ring[z & 1];
+      S f[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) f[q] = next[q];
+      if (more) load(z + 1, next);
+      collide_any(f, r);
+      if (first) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) plane[q][t] = f[q];
+      }
+      __syncthreads();
+      pull(plane, f);
+      const bool out = second && z > z0;
+      if (out) collide_any(f, r);
+      if (more) arrived();
+      if (out) store(z - 1, f);
+    };
+    for (int z = z0 - 1; z < z1; ++z) walk(z, true);
+    walk(z1, false);
   }
 }
 

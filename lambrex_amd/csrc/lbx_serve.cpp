@@ -53,8 +53,8 @@ constexpr int kInFlight = 4;
 constexpr size_t kAlign = 256;
 // Launches of two steps from this many cells in all active single-level runs
 // on.  Us per step, one and two at a time: FP32 2 x 64^3 17.0 and 18.9, 16 x
-// 32^3 19.4 and 19.0, 96^3 24.6 and 20.4, 30 runs of 32^3 to 128^3 414 and 335;
-// FP64 27.6 and 27.3, 29.9 and 27.3, 41.8 and 29.9, 823 and 563.
+// 32^3 19.4 and 19.0, 96^3 24.6 and 20.4, 30 runs of 32^3 to 128^3 414 and 305;
+// FP64 27.6 and 27.3, 29.9 and 27.3, 41.8 and 29.9, 823 and 543.
 constexpr long long kPairCells = 640 << 10;
 // device memory left free when a refined run is admitted
 constexpr size_t kRefinedReserve = (size_t)512 << 20;

@@ -92,8 +92,8 @@ __global__ __launch_bounds__(256) void k_serve_step(ServeBatch B) {
 // small run wastes few lanes.  Bound like k_step_pair: by the collisions (the
 // ring repeats a fifth of the first ones) with one workgroup of 10 waves per CU
 // in FP64, by the reads and writes beside them in FP32 with two.  30 runs of
-// 32^3 to 128^3, us per step: FP32 414 -> 335, FP64 823 -> 563; 8 runs of 64^3
-// 48 -> 38 and 88 -> 63.
+// 32^3 to 128^3, us per step: FP32 414 -> 305, FP64 823 -> 543; 8 runs of 64^3
+// 48 -> 36 and 88 -> 62.
 template <typename S>
 __global__ __launch_bounds__(kServePairCells, sizeof(S) == 4 ? 5 : 3) void k_serve_pair(ServeBatch B) {
   __shared__ S ring[2][NV][kServePairCells];
@@ -143,40 +143,47 @@ __global__ __launch_bounds__(kServePairCells, sizeof(S) == 4 ? 5 : 3) void k_ser
   S next[NV], keep1[NV], keep2[NV];
 #pragma unroll
   for (int q = 0; q < NV; ++q) next[q] = keep1[q] = keep2[q] = S(0);
-  if (first) load(z0 - 1, next);
-  for (int z = z0 - 1; z <= z1; ++z) {
-    S(*plane)[kServePairCells] = ring[z & 1];
-    if (first) {
-      S f[NV];
+  // as in k_step_pair, every lane loads and pulls
+  auto arrived = [&] {
 #pragma unroll
-      for (int q = 0; q < NV; ++q) f[q] = next[q];
-      if (z < z1) load(z + 1, next);
-      if (kind & PAIR_COLLIDE1) collide(f);
+    for (int q = 0; q < NV; ++q) asm volatile("" : "+v"(next[q]));
+  };
+  load(z0 - 1, next);
+  arrived();
+  auto walk = [&](int z, bool more) {
+    S(*plane)[kServePairCells] = ring[z & 1];
+    S f[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) f[q] = next[q];
+    if (more) load(z + 1, next);
+    if (kind & PAIR_COLLIDE1) collide(f);
+    if (first) {
 #pragma unroll
       for (int q = 0; q < NV; ++q) plane[q][t] = f[q];
     }
     __syncthreads();
-    if (second) {
-      S f[NV];
 #pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        const S v = plane[q][mid - kC[q][1] * wx - kC[q][0]];
-        if (kC[q][2] < 0) {
-          f[q] = v;
-        } else {
-          f[q] = keep1[q];
-          keep1[q] = kC[q][2] == 0 ? v : keep2[q];
-          if (kC[q][2] > 0) keep2[q] = v;
-        }
-      }
-      if (z > z0) {
-        if (kind & PAIR_COLLIDE2) collide(f);
-        S* out = dst + (z - 1) * zst + self;
-#pragma unroll
-        for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], out + q * ps);
+    for (int q = 0; q < NV; ++q) {
+      const S v = plane[q][mid - kC[q][1] * wx - kC[q][0]];
+      if (kC[q][2] < 0) {
+        f[q] = v;
+      } else {
+        f[q] = keep1[q];
+        keep1[q] = kC[q][2] == 0 ? v : keep2[q];
+        if (kC[q][2] > 0) keep2[q] = v;
       }
     }
-  }
+    const bool out = second && z > z0;
+    if (out && (kind & PAIR_COLLIDE2)) collide(f);
+    if (more) arrived();
+    if (out) {
+      S* to = dst + (z - 1) * zst + self;
+#pragma unroll
+      for (int q = 0; q < NV; ++q) __builtin_nontemporal_store(f[q], to + q * ps);
+    }
+  };
+  for (int z = z0 - 1; z < z1; ++z) walk(z, true);
+  walk(z1, false);
 }
 
 // Equilibrium of a plane pulse (rho = 1 + amplitude on one plane normal to
