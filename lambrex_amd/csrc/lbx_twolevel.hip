@@ -510,6 +510,16 @@ __global__ __launch_bounds__(kFineThreads) void k_fine_step(
 #pragma unroll
     for (int q = 1; q < NV; ++q) planes[q - 1][kB][t] = zero_pop<S>(q, r.rho0);
   }
+  // A plane's loads are waited for before its predecessor's stores are issued:
+  // a wait after them would be for the stores as well.
+  auto arrived = [&] {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) asm volatile("" : "+v"(next[q]));
+    asm volatile("" : "+v"(fill_next));
+    if constexpr (MASK) asm volatile("" : "+v"(mask_next));
+    if constexpr (SUM) asm volatile("" : "+v"(span_next));
+  };
+  arrived();
   const int steps_behind = FINEST ? 2 : 1;
   for (int k = a0; k < T.hi[2] + steps_behind; ++k) {
     const bool more = k + 1 < a1;
@@ -625,7 +635,6 @@ __global__ __launch_bounds__(kFineThreads) void k_fine_step(
         int lane = t;
         asm volatile("" : "+v"(lane));  // no address per round held in registers
         const int task_cell = (lane & ~63) + 2 * (lane & 15);
-        double* here = avg + P.avg_base + (long long)(zc >> 1) * ((gx >> 1) * (gy >> 1));
 #pragma unroll
         for (int q = 1; q < NV; ++q) meet(q, q - 1);
         wave_sync();
@@ -643,18 +652,21 @@ __global__ __launch_bounds__(kFineThreads) void k_fine_step(
             for (int c = 0; c < 4; ++c)
               s += to_f64_any(planes[q < NV ? q - 1 : 0][0][task_cell + (c & 1) + 32 * (c >> 1)], qq, r.rho0);
             sum[j] = s;
-            if (zc & 1) here[qq * avg_stride + task_block] = s * 0.125;
           }
         }
       }
     }
-    // The next plane's loads are waited for here, before the stores are
-    // issued: a wait after them would be for the stores as well.
+    arrived();
+    if constexpr (AVG) {
+      if (task & (zc >= T.lo[2]) & (zc & 1)) {
+        double* here = avg + P.avg_base + (long long)(zc >> 1) * ((gx >> 1) * (gy >> 1)) + task_block;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) asm volatile("" : "+v"(next[q]));
-    asm volatile("" : "+v"(fill_next));
-    if constexpr (MASK) asm volatile("" : "+v"(mask_next));
-    if constexpr (SUM) asm volatile("" : "+v"(span_next));
+        for (int j = 0; j < 4; ++j) {
+          const int q = 1 + 4 * j + (t >> 4 & 3);
+          if (q <= NV) here[(q < NV ? q : 0) * avg_stride] = sum[j] * 0.125;
+        }
+      }
+    }
     if (in_c & valid_c & (zc >= T.lo[2])) {
       S* out = fnext + (P.origin + (long long)zc * P.plane);
 #pragma unroll
