@@ -754,6 +754,7 @@ int define_level0(lbx_sim* sim, const std::vector<Box>& boxes) {
                   hipGetErrorString(e));
     }
   }
+  long long valid = 0;
   for (const Box& b : boxes) {
     PatchDesc d{};
     for (int k = 0; k < 3; ++k) {
@@ -762,6 +763,8 @@ int define_level0(lbx_sim* sim, const std::vector<Box>& boxes) {
       d.g[k] = b.n(k);
     }
     d.cells = (int)b.cells();
+    d.first = valid;
+    valid += d.cells;
     L.max_cells = std::max(L.max_cells, d.cells);
     L.desc.push_back(d);
   }
@@ -1006,7 +1009,7 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
   // ng = 2 / r coarse cells (AMReX's sum_fine_to_coarse: the fine ghosts
   // over the ratio), c[d] blocks per direction.
   const int ng = 2 / r;
-  long long base = 0, fill_base = 0, avg_base = 0;
+  long long base = 0, fill_base = 0, avg_base = 0, valid = 0;
   for (const Box& b : boxes) {
     PatchDesc d{};
     for (int k = 0; k < 3; ++k) {
@@ -1024,6 +1027,8 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
     d.row = packed ? b.n(0) : d.g[0];
     d.plane = packed ? b.n(0) * b.n(1) : d.g[0] * d.g[1];
     d.qs = ((packed ? b.cells() : cells) + 63) / 64 * 64;
+    d.first = valid;
+    valid += b.cells();
     d.fill_base = fill_base;
     d.avg_base = avg_base;
     const int blocks = (b.n(0) / r + 2 * ng) * (b.n(1) / r + 2 * ng) * (b.n(2) / r + 2 * ng);
@@ -1675,7 +1680,7 @@ int lbx_upload_f(lbx_sim* sim, int level, int box, const double* f) {
   LBX_HIP(ctx, hipMemcpyAsync(t, f, n * lbx::NV_TOTAL * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
   if (L.patched)
     LBX_HIP(ctx, lbx::launch_patch_io(sim->precision, 1, L.buf[L.cur], L.d_desc, box, (int)n, (double*)t,
-                                      nullptr, sim->rho0, ctx->stream));
+                                      sim->rho0, ctx->stream));
   else
     LBX_HIP(ctx, lbx::launch_unpack_f(sim->precision, L.buf[L.cur], L.lat, region_of(L.boxes[box]),
                                       (const double*)t, sim->rho0, ctx->stream));
@@ -1695,7 +1700,7 @@ int lbx_download_f(lbx_sim* sim, int level, int box, double* f) {
   LBX_HIP(ctx, stage_buffer(ctx, n * lbx::NV_TOTAL * sizeof(double), &t));
   if (L.patched)
     LBX_HIP(ctx, lbx::launch_patch_io(sim->precision, 0, L.buf[L.cur], L.d_desc, box, (int)n, (double*)t,
-                                      nullptr, sim->rho0, ctx->stream));
+                                      sim->rho0, ctx->stream));
   else
     LBX_HIP(ctx, lbx::launch_pack_f(sim->precision, L.post, L.buf[L.cur], L.lat, region_of(L.boxes[box]),
                                     (double*)t, sim->rho0, ctx->stream));
@@ -1760,8 +1765,8 @@ int lbx_hydro(lbx_sim* sim, int level, int box, double* rho, double* u) {
   double* drho = (double*)t;
   double* du = drho + n;
   if (L.patched)
-    LBX_HIP(ctx, lbx::launch_patch_io(sim->precision, 2, L.buf[L.cur], L.d_desc, box, (int)n, drho, du,
-                                      sim->rho0, ctx->stream));
+    LBX_HIP(ctx, lbx::launch_patch_hydro(sim->precision, L.buf[L.cur], L.d_desc, box, 1, (long long)n, drho, du,
+                                         sim->rho0, ctx->stream));
   else
     LBX_HIP(ctx, lbx::launch_hydro(sim->precision, L.post, L.buf[L.cur], L.lat, region_of(L.boxes[box]), drho,
                                    du, sim->rho0, ctx->stream));
@@ -1783,16 +1788,20 @@ int lbx_hydro_level(lbx_sim* sim, int level, double* rho, double* u) {
   LBX_HIP(ctx, stage_buffer(ctx, total * 4 * sizeof(double), &t));
   double* drho = (double*)t;
   double* du = drho + total;
-  size_t off = 0;
-  for (size_t b = 0; b < L.boxes.size(); ++b) {
-    const size_t n = (size_t)L.boxes[b].cells();
+  // One launch for all boxes if that is not mostly workgroups without cells
+  // (the grid is as wide as the largest box), else one per box.
+  size_t largest = 0;
+  for (const Box& b : L.boxes) largest = std::max(largest, (size_t)b.cells());
+  const int nbox = (int)L.boxes.size(), step = largest * nbox <= 2 * total + (1 << 20) ? nbox : 1;
+  for (int b = 0; b < nbox; b += step) {
+    const long long n = step == 1 ? L.boxes[b].cells() : (long long)largest;
+    const long long off = L.desc[b].first;
     if (L.patched)
-      LBX_HIP(ctx, lbx::launch_patch_io(sim->precision, 2, L.buf[L.cur], L.d_desc, (int)b, (int)n, drho + off,
-                                        du + 3 * off, sim->rho0, ctx->stream));
+      LBX_HIP(ctx, lbx::launch_patch_hydro(sim->precision, L.buf[L.cur], L.d_desc, b, step, n, drho + off,
+                                           du + 3 * off, sim->rho0, ctx->stream));
     else
-      LBX_HIP(ctx, lbx::launch_hydro(sim->precision, L.post, L.buf[L.cur], L.lat, region_of(L.boxes[b]),
-                                     drho + off, du + 3 * off, sim->rho0, ctx->stream));
-    off += n;
+      LBX_HIP(ctx, lbx::launch_hydro_boxes(sim->precision, L.post, L.buf[L.cur], L.lat, L.d_desc, b, step, n,
+                                           drho + off, du + 3 * off, sim->rho0, ctx->stream));
   }
   LBX_HIP(ctx, read_back(ctx, {{rho, drho, total * sizeof(double)}, {u, du, 3 * total * sizeof(double)}}));
   return LBX_OK;

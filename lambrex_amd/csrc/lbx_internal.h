@@ -123,6 +123,7 @@ BlockShape block_shape(const Lattice& L);
 hipError_t launch_step_block(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
                              const BlockShape& b, int steps, hipStream_t st);
 
+struct PatchDesc;
 // Equilibrium of a region from device rho[nz][ny][nx], u[3][nz][ny][nx].
 hipError_t launch_equilibrium(int precision, void* f, const Lattice& L, const Region& R,
                               const double* rho, const double* u, double rho0, hipStream_t st);
@@ -138,6 +139,12 @@ hipError_t launch_unpack_f(int precision, void* f, const Lattice& L, const Regio
 // Density and velocity of a region into packed FP64 buffers.
 hipError_t launch_hydro(int precision, bool pull, const void* f, const Lattice& L, const Region& R,
                         double* rho, double* u, double rho0, hipStream_t st);
+// ... of the boxes [first_box, first_box + nbox) of a level in one launch (at
+// most max_cells cells each), box after box as [n2][n1][n0] and
+// [3][n2][n1][n0].
+hipError_t launch_hydro_boxes(int precision, bool pull, const void* f, const Lattice& L, const PatchDesc* boxes,
+                              int first_box, int nbox, long long max_cells, double* rho, double* u, double rho0,
+                              hipStream_t st);
 // FP64 sums over the whole lattice: partials[nblocks*4] then out[4].
 // tag[(z*ny + y)*nx + x] = 1 where criterion 0 (|grad rho|^2) or 1 (|u|^2)
 // exceeds thr2.
@@ -160,6 +167,7 @@ struct PatchDesc {
   long long origin;  // ... of grown cell (0, 0, 0), stored or not
   long long qs;      // population stride
   LBX_IHD long long at(int x, int y, int z) const { return origin + (long long)z * plane + y * row + x; }
+  long long first;      // valid cells of the boxes before it (box order)
   long long fill_base;  // offset of this patch's rows in the fill table
   long long avg_base;   // offset of this patch's 2x2x2 block averages ((g/2)^3 per population)
 };
@@ -266,10 +274,12 @@ hipError_t launch_fine_from_coarse(int precision, void* fnow, const void* cnow, 
 hipError_t launch_fine_remake(int precision, void* fnew, const void* fold, const void* cnow, const Lattice& clat,
                               const PatchDesc* cpatches, const PatchDesc* patches, int npatch, int max_cells,
                               const PatchDesc* old_patches, const long long* src, hipStream_t st);
-// op 0: pack valid cells of patch b into FP64 f a[15][n]; 1: unpack; 2: hydro
-// into a (rho), u.
+// op 0: pack valid cells of patch b into FP64 f a[15][n]; 1: unpack.
 hipError_t launch_patch_io(int precision, int op, void* f, const PatchDesc* patches, int b, int valid_cells,
-                           double* a, double* u, double rho0, hipStream_t st);
+                           double* a, double rho0, hipStream_t st);
+// launch_hydro_boxes for a patched level.
+hipError_t launch_patch_hydro(int precision, const void* f, const PatchDesc* patches, int first_box, int nbox,
+                              long long max_cells, double* rho, double* u, double rho0, hipStream_t st);
 
 // Serving: one active run of the batch, passed by value in the kernel
 // arguments (kServeMaxRuns * sizeof(ServeRun) stays under 4 KB).

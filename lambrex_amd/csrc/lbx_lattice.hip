@@ -523,6 +523,29 @@ __global__ __launch_bounds__(256) void k_hydro(const S* __restrict__ f, Lattice 
   u[2 * n + i] = u2;
 }
 
+// k_hydro for every box of a level (blockIdx.y): a launch per box is 4 us, more
+// than most boxes take.
+template <typename S, bool PULL>
+__global__ __launch_bounds__(256) void k_hydro_boxes(const S* __restrict__ f, Lattice L,
+                                                     const PatchDesc* __restrict__ boxes, int first_box, int nbox,
+                                                     double* __restrict__ rho, double* __restrict__ u, double rho0) {
+  for (int b = blockIdx.y; b < nbox; b += gridDim.y) {
+    const PatchDesc& B = boxes[first_box + b];
+    const int n0 = B.hi[0] - B.lo[0] + 1, n1 = B.hi[1] - B.lo[1] + 1, n = n0 * n1 * (B.hi[2] - B.lo[2] + 1);
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) continue;
+    const int t = i / n0, x = i - t * n0, z = t / n1, y = t - z * n1;
+    double g[NV], r, u0, u1, u2;
+    cell_at<S, PULL>(f, L, B.lo[0] + x, B.lo[1] + y, B.lo[2] + z, rho0, g);
+    hydro_f64(g, r, u0, u1, u2);
+    const long long at = B.first - boxes[first_box].first;
+    rho[at + i] = r;
+    u[3 * at + i] = u0;
+    u[3 * at + n + i] = u1;
+    u[3 * at + 2ll * n + i] = u2;
+  }
+}
+
 constexpr int kTagX = 32, kTagY = 16;  // k_tag_gradient's tile
 constexpr int kTagGroups = 1024;       // and the workgroups it cuts z for
 // Cells from which a tile pays: k_tag against it, 32^3 6.4 and 8.8 us (FP32
@@ -932,6 +955,14 @@ hipError_t launch_hydro(int precision, bool pull, const void* f, const Lattice& 
                         double* rho, double* u, double rho0, hipStream_t st) {
   const long long n = (long long)R.n[0] * R.n[1] * R.n[2];
   LBX_PULL_LAUNCH(k_hydro, blocks_for(n), L, R, rho, u, rho0);
+  return hipGetLastError();
+}
+
+hipError_t launch_hydro_boxes(int precision, bool pull, const void* f, const Lattice& L, const PatchDesc* boxes,
+                              int first_box, int nbox, long long max_cells, double* rho, double* u, double rho0,
+                              hipStream_t st) {
+  const dim3 grid(blocks_for(max_cells), nbox < 65535 ? nbox : 65535);
+  LBX_PULL_LAUNCH(k_hydro_boxes, grid, L, boxes, first_box, nbox, rho, u, rho0);
   return hipGetLastError();
 }
 

@@ -855,7 +855,7 @@ __global__ __launch_bounds__(256) void k_fine_remake(S* __restrict__ fnew, const
 // patch.
 template <int OP, typename S>  // 0 pack, 1 unpack, 2 hydro
 __global__ __launch_bounds__(256) void k_patch_io(S* __restrict__ f, const PatchDesc* __restrict__ patches, int b,
-                                                  double* __restrict__ a, double* __restrict__ u, double rho0) {
+                                                  double* __restrict__ a, double rho0) {
   const PatchDesc P = patches[b];
   const int nx = P.hi[0] - P.lo[0] + 1, ny = P.hi[1] - P.lo[1] + 1, nz = P.hi[2] - P.lo[2] + 1;
   const int n = nx * ny * nz;
@@ -866,32 +866,45 @@ __global__ __launch_bounds__(256) void k_patch_io(S* __restrict__ f, const Patch
   if (OP == 0) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) a[(long long)q * n + i] = to_f64(f[li + q * P.qs], q, rho0);
-  } else if (OP == 1) {
+  } else {
 #pragma unroll
     for (int q = 0; q < NV; ++q) f[li + q * P.qs] = from_f64<S>(a[(long long)q * n + i], q, rho0);
-  } else {
-    double g[NV];
+  }
+}
+
+// Density and velocity of the valid cells of every patch (blockIdx.y) in one
+// launch.
+template <typename S>
+__global__ __launch_bounds__(256) void k_patch_hydro(const S* __restrict__ f, const PatchDesc* __restrict__ patches,
+                                                     int first_box, int nbox, double* __restrict__ rho,
+                                                     double* __restrict__ u, double rho0) {
+  for (int b = blockIdx.y; b < nbox; b += gridDim.y) {
+    const PatchDesc& P = patches[first_box + b];
+    const int n0 = P.hi[0] - P.lo[0] + 1, n1 = P.hi[1] - P.lo[1] + 1, n = n0 * n1 * (P.hi[2] - P.lo[2] + 1);
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) continue;
+    const int t = i / n0, x = i - t * n0, z = t / n1, y = t - z * n1;
+    const long long li = P.at(x + 2, y + 2, z + 2);
+    double g[NV], r, u0, u1, u2;
 #pragma unroll
     for (int q = 0; q < NV; ++q) g[q] = to_f64(f[li + q * P.qs], q, rho0);
-    double rr, u0, u1, u2;
-    hydro_f64(g, rr, u0, u1, u2);
-    a[i] = rr;
-    u[i] = u0;
-    u[n + i] = u1;
-    u[2 * n + i] = u2;
+    hydro_f64(g, r, u0, u1, u2);
+    const long long at = P.first - patches[first_box].first;
+    rho[at + i] = r;
+    u[3 * at + i] = u0;
+    u[3 * at + n + i] = u1;
+    u[3 * at + 2ll * n + i] = u2;
   }
 }
 
 template <typename S>
-hipError_t patch_io(int op, S* f, const PatchDesc* patches, int b, int valid_cells, double* a, double* u,
-                    double rho0, hipStream_t st) {
+hipError_t patch_io(int op, S* f, const PatchDesc* patches, int b, int valid_cells, double* a, double rho0,
+                    hipStream_t st) {
   const int blocks = (valid_cells + 255) / 256;
   if (op == 0)
-    k_patch_io<0, S><<<blocks, 256, 0, st>>>(f, patches, b, a, u, rho0);
-  else if (op == 1)
-    k_patch_io<1, S><<<blocks, 256, 0, st>>>(f, patches, b, a, u, rho0);
+    k_patch_io<0, S><<<blocks, 256, 0, st>>>(f, patches, b, a, rho0);
   else
-    k_patch_io<2, S><<<blocks, 256, 0, st>>>(f, patches, b, a, u, rho0);
+    k_patch_io<1, S><<<blocks, 256, 0, st>>>(f, patches, b, a, rho0);
   return hipGetLastError();
 }
 
@@ -1064,9 +1077,19 @@ hipError_t launch_fine_remake(int precision, void* fnew, const void* fold, const
 }
 
 hipError_t launch_patch_io(int precision, int op, void* f, const PatchDesc* patches, int b, int valid_cells,
-                           double* a, double* u, double rho0, hipStream_t st) {
-  if (precision == 0) return patch_io(op, (double*)f, patches, b, valid_cells, a, u, rho0, st);
-  return patch_io(op, (float*)f, patches, b, valid_cells, a, u, rho0, st);
+                           double* a, double rho0, hipStream_t st) {
+  if (precision == 0) return patch_io(op, (double*)f, patches, b, valid_cells, a, rho0, st);
+  return patch_io(op, (float*)f, patches, b, valid_cells, a, rho0, st);
+}
+
+hipError_t launch_patch_hydro(int precision, const void* f, const PatchDesc* patches, int first_box, int nbox,
+                              long long max_cells, double* rho, double* u, double rho0, hipStream_t st) {
+  const dim3 grid((unsigned)((max_cells + 255) / 256), nbox < 65535 ? nbox : 65535);
+  if (precision == 0)
+    k_patch_hydro<double><<<grid, 256, 0, st>>>((const double*)f, patches, first_box, nbox, rho, u, rho0);
+  else
+    k_patch_hydro<float><<<grid, 256, 0, st>>>((const float*)f, patches, first_box, nbox, rho, u, rho0);
+  return hipGetLastError();
 }
 
 }  // namespace lbx
