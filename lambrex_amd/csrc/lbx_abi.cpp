@@ -806,20 +806,6 @@ long long grown_index(const PatchDesc& P, int x, int y, int z) {
   return ((long long)(z - P.lo[2] + 2) * P.g[1] + (y - P.lo[1] + 2)) * P.g[0] + (x - P.lo[0] + 2);
 }
 
-// Element of population 0 of grown cell `index` of patch P, which is stored.
-long long stored_element(const PatchDesc& P, long long index) {
-  const long long plane = (long long)P.g[0] * P.g[1];
-  return P.at((int)(index % P.g[0]), (int)(index % plane / P.g[0]), (int)(index / plane));
-}
-
-// A reference to a stored cell of level C from cell_ref's, as the remake
-// kernel takes it: elements from the patch's base instead of a grown index.
-long long stored_ref(const Level& C, long long ref) {
-  if (!C.patched) return ref;
-  const PatchDesc& P = C.desc[ref >> 32];
-  return (ref >> 32 << 32) | (stored_element(P, ref & 0xffffffffll) - P.base);
-}
-
 // Where a level keeps the valid cell at (x, y, z) of its own index space
 // (already wrapped into the domain): the element of population 0 in a level
 // array, or (patch << 32) | grown index on a patched level.  False if no
@@ -1264,43 +1250,10 @@ int remake_level(lbx_sim* sim, int level, const std::vector<Box>& boxes) {
     return fail(ctx, LBX_E_STATE, "level %d has finer levels; clear them before remaking it", level);
   Level nf;
   if (int rc = build_level(sim, level, boxes, nf)) return rc;
-  // Source of every new valid cell: (old patch << 32) | old grown index, or
-  // -1 - parent reference.
-  std::vector<long long> src((size_t)nf.grown_cells, 0);
-  int chint = 0;
-  for (size_t b = 0; b < boxes.size(); ++b) {
-    const PatchDesc& P = nf.desc[b];
-    for (int z = P.lo[2]; z <= P.hi[2]; ++z)
-      for (int y = P.lo[1]; y <= P.hi[1]; ++y)
-        for (int x = P.lo[0]; x <= P.hi[0]; ++x) {
-          long long ref = 0;
-          (void)cell_ref(C, x / nf.ratio, y / nf.ratio, z / nf.ratio, &ref, chint);  // nesting checked by build_level
-          src[P.fill_base + grown_index(P, x, y, z)] = -1 - stored_ref(C, ref);
-        }
-    for (size_t o = 0; o < F.boxes.size(); ++o) {
-      const PatchDesc& O = F.desc[o];
-      int lo[3], hi[3];
-      bool empty = false;
-      for (int d = 0; d < 3; ++d) {
-        lo[d] = std::max(P.lo[d], O.lo[d]);
-        hi[d] = std::min(P.hi[d], O.hi[d]);
-        empty |= lo[d] > hi[d];
-      }
-      if (empty) continue;
-      for (int z = lo[2]; z <= hi[2]; ++z)
-        for (int y = lo[1]; y <= hi[1]; ++y)
-          for (int x = lo[0]; x <= hi[0]; ++x)
-            src[P.fill_base + grown_index(P, x, y, z)] = stored_ref(F, ((long long)o << 32) | grown_index(O, x, y, z));
-    }
-  }
-  DeviceTemp t;
-  hipError_t e = hipMalloc(&t.p, src.size() * sizeof(long long));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(t.p, src.data(), src.size() * sizeof(long long), hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess)
-    e = lbx::launch_fine_remake(sim->precision, nf.buf[0], F.buf[F.cur], C.buf[C.cur], C.lat,
-                                C.patched ? C.d_desc : nullptr, nf.d_desc, (int)nf.desc.size(), nf.max_cells,
-                                F.d_desc, (const long long*)t.p, ctx->stream);
+  hipError_t e = lbx::launch_fine_remake(sim->precision, nf.buf[0], F.buf[F.cur], C.buf[C.cur], C.lat,
+                                         C.patched ? C.d_desc : nullptr, (int)C.desc.size(), nf.d_desc,
+                                         (int)nf.desc.size(), nf.max_cells, F.d_desc, (int)F.desc.size(), nf.ratio,
+                                         ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) {
     free_level(nf);
@@ -1311,35 +1264,6 @@ int remake_level(lbx_sim* sim, int level, const std::vector<Box>& boxes) {
   nf.relax_set = F.relax_set;
   free_level(F);
   F = nf;
-  return LBX_OK;
-}
-
-// DistFnFillFromCoarse (src/AmrSim.cpp:393-411) for a level whose parent is
-// patched: every valid cell copies its parent through the remake kernel.
-int fill_from_patched(lbx_sim* sim, int level) {
-  lbx_ctx* ctx = sim->ctx;
-  const Level& C = sim->lev[level - 1];
-  Level& F = sim->lev[level];
-  std::vector<long long> src((size_t)F.grown_cells, 0);
-  int chint = 0;
-  for (size_t b = 0; b < F.boxes.size(); ++b) {
-    const PatchDesc& P = F.desc[b];
-    for (int z = P.lo[2]; z <= P.hi[2]; ++z)
-      for (int y = P.lo[1]; y <= P.hi[1]; ++y)
-        for (int x = P.lo[0]; x <= P.hi[0]; ++x) {
-          long long ref;
-          if (!cell_ref(C, x / F.ratio, y / F.ratio, z / F.ratio, &ref, chint))
-            return fail(ctx, LBX_E_STATE, "level %d is not nested in level %d", level, level - 1);
-          src[P.fill_base + grown_index(P, x, y, z)] = -1 - stored_ref(C, ref);
-        }
-  }
-  DeviceTemp t;
-  LBX_HIP(ctx, hipMalloc(&t.p, src.size() * sizeof(long long)));
-  LBX_HIP(ctx, hipMemcpyAsync(t.p, src.data(), src.size() * sizeof(long long), hipMemcpyHostToDevice, ctx->stream));
-  LBX_HIP(ctx, lbx::launch_fine_remake(sim->precision, F.buf[F.cur], nullptr, C.buf[C.cur], C.lat, C.d_desc,
-                                       F.d_desc, (int)F.boxes.size(), F.max_cells, F.d_desc, (const long long*)t.p,
-                                       ctx->stream));
-  LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return LBX_OK;
 }
 
@@ -1634,9 +1558,13 @@ int lbx_fill_from_coarse(lbx_sim* sim, int level) {
   if (!C.defined || !F.defined) return fail(ctx, LBX_E_STATE, "levels %d and %d must be defined", level - 1, level);
   LBX_HIP(ctx, hipSetDevice(ctx->device));
   if (int rc = materialise(sim)) return rc;
-  if (C.patched) return fill_from_patched(sim, level);
-  LBX_HIP(ctx, lbx::launch_fine_from_coarse(sim->precision, F.buf[F.cur], C.buf[C.cur], C.lat, F.d_desc,
-                                            (int)F.boxes.size(), F.max_cells, F.ratio, ctx->stream));
+  if (C.patched)
+    LBX_HIP(ctx, lbx::launch_fine_remake(sim->precision, F.buf[F.cur], nullptr, C.buf[C.cur], C.lat, C.d_desc,
+                                         (int)C.desc.size(), F.d_desc, (int)F.desc.size(), F.max_cells, nullptr, 0,
+                                         F.ratio, ctx->stream));
+  else
+    LBX_HIP(ctx, lbx::launch_fine_from_coarse(sim->precision, F.buf[F.cur], C.buf[C.cur], C.lat, F.d_desc,
+                                              (int)F.boxes.size(), F.max_cells, F.ratio, ctx->stream));
   LBX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return LBX_OK;
 }

@@ -268,12 +268,11 @@ hipError_t launch_sum_apply(int precision, const double* avg, long long avg_stri
 hipError_t launch_fine_from_coarse(int precision, void* fnow, const void* cnow, const Lattice& clat,
                                    const PatchDesc* patches, int npatch, int max_cells, int ratio,
                                    hipStream_t st);
-// Valid cells of new patches from old patches or the coarse parent
-// (src per new grown cell: (old patch << 32) | element from its base, or a
-// coarse reference likewise).
+// Valid cells of new patches from the nold old patches, and from the parent
+// (ncoarse patches, or with cpatches null a level array) where none holds them.
 hipError_t launch_fine_remake(int precision, void* fnew, const void* fold, const void* cnow, const Lattice& clat,
-                              const PatchDesc* cpatches, const PatchDesc* patches, int npatch, int max_cells,
-                              const PatchDesc* old_patches, const long long* src, hipStream_t st);
+                              const PatchDesc* cpatches, int ncoarse, const PatchDesc* patches, int npatch,
+                              int max_cells, const PatchDesc* old_patches, int nold, int ratio, hipStream_t st);
 // op 0: pack valid cells of patch b into FP64 f a[15][n]; 1: unpack.
 hipError_t launch_patch_io(int precision, int op, void* f, const PatchDesc* patches, int b, int valid_cells,
                            double* a, double rho0, hipStream_t st);

@@ -811,41 +811,74 @@ __global__ __launch_bounds__(256) void k_fine_from_coarse(S* __restrict__ fnow, 
   }
 }
 
-// RemakeLevel's fill (src/AmrSim.cpp:715-744 via DistFnFillPatch): each
-// valid cell of the new patches copies its populations from an old fine
-// patch (src >= 0: (old patch << 32) | element from its base) or from its
-// coarse parent (src < 0: -1 - coarse element of population 0, or with PC
-// -1 - ((coarse patch << 32) | element from its base)).  With every source a parent it
-// is DistFnFillFromCoarse on a level whose parent is patched.
+// The patches of boxes [0, n) that meet the box [lo, hi], listed by the
+// workgroup in `list`, which has room for kNear; their number, or -1 if it has
+// not.  A barrier at either end.
+constexpr int kNear = 512;
+__device__ __forceinline__ int near_boxes(const PatchDesc* __restrict__ boxes, int n, const int* lo, const int* hi,
+                                          int* list, int* count) {
+  __syncthreads();
+  if (threadIdx.x == 0) *count = 0;
+  __syncthreads();
+  for (int b = threadIdx.x; b < n; b += 256) {
+    const PatchDesc& B = boxes[b];
+    bool meets = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) meets &= B.lo[d] <= hi[d] && B.hi[d] >= lo[d];
+    if (meets) {
+      const int k = atomicAdd(count, 1);
+      if (k < kNear) list[k] = b;
+    }
+  }
+  __syncthreads();
+  return *count <= kNear ? *count : -1;
+}
+
+// RemakeLevel's fill (src/AmrSim.cpp:715-744 via DistFnFillPatch) and, with no
+// old patches, DistFnFillFromCoarse (src/AmrSim.cpp:393-411) from a patched
+// parent: each valid cell of the new patches takes the value of the old patch
+// that holds it, else of its parent.  A workgroup first lists the old and the
+// parent's patches that meet its own, of which every lane then looks for the
+// one that holds its cell (boxes of a level are disjoint).  A table of the
+// sources, made cell by cell on the host, took 14 ms for the 2 M cells of
+// 32x256x256; this takes 0.1.
 template <typename S, bool PC>
 __global__ __launch_bounds__(256) void k_fine_remake(S* __restrict__ fnew, const S* __restrict__ fold,
                                                      const S* __restrict__ cnow, Lattice clat,
-                                                     const PatchDesc* __restrict__ cpatches,
+                                                     const PatchDesc* __restrict__ cpatches, int ncoarse,
                                                      const PatchDesc* __restrict__ patches,
-                                                     const PatchDesc* __restrict__ old_patches,
-                                                     const long long* __restrict__ src) {
-  const PatchDesc P = patches[blockIdx.y];
+                                                     const PatchDesc* __restrict__ old_patches, int nold, int ratio) {
+  __shared__ int list[kNear], count;
+  const PatchDesc& P = patches[blockIdx.y];
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= P.cells) return;
+  if ((int)blockIdx.x * 256 >= P.cells) return;
   int gx, gy, gz;
   patch_coords(P, i, gx, gy, gz);
-  if (!patch_valid(P, gx, gy, gz)) return;
-  const long long d = src[P.fill_base + i];
-  const S* from;
-  long long stride;
-  if (d >= 0) {
-    const PatchDesc& O = old_patches[d >> 32];
-    from = fold + O.base + (d & 0xffffffffll);
-    stride = O.qs;
-  } else if constexpr (PC) {
-    const long long e = -1 - d;
-    const PatchDesc& CP = cpatches[e >> 32];
-    from = cnow + CP.base + (e & 0xffffffffll);
-    stride = CP.qs;
-  } else {
-    from = cnow + (-1 - d);
+  const bool valid = i < P.cells && patch_valid(P, gx, gy, gz);
+  const S* from = nullptr;
+  long long stride = 0;
+  auto look = [&](const PatchDesc* boxes, int n, const S* state, int r) {
+    const int lo[3] = {P.lo[0] / r, P.lo[1] / r, P.lo[2] / r}, hi[3] = {P.hi[0] / r, P.hi[1] / r, P.hi[2] / r};
+    const int x = (P.lo[0] - 2 + gx) / r, y = (P.lo[1] - 2 + gy) / r, z = (P.lo[2] - 2 + gz) / r;
+    const int near = near_boxes(boxes, n, lo, hi, list, &count);
+    for (int k = 0; k < (near < 0 ? n : near); ++k) {
+      const PatchDesc& B = boxes[near < 0 ? k : __builtin_amdgcn_readfirstlane(list[k])];
+      if (valid && from == nullptr && x >= B.lo[0] && x <= B.hi[0] && y >= B.lo[1] && y <= B.hi[1] && z >= B.lo[2] &&
+          z <= B.hi[2]) {
+        from = state + B.at(x - B.lo[0] + 2, y - B.lo[1] + 2, z - B.lo[2] + 2);
+        stride = B.qs;
+      }
+    }
+  };
+  look(old_patches, nold, fold, 1);
+  if constexpr (PC) {
+    look(cpatches, ncoarse, cnow, ratio);
+  } else if (valid && from == nullptr) {
+    const int x = (P.lo[0] - 2 + gx) / ratio, y = (P.lo[1] - 2 + gy) / ratio, z = (P.lo[2] - 2 + gz) / ratio;
+    from = cnow + clat.at(0, y * clat.nx + x, z);
     stride = clat.ps;
   }
+  if (from == nullptr) return;
   const long long to = P.at(gx, gy, gz);
 #pragma unroll
   for (int q = 0; q < NV; ++q) fnew[to + q * P.qs] = from[q * stride];
@@ -1058,21 +1091,21 @@ hipError_t launch_fine_avg_valid(int precision, const void* f, double* avg, long
 }
 
 hipError_t launch_fine_remake(int precision, void* fnew, const void* fold, const void* cnow, const Lattice& clat,
-                              const PatchDesc* cpatches, const PatchDesc* patches, int npatch, int max_cells,
-                              const PatchDesc* old_patches, const long long* src, hipStream_t st) {
+                              const PatchDesc* cpatches, int ncoarse, const PatchDesc* patches, int npatch,
+                              int max_cells, const PatchDesc* old_patches, int nold, int ratio, hipStream_t st) {
   const dim3 grid((max_cells + 255) / 256, npatch);
   if (precision == 0 && cpatches)
     k_fine_remake<double, true><<<grid, 256, 0, st>>>((double*)fnew, (const double*)fold, (const double*)cnow, clat,
-                                                      cpatches, patches, old_patches, src);
+                                                      cpatches, ncoarse, patches, old_patches, nold, ratio);
   else if (precision == 0)
     k_fine_remake<double, false><<<grid, 256, 0, st>>>((double*)fnew, (const double*)fold, (const double*)cnow, clat,
-                                                       cpatches, patches, old_patches, src);
+                                                       cpatches, ncoarse, patches, old_patches, nold, ratio);
   else if (cpatches)
     k_fine_remake<float, true><<<grid, 256, 0, st>>>((float*)fnew, (const float*)fold, (const float*)cnow, clat,
-                                                     cpatches, patches, old_patches, src);
+                                                     cpatches, ncoarse, patches, old_patches, nold, ratio);
   else
     k_fine_remake<float, false><<<grid, 256, 0, st>>>((float*)fnew, (const float*)fold, (const float*)cnow, clat,
-                                                      cpatches, patches, old_patches, src);
+                                                      cpatches, ncoarse, patches, old_patches, nold, ratio);
   return hipGetLastError();
 }
 
