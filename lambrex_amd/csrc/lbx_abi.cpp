@@ -98,8 +98,8 @@ struct Level {
   std::vector<PatchDesc> gdesc;
   PatchDesc* d_gdesc = nullptr;
   std::vector<std::pair<int, int>> groups;  // (first position in gdesc, count)
-  lbx::FineTile* d_tiles = nullptr;
-  int ntiles = 0;
+  lbx::FineTile* d_tiles = nullptr;  // the finest level's, then a middle level's
+  int ntiles[2] = {0, 0};
   double* d_avg = nullptr;       // 15 planes of avg_stride 2x2x2 block averages
   long long avg_stride = 0;
   int max_blocks = 0;            // largest (g/2)^3 of a patch
@@ -509,8 +509,8 @@ lbx::FineStep fine_step_args(const lbx_sim* sim, int l, bool finest, bool averag
   a.next = L.buf[1 - par[l]];
   a.parent = P.buf[par[l - 1]];
   a.own = L.d_gdesc;
-  a.tiles = L.d_tiles;
-  a.ntiles = L.ntiles;
+  a.tiles = L.d_tiles + (finest ? 0 : L.ntiles[0]);
+  a.ntiles = L.ntiles[finest ? 0 : 1];
   a.fill = (const unsigned long long*)L.d_fill;
   a.strides = L.d_strides;
   a.parent_stride = P.patched ? P.gdesc[0].qs : P.lat.ps;
@@ -862,11 +862,13 @@ int part_begin(int g, int n, int k) { return 2 * (int)((long long)(g / 2) * k / 
 // of at most `want` cells per direction; the target that costs least is taken:
 // rounds of workgroups over the CUs x planes a workgroup walks (its own and
 // up to 4 around them, and 2 of the pipeline) x time of a plane (2.5 us + 0.4
-// us per wave of its A plane, fitted to FP64 steps of 36^3 patches).  The
-// model only ranks the targets: of a sweep that forced each of them on 36^3
-// and 28^3 patches, none was faster than the one it takes by more than the
-// runs differed.
-std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches) {
+// us, in FP32 0.2, per wave of its A plane).  The model only ranks the targets:
+// of a sweep that forced each of them on 36^3 and 28^3 patches in FP64, none was
+// faster than the one it takes by more than the runs differed; in FP32 0.4 a
+// wave takes smaller tiles and is slower (64^3 with a 32x128x128 level 72 us a
+// step, 68 so; three levels over 32^3 152 and 138).
+std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int elem_bytes, bool finest) {
+  const int room = lbx::fine_tile_cells(elem_bytes, finest);
   std::map<std::tuple<int, int, int>, int> shapes;  // grown extents -> patches
   int gmax[3] = {2, 2, 2};
   for (const PatchDesc& p : patches) {
@@ -907,8 +909,8 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches) {
         cells = std::max(cells, widest(gx, nx) * widest(gy, ny));
         columns += (long long)nx * ny * s.second;
       }
-      if (cells > lbx::kFineTileCells || columns > (1 << 24)) continue;
-      const double plane_us = 2.5 + 0.4 * ((cells + 63) / 64);
+      if (cells > room || columns > (1 << 24)) continue;
+      const double plane_us = 2.5 + (elem_bytes == 8 ? 0.4 : 0.2) * ((cells + 63) / 64);
       for (int wz : tz) {
         long long n = 0;
         int planes = 0;
@@ -1060,8 +1062,12 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
     }
   }
   std::vector<lbx::FineTile> tiles;
-  if (r == 2) tiles = plan_tiles(F.gdesc);
-  F.ntiles = (int)tiles.size();
+  for (int middle = 0; r == 2 && middle < 2; ++middle) {
+    const std::vector<lbx::FineTile> t =
+        plan_tiles(F.gdesc, (int)elem_size(sim->precision), !middle);
+    F.ntiles[middle] = (int)t.size();
+    tiles.insert(tiles.end(), t.begin(), t.end());
+  }
   // Ghost fill sources (FillPatchTwoLevels with piecewise-constant
   // interpolation, src/AmrSim.cpp:373-388): the valid cell of this level
   // holding the periodic image if a box has it, else the coarse parent.

@@ -216,12 +216,15 @@ hipError_t launch_fine_stream_zero(int precision, const void* in, void* out, con
                                    const double* avg, long long avg_stride, const int* contrib, hipStream_t st);
 // A tile of a patch in k_fine_step: grown cells [lo, hi), even on both ends,
 // of patch `patch` (launch order).  With the 2 cells around it in x and y
-// (inside the patch) it holds at most kFineTileCells cells per plane.
+// (inside the patch) it holds at most fine_tile_cells cells per plane.
 struct FineTile {
   int patch;
   int lo[3], hi[3];
 };
-constexpr int kFineTileCells = 512;
+// 8 waves, whose 256 registers a lane FP64 and the middle levels' sums need; the
+// finest level in FP32 does with 168 and so takes 12 (128^3 with a 64x256x256
+// level 360 -> 306 us a step; a middle level spills).
+constexpr int fine_tile_cells(int elem_bytes, bool finest) { return elem_bytes == 4 && finest ? 768 : 512; }
 
 constexpr unsigned long long kFillParent = 1ull << 63, kFillElement = (1ull << 40) - 1;
 constexpr int kFillStrideShift = 40;

@@ -344,8 +344,6 @@ __global__ __launch_bounds__(256) void k_fine_stream_zero(const S* __restrict__ 
 // workgroup a CU (114 KB of LDS, 2 waves a SIMD at 256 registers).  Slower: 12
 // waves on tiles of 36 x 20 cells at 168 registers (484 us), the loads of a
 // plane in one piece or after the first barrier (503 to 627 us).
-constexpr int kFineThreads = 512;  // 8 waves
-constexpr int kFineCells = kFineTileCells;
 
 // Orders a wave's LDS accesses among its own lanes.
 __device__ __forceinline__ void wave_sync() {
@@ -369,7 +367,7 @@ __device__ constexpr int lateral(int q) { return (kC[q][1] + 1) * 3 + kC[q][0] +
 __device__ constexpr int pull_first(int c) { return c < 4 ? c + 1 : 2 * c - 3; }
 
 template <typename S, bool FINEST, bool MASK, bool SUM, bool AVG>
-__global__ __launch_bounds__(kFineThreads) void k_fine_step(
+__global__ __launch_bounds__(fine_tile_cells(sizeof(S), FINEST)) void k_fine_step(
     const S* __restrict__ fnow, S* __restrict__ fnext, const S* __restrict__ cnow,
     const PatchDesc* __restrict__ own, const FineTile* __restrict__ tiles, int ntiles,
     const unsigned long long* __restrict__ fill, const unsigned* __restrict__ strides, long long parent_stride,
@@ -378,6 +376,7 @@ __global__ __launch_bounds__(kFineThreads) void k_fine_step(
     const int* __restrict__ contrib) {
   // plane A of population q, then plane B of it
   constexpr int kSets = FINEST ? 2 : 1;
+  constexpr int kFineCells = fine_tile_cells(sizeof(S), FINEST);
   __shared__ S planes[NV - 1][kSets][kFineCells];
   constexpr int kB = kSets - 1;
   constexpr int kCut1 = 5, kCut2 = 10;
@@ -996,7 +995,7 @@ hipError_t launch_fine_stream_zero(int precision, const void* in, void* out, con
 template <typename S>
 static hipError_t fine_step(const FineStep& a, dim3 grid, hipStream_t st) {
 #define LBX_FINE_STEP(FINEST, MIDDLE, AVG)                                                                     \
-  k_fine_step<S, FINEST, MIDDLE, MIDDLE, AVG><<<grid, kFineThreads, 0, st>>>(                                   \
+  k_fine_step<S, FINEST, MIDDLE, MIDDLE, AVG><<<grid, fine_tile_cells(sizeof(S), FINEST), 0, st>>>(                                   \
       (const S*)a.now, (S*)a.next, (const S*)a.parent, a.own, a.tiles, a.ntiles, a.fill, a.strides,             \
       a.parent_stride, a.mask, a.relax, a.avg, a.avg_stride, a.spans, a.cavg, a.cavg_stride, a.contrib)
   if (a.finest)
