@@ -99,14 +99,15 @@ hipError_t launch_step_f64(StepKind kind, const double* src, double* dst, const 
 hipError_t launch_step_f32s(StepKind kind, const float* src, float* dst, const Lattice& L,
                             const Relax& r, LaunchShape s, hipStream_t st);
 
-// Two fused steps in one pass (k_step_pair): tx x ty columns of cells, each in
-// tz chunks of `depth` planes; tx = 0: not used for this lattice.
+// Two fused steps in one pass (k_step_pair): tx x ty columns of bx x by cells,
+// each in tz chunks of `depth` planes; tx = 0: not used for this lattice.
 struct PairShape {
-  int wide;  // columns of kPairWide cells, else kPairSquare
+  int bx, by;
   int tx, ty, tz, depth;
 };
 constexpr int kPairWide[2] = {64, 8};     // whole cache lines in x
 constexpr int kPairSquare[2] = {32, 16};  // smaller ring, less waste at ragged extents
+constexpr int kPairCells = 682;  // of a column and the ring around it, at most: two FP64 planes fill the 160 KB of LDS
 PairShape pair_shape(const Lattice& L, int precision);
 hipError_t launch_step_pair(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
                             const PairShape& p, hipStream_t st);

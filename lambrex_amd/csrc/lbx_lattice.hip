@@ -172,7 +172,8 @@ __global__ __launch_bounds__(512) void k_step_f32s(const float* __restrict__ src
 // workgroups per CU, separate waves for the two steps, non-temporal loads (the
 // ring misses L2); in FP32 32 x 16 (221), 64 x 12 (229), 128 x 5 (226) and 64 x
 // 7 with two workgroups (238).
-constexpr int pair_threads(int bx, int by) { return ((bx + 2) * (by + 2) + 63) / 64 * 64; }
+constexpr int pair_cells(int bx, int by) { return bx ? (bx + 2) * (by + 2) : kPairCells; }
+constexpr int pair_threads(int bx, int by) { return (pair_cells(bx, by) + 63) / 64 * 64; }
 
 template <typename S>
 __device__ __forceinline__ void collide_any(S* f, const Relax& r) {
@@ -198,29 +199,31 @@ __device__ __forceinline__ unsigned lateral_faces(int x, int y, const Lattice& L
   return m;
 }
 
+// BX = 0: columns of p.bx x p.by cells (1 % slower than the same known here)
 template <typename S, int BX, int BY, bool WALLS>
 __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __restrict__ src,
                                                                     S* __restrict__ dst, Lattice L, Relax r,
                                                                     PairShape p) {
-  constexpr int WX = BX + 2, NC = WX * (BY + 2);
+  constexpr int NC = pair_cells(BX, BY);
   __shared__ S ring[2][NV][NC];
+  const int bx = BX ? BX : p.bx, by = BX ? BY : p.by, wx = bx + 2;
   // XCD k takes the k-th eighth of the columns (consecutive workgroups go
   // to the 8 XCDs in turn; the grid is a multiple of 8)
   const int w = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (w >= p.tx * p.ty * p.tz) return;
-  const int x0 = (w % p.tx) * BX, y0 = (w / p.tx % p.ty) * BY, z0 = w / (p.tx * p.ty) * p.depth;
+  const int x0 = (w % p.tx) * bx, y0 = (w / p.tx % p.ty) * by, z0 = w / (p.tx * p.ty) * p.depth;
   const int z1 = min(z0 + p.depth, L.nz);
   const int t = threadIdx.x;
 
   // first step: cell t of the ring, its periodic image in the domain
-  const bool first = t < NC;
-  const int rx = (x0 - 1 + (first ? t % WX : 0) + L.nx) % L.nx, ry = (y0 - 1 + (first ? t / WX : 0) + L.ny) % L.ny;
+  const bool first = t < wx * (by + 2);
+  const int rx = (x0 - 1 + (first ? t % wx : 0) + L.nx) % L.nx, ry = (y0 - 1 + (first ? t / wx : 0) + L.ny) % L.ny;
   const Upstream u = upstream(rx, ry, 0, L);
   // second step: cell (ox, oy) of the column
-  const int ox = x0 + t % BX, oy = y0 + t / BX;
-  const bool second = t < BX * BY && ox < L.nx && oy < L.ny;
+  const int cx = t % bx, cy = t / bx, ox = x0 + cx, oy = y0 + cy;
+  const bool second = cy < by && ox < L.nx && oy < L.ny;
   const int self = oy * L.nx + ox;
-  const int mid = WALLS || t < BX * BY ? (t / BX + 1) * WX + t % BX + 1 : WX + 1;
+  const int mid = WALLS || cy < by ? (cy + 1) * wx + cx + 1 : wx + 1;
 
   // wall faces that a cell touches in x and y, and those that plane z lies on,
   // as a mask of wall_faces(); a population that comes from behind one of
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __r
   auto pull = [&](const S(*plane)[NC], S* f) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
-      const S v = plane[q][mid - kC[q][1] * WX - kC[q][0]];
+      const S v = plane[q][mid - kC[q][1] * wx - kC[q][0]];
       if (kC[q][2] < 0) {
         f[q] = v;
       } else {
@@ -829,15 +832,24 @@ BlockShape block_shape(const Lattice& L) {
   return BlockShape{};
 }
 
-// Shape of the two-step pass for a lattice, or none (p.tx = 0) where two
-// single passes are the faster.  Every workgroup count that fills the device
-// for one or more rounds is a candidate: rounds x (planes of a workgroup + 2
-// of the ring + 1 to start) x the time of a plane, measured as 6.8 us (FP64)
-// and 4.1 us (FP32) at 256^3 and 4.4 and 2.8 us where both buffers stay in
-// the 256 MB MALL.  A single pass is taken at 5.3 TB/s.  At 64^3 the rule
-// takes the pair in FP64 (10.3 against 12.4 us a step) and not in FP32 (6.9
-// against 5.9); at 48^3 in neither (7.1 against 6.4, 5.6 against 4.7); at
-// 96x80x72 in both (19.5 against 25.7, 12.6 against 12.9).
+// Shape of the two-step pass for a lattice, or none (tx = 0) where two single
+// passes are the faster.  Every workgroup count that fills the device for one
+// or more rounds is a candidate: rounds x (planes of a workgroup + 2 of the
+// ring + 1 to start) x the time of a plane, measured as 6.8 us (FP64) and 4.1
+// us (FP32) at 256^3 and 4.4 and 2.8 us where both buffers stay in the 256 MB
+// MALL.  A single pass is taken at 5.3 TB/s.  At 64^3 the rule takes the pair
+// in FP64 (10.2 against 12.4 us a step) and not in FP32 (6.9 against 5.9); at
+// 48^3 in neither (7.1 against 6.4, 5.6 against 4.7); at 96x80x72 in both (18.5
+// against 25.7, 12.2 against 12.9).
+// Columns are 64 x 8 or 32 x 16 cells, or, where that wastes enough of them at
+// the lattice's edges, an even part of a row (or all of it) with as many rows
+// as the ring has room for.  Their rows cross the lines that a wave's lanes
+// share, which is dearer: 1.2 x the time of a plane (1.35 x below 32 cells) and
+// 1.5 x beyond the MALL cover what was measured.  Us per step, with the two
+// and so: 72^3 FP64 18.6 and 14.4, 100^3 FP64 37.5 and 32.4 (FP32 23.3 and
+// 20.2), 48x48x256 21.7 and 18.6 (15.4 and 11.9), 10x256x256 33.0 and 24.4;
+// taken there too it would be slower at 250^3 (405 and 478, 229 and 310) and
+// 161x130x97 (70 and 71, 40.5 and 42).
 PairShape pair_shape(const Lattice& L, int precision) {
   const int cus = compute_units();
   PairShape best{};
@@ -845,21 +857,29 @@ PairShape pair_shape(const Lattice& L, int precision) {
   const bool mall = 2 * bytes <= 256e6;
   const double plane_us = precision == 0 ? (mall ? 4.4 : 6.8) : (mall ? 2.8 : 4.1);
   double best_us = 2 * (2 * bytes / 5.3e6);  // two single passes
-  for (int wide = 1; wide >= 0; --wide) {
-    const int bx = wide ? kPairWide[0] : kPairSquare[0], by = wide ? kPairWide[1] : kPairSquare[1];
+  auto consider = [&](int bx, int by, double factor) {
     const long long tx = (L.nx + bx - 1) / bx, ty = (L.ny + by - 1) / by;
-    if (tx * ty > (1 << 20)) continue;
+    if (tx * ty > (1 << 20)) return;
     for (int chunks = 1; 2 * chunks <= L.nz || chunks == 1; ++chunks) {
       const int depth = (L.nz + chunks - 1) / chunks;
       const long long n = tx * ty * ((L.nz + depth - 1) / depth);
       const long long rounds = (n + cus - 1) / cus;
-      const double us = double(rounds) * (depth + 3) * plane_us;
+      const double us = double(rounds) * (depth + 3) * plane_us * factor;
       if (us < best_us) {
         best_us = us;
-        best = PairShape{wide, (int)tx, (int)ty, (L.nz + depth - 1) / depth, depth};
+        best = PairShape{bx, by, (int)tx, (int)ty, (L.nz + depth - 1) / depth, depth};
       }
       if (rounds > 16) break;  // deeper splits only add ring planes
     }
+  };
+  consider(kPairWide[0], kPairWide[1], 1.0);
+  consider(kPairSquare[0], kPairSquare[1], 1.0);
+  for (int parts = 1; parts <= L.nx; ++parts) {
+    const int bx = (L.nx + parts - 1) / parts, rows = kPairCells / (bx + 2) - 2;
+    if (rows < 1) continue;
+    if (bx < 16 && parts > 1) break;
+    const int pieces = (L.ny + rows - 1) / rows;
+    consider(bx, (L.ny + pieces - 1) / pieces, !mall ? 1.5 : bx < 32 && parts > 1 ? 1.35 : 1.2);
   }
   return best;
 }
@@ -869,15 +889,19 @@ static hipError_t step_pair(const S* src, S* dst, const Lattice& L, const Relax&
                             hipStream_t st) {
   constexpr int wx = kPairWide[0], wy = kPairWide[1], qx = kPairSquare[0], qy = kPairSquare[1];
   const unsigned grid = unsigned(((long long)p.tx * p.ty * p.tz + 7) / 8 * 8);
-  const bool walls = L.walls != 0;
-  if (p.wide && walls)
+  const bool walls = L.walls != 0, wide = p.bx == wx && p.by == wy, square = p.bx == qx && p.by == qy;
+  if (wide && walls)
     k_step_pair<S, wx, wy, true><<<grid, pair_threads(wx, wy), 0, st>>>(src, dst, L, r, p);
-  else if (p.wide)
+  else if (wide)
     k_step_pair<S, wx, wy, false><<<grid, pair_threads(wx, wy), 0, st>>>(src, dst, L, r, p);
-  else if (walls)
+  else if (square && walls)
     k_step_pair<S, qx, qy, true><<<grid, pair_threads(qx, qy), 0, st>>>(src, dst, L, r, p);
-  else
+  else if (square)
     k_step_pair<S, qx, qy, false><<<grid, pair_threads(qx, qy), 0, st>>>(src, dst, L, r, p);
+  else if (walls)
+    k_step_pair<S, 0, 0, true><<<grid, pair_threads(0, 0), 0, st>>>(src, dst, L, r, p);
+  else
+    k_step_pair<S, 0, 0, false><<<grid, pair_threads(0, 0), 0, st>>>(src, dst, L, r, p);
   return hipGetLastError();
 }
 
