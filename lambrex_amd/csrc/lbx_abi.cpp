@@ -919,7 +919,8 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
           n += (long long)parts(std::get<0>(s.first), wx) * parts(std::get<1>(s.first), wy) * nz * s.second;
           planes = std::max(planes, widest(gz, nz) + 2);
         }
-        const double us = (double)((n + cus - 1) / cus) * planes * plane_us;
+        const long long slots = room <= 256 ? 2 * cus : cus;  // workgroups of 4 waves: two to a CU
+        const double us = (double)((n + slots - 1) / slots) * planes * plane_us;
         if (n < (1 << 24) && us < best_us) {
           best_us = us;
           best[0] = wx;

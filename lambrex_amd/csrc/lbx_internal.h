@@ -222,10 +222,17 @@ struct FineTile {
   int patch;
   int lo[3], hi[3];
 };
-// 8 waves, whose 256 registers a lane FP64 and the middle levels' sums need; the
-// finest level in FP32 does with 168 and so takes 12 (128^3 with a 64x256x256
-// level 360 -> 306 us a step; a middle level spills).
-constexpr int fine_tile_cells(int elem_bytes, bool finest) { return elem_bytes == 4 && finest ? 768 : 512; }
+// FP64 needs 220 registers a lane, so 8 waves a CU: the finest level's in one
+// workgroup; a middle level's in two of 4 waves, one of which goes on while the
+// other waits for the block averages of cells that several of the child's
+// patches touch (three levels over 64^3 650 -> 587 us a step, over 128^3 2494 ->
+// 2294; the finest level loses by it, 549 -> 639 us for 128^3 with a 64x256x256
+// level).  In FP32 the finest level does with 168 and so takes 12 waves (360 ->
+// 306 us for that hierarchy); a middle level spills there, and two workgroups
+// of 4 are slower (370 -> 398 us for three levels over 64^3).
+constexpr int fine_tile_cells(int elem_bytes, bool finest) {
+  return elem_bytes == 8 ? finest ? 512 : 256 : finest ? 768 : 512;
+}
 
 constexpr unsigned long long kFillParent = 1ull << 63, kFillElement = (1ull << 40) - 1;
 constexpr int kFillStrideShift = 40;
