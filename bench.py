@@ -134,8 +134,10 @@ def traffic_for(kernel, workload):
 
 def step_traffic(key, workload):
     """Measured bytes per level-0 step of a hierarchy (every kernel of the
-    step, FETCH_SIZE + WRITE_SIZE scaled) against its algorithmic 240 B per
-    lattice update, from the committed counter summary, or None."""
+    step, FETCH_SIZE + WRITE_SIZE scaled) against its algorithmic bytes (240 B
+    per lattice update for the entries of one pass per stage, each level's
+    state read and written once per pass over it for the fused ones), from the
+    committed counter summary, or None."""
     try:
         d = json.loads(TRAFFIC_FILE.read_text())[key][workload]
         return {"bytes_per_step": d["bytes_per_step"], "algorithmic_bytes_per_step": d["algorithmic_bytes"],
@@ -144,13 +146,14 @@ def step_traffic(key, workload):
         return None
 
 
-def hierarchy_roofline(mlups, ms_per_step, precision, traffic):
+def hierarchy_roofline(state_cells, ms_per_step, precision, traffic):
     """Where a hierarchy step sits against the 8 TB/s HBM peak: its
-    algorithmic bytes (240 B or 120 B per lattice update) per second, and,
-    for FP64, the measured bytes per step (every kernel's FETCH_SIZE +
-    WRITE_SIZE, which also count lines served by the MALL) per second."""
-    bpl = 240 if precision == lbx.LBX_FP64 else 120
-    alg = mlups * 1e6 * bpl / 1e9
+    algorithmic bytes (each level's state read and written once per pass over
+    it: 240 B or 120 B for each of `state_cells` cells) per second, and, for
+    FP64, the measured bytes per step (every kernel's FETCH_SIZE + WRITE_SIZE,
+    which also count lines served by the MALL) per second."""
+    bpc = 240 if precision == lbx.LBX_FP64 else 120
+    alg = state_cells * bpc / (ms_per_step * 1e-3) / 1e9
     out = {"bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s", "algorithmic_gbs": round(alg, 1),
            "algorithmic_frac": round(alg / HBM_PEAK_GBS, 4)}
     if traffic:
@@ -322,13 +325,13 @@ def two_level(ctx, steps, warmup, precision=lbx.LBX_FP64):
         sim.close()
     lu = lu_per_step * steps
     name = "FP64" if precision == lbx.LBX_FP64 else "FP32-shifted"
-    traffic = step_traffic("two_level_step", "128^3 + 64x256x256") if precision == lbx.LBX_FP64 else None
+    traffic = step_traffic("two_level_fused_step", "128^3 + 64x256x256") if precision == lbx.LBX_FP64 else None
     return {"workload": "coarse 128^3 (64 boxes of 32^3) + fine 64x256x256 (128 boxes of 32^3), "
                         f"ratio 2, 2 fine substeps per coarse step, {name}",
             "coarse_steps": steps, "warmup_steps": warmup, "mlups": lu / (t1 - t0) / 1e6,
             "ms_per_coarse_step": (t1 - t0) * 1e3 / steps,
             "traffic_per_step": traffic,
-            "roofline": hierarchy_roofline(lu / (t1 - t0) / 1e6, (t1 - t0) * 1e3 / steps, precision, traffic)}, fields
+            "roofline": hierarchy_roofline(128 ** 3 + 64 * 256 ** 2, (t1 - t0) * 1e3 / steps, precision, traffic)}, fields
 
 
 def three_level_geometry():
@@ -377,14 +380,15 @@ def three_level(ctx, steps, warmup, precision=lbx.LBX_FP64):
         sim.close()
     lu = lu_per_step * steps
     name = "FP64" if precision == lbx.LBX_FP64 else "FP32-shifted"
-    traffic = (step_traffic("three_level_step", "128^3 + 64x256x256 + 32x512x512")
+    traffic = (step_traffic("three_level_fused_step", "128^3 + 64x256x256 + 32x512x512")
                if precision == lbx.LBX_FP64 else None)
     return {"workload": "coarse 128^3 (64 boxes of 32^3) + level 1 64x256x256 (128 boxes of 32^3) + level 2 "
                         f"32x512x512 (256 boxes of 32^3), ratio 2, {name}",
             "coarse_steps": steps, "warmup_steps": warmup, "mlups": lu / (t1 - t0) / 1e6,
             "ms_per_coarse_step": (t1 - t0) * 1e3 / steps,
             "traffic_per_step": traffic,
-            "roofline": hierarchy_roofline(lu / (t1 - t0) / 1e6, (t1 - t0) * 1e3 / steps, precision, traffic),
+            "roofline": hierarchy_roofline(128 ** 3 + 2 * 64 * 256 ** 2 + 2 * 32 * 512 ** 2, (t1 - t0) * 1e3 / steps,
+                                           precision, traffic),
             "final_rho_range_per_level": [[float(np.min(r)), float(np.max(r))] for r in rhos]}, rhos
 
 
