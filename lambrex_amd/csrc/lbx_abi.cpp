@@ -98,7 +98,7 @@ struct Level {
   std::vector<PatchDesc> gdesc;
   PatchDesc* d_gdesc = nullptr;
   std::vector<std::pair<int, int>> groups;  // (first position in gdesc, count)
-  lbx::FineTile* d_tiles = nullptr;  // the finest level's, then a middle level's
+  lbx::FineTile* d_tiles[2] = {nullptr, nullptr};  // as the finest level; with a finer one, planned with that
   int ntiles[2] = {0, 0};
   double* d_avg = nullptr;       // 15 planes of avg_stride 2x2x2 block averages
   long long avg_stride = 0;
@@ -239,7 +239,8 @@ void free_level(Level& L) {
   if (L.d_sum_contrib) (void)hipFree(L.d_sum_contrib);
   if (L.d_sum_span) (void)hipFree(L.d_sum_span);
   if (L.d_gdesc) (void)hipFree(L.d_gdesc);
-  if (L.d_tiles) (void)hipFree(L.d_tiles);
+  for (lbx::FineTile* t : L.d_tiles)
+    if (t) (void)hipFree(t);
   if (L.d_avg) (void)hipFree(L.d_avg);
   L = Level{};
 }
@@ -509,7 +510,7 @@ lbx::FineStep fine_step_args(const lbx_sim* sim, int l, bool finest, bool averag
   a.next = L.buf[1 - par[l]];
   a.parent = P.buf[par[l - 1]];
   a.own = L.d_gdesc;
-  a.tiles = L.d_tiles + (finest ? 0 : L.ntiles[0]);
+  a.tiles = L.d_tiles[finest ? 0 : 1];
   a.ntiles = L.ntiles[finest ? 0 : 1];
   a.fill = (const unsigned long long*)L.d_fill;
   a.strides = L.d_strides;
@@ -859,7 +860,9 @@ std::vector<unsigned char> patch_mask(const Level& C, const std::vector<Box>& ma
 int part_begin(int g, int n, int k) { return 2 * (int)((long long)(g / 2) * k / n); }
 
 // Cuts patches into tiles for launch_fine_step.  Every patch is cut into parts
-// of at most `want` cells per direction; the target that costs least is taken:
+// of at most `want` cells per direction (4 or more, in z 2: on a small level the
+// planes a workgroup walks are all the time, 24^3 with a 16-wide level 42 -> 37
+// us a step); the target that costs least is taken:
 // rounds of workgroups over the CUs x planes a workgroup walks (its own and
 // up to 4 around them, and 2 of the pipeline) x time of a plane (2.5 us + 0.4
 // us, in FP32 0.2, per wave of its A plane).  The model only ranks the targets:
@@ -888,17 +891,17 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   int best[3] = {4, 4, gmax[2]};
   double best_us = 1e300;
-  auto targets = [](int g) {
+  auto targets = [](int g, int least) {
     std::vector<int> t;
     for (int n = 1; n <= 64; ++n) {
       const int want = ((g + n - 1) / n + 1) / 2 * 2;
-      if (want >= 4 && (t.empty() || t.back() != want)) t.push_back(want);
+      if (want >= least && (t.empty() || t.back() != want)) t.push_back(want);
     }
     if (t.empty()) t.push_back(g);
-    if (t.back() > 4) t.push_back(4);
+    if (t.back() > least) t.push_back(least);
     return t;
   };
-  const std::vector<int> tx = targets(gmax[0]), ty = targets(gmax[1]), tz = targets(gmax[2]);
+  const std::vector<int> tx = targets(gmax[0], 4), ty = targets(gmax[1], 4), tz = targets(gmax[2], 2);
   for (int wx : tx)
     for (int wy : ty) {
       long long columns = 0;
@@ -948,6 +951,14 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
         }
   }
   return tiles;
+}
+
+// Plans and uploads a level's tiles for its steps as the finest or a middle
+// level; returns when they have arrived.
+hipError_t set_tiles(lbx_sim* sim, Level& L, bool finest) {
+  const std::vector<lbx::FineTile> t = plan_tiles(L.gdesc, (int)elem_size(sim->precision), finest);
+  L.ntiles[finest ? 0 : 1] = (int)t.size();
+  return upload(&L.d_tiles[finest ? 0 : 1], t, sim->ctx->stream);
 }
 
 // Level l >= 1: patches grown by 2; ghost-fill sources; average-down table
@@ -1062,13 +1073,6 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
       k += n;
     }
   }
-  std::vector<lbx::FineTile> tiles;
-  for (int middle = 0; r == 2 && middle < 2; ++middle) {
-    const std::vector<lbx::FineTile> t =
-        plan_tiles(F.gdesc, (int)elem_size(sim->precision), !middle);
-    F.ntiles[middle] = (int)t.size();
-    tiles.insert(tiles.end(), t.begin(), t.end());
-  }
   // Ghost fill sources (FillPatchTwoLevels with piecewise-constant
   // interpolation, src/AmrSim.cpp:373-388): the valid cell of this level
   // holding the periodic image if a box has it, else the coarse parent.
@@ -1081,13 +1085,18 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
   for (const PatchDesc& p : F.desc) same &= p.qs == F.desc[0].qs;
   for (const PatchDesc& p : C.desc) same &= !C.patched || p.qs == C.desc[0].qs;
   std::map<long long, unsigned> stride_ids;
-  auto packed_source = [&](unsigned long long parent, long long elem, long long qs) {
-    unsigned long long id = 0;
-    if (!same) {
-      const auto it = stride_ids.emplace(qs, (unsigned)stride_ids.size());
-      if (it.second) strides.push_back((unsigned)qs);
-      id = it.first->second;
-    }
+  auto stride_id = [&](long long qs) {
+    const auto it = stride_ids.emplace(qs, (unsigned)stride_ids.size());
+    if (it.second) strides.push_back((unsigned)qs);
+    return it.first->second;
+  };
+  std::vector<unsigned> own_id, parent_id;  // per patch; a level array has one
+  if (r == 2 && !same) {
+    for (const PatchDesc& p : F.desc) own_id.push_back(stride_id(p.qs));
+    for (const PatchDesc& p : C.desc) parent_id.push_back(stride_id(C.patched ? p.qs : C.lat.ps));
+  }
+  auto packed_source = [&](unsigned long long parent, const std::vector<unsigned>& ids, int patch, long long elem) {
+    const unsigned long long id = same ? 0 : ids[patch];
     return (long long)(parent | id << lbx::kFillStrideShift | (unsigned long long)elem);
   };
   int hint = 0;
@@ -1113,7 +1122,7 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
           if (src >= 0) {
             hint = src;
             const PatchDesc& Q = F.desc[src];
-            d = r == 2 ? packed_source(0, Q.at(wx - Q.lo[0] + 2, wy - Q.lo[1] + 2, wz - Q.lo[2] + 2), Q.qs)
+            d = r == 2 ? packed_source(0, own_id, src, Q.at(wx - Q.lo[0] + 2, wy - Q.lo[1] + 2, wz - Q.lo[2] + 2))
                        : ((long long)src << 32) | grown_index(Q, wx, wy, wz);
           } else {
             long long ref;
@@ -1126,10 +1135,10 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
               d = -1 - ref;
             } else if (C.patched) {
               const PatchDesc& Q = C.desc[ref >> 32];
-              d = packed_source(lbx::kFillParent,
-                                Q.at(wx / r - Q.lo[0] + 2, wy / r - Q.lo[1] + 2, wz / r - Q.lo[2] + 2), Q.qs);
+              d = packed_source(lbx::kFillParent, parent_id, (int)(ref >> 32),
+                                Q.at(wx / r - Q.lo[0] + 2, wy / r - Q.lo[1] + 2, wz / r - Q.lo[2] + 2));
             } else {
-              d = packed_source(lbx::kFillParent, ref, C.lat.ps);
+              d = packed_source(lbx::kFillParent, parent_id, 0, ref);
             }
           }
           fill[P.fill_base + ((long long)gz * P.g[1] + gy) * P.g[0] + gx] = d;
@@ -1203,7 +1212,8 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
   }
   hipError_t e = upload(&F.d_desc, F.desc, ctx->stream);
   if (e == hipSuccess) e = upload(&F.d_gdesc, F.gdesc, ctx->stream);
-  if (e == hipSuccess) e = upload(&F.d_tiles, tiles, ctx->stream);
+  if (e == hipSuccess && r == 2) e = set_tiles(sim, F, true);
+  if (e == hipSuccess && C.patched && r == 2 && !C.d_tiles[1]) e = set_tiles(sim, C, false);
   if (e == hipSuccess) e = upload(&F.d_fill, fill, ctx->stream);
   if (e == hipSuccess) e = upload(&F.d_strides, strides, ctx->stream);
   if (e == hipSuccess && !C.patched) e = upload(&F.d_sum_cell, cell, ctx->stream);
