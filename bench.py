@@ -103,7 +103,7 @@ def measure(ctx, dims, mgs, tau, rho, u, precision, steps, warmup, keep_fields=F
     storage = "double" if precision == lbx.LBX_FP64 else "float"
     wall_arg = "" if all(periodic) else ", walls"
     if launches and 2 * launches <= steps + 1 and steps > 1:
-        name = "k_step_block" if cells <= 65536 else "k_step_pair"  # blocks of at most 256 cells on 256 CUs
+        name = "k_step_block" if cells <= 110592 else "k_step_pair"  # blocks of at most 432 cells per CU
         kernel = f"{name}<{storage}{wall_arg}>"
     else:
         kernel = f"k_step_{'f64' if precision == lbx.LBX_FP64 else 'f32s'}<STEP_FUSED{wall_arg}>"

@@ -743,7 +743,7 @@ int define_level0(lbx_sim* sim, const std::vector<Box>& boxes) {
   L.boxes = boxes;
   L.lat = lbx::make_lattice(sim->dims[0], sim->dims[1], sim->dims[2], (int)elem_size(sim->precision));
   L.lat.walls = sim->walls;
-  L.block = lbx::block_shape(L.lat);
+  L.block = lbx::block_shape(L.lat, sim->precision);
   L.pair = L.block.steps ? lbx::PairShape{} : lbx::pair_shape(L.lat, sim->precision);
   const size_t bytes = (size_t)L.lat.elems() * elem_size(sim->precision);
   for (int i = 0; i < 2; ++i) {

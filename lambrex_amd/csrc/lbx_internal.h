@@ -120,7 +120,7 @@ struct BlockShape {
   int b[3], n[3];
 };
 constexpr int kBlockCells = 768;  // of a block and its ring, at most
-BlockShape block_shape(const Lattice& L);
+BlockShape block_shape(const Lattice& L, int precision);
 hipError_t launch_step_block(int precision, const void* src, void* dst, const Lattice& L, const Relax& r,
                              const BlockShape& b, int steps, hipStream_t st);
 

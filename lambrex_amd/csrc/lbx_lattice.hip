@@ -228,7 +228,8 @@ __global__ __launch_bounds__(pair_threads(BX, BY)) void k_step_pair(const S* __r
   // wall faces that a cell touches in x and y, and those that plane z lies on,
   // as a mask of wall_faces(); a population that comes from behind one of
   // them is the cell's own opposite population
-  const unsigned first_faces = WALLS ? lateral_faces(rx, ry, L) : 0, second_faces = WALLS ? lateral_faces(ox, oy, L) : 0;
+  const unsigned first_faces = WALLS ? lateral_faces(rx, ry, L) : 0;
+  const unsigned second_faces = WALLS ? lateral_faces(ox, oy, L) : 0;
   auto z_faces = [&](int z) { return (L.walls & 4u) ? (z == 0 ? 16u : 0u) | (z == L.nz - 1 ? 32u : 0u) : 0u; };
 
   auto load = [&](int z, S* f) {
@@ -814,20 +815,24 @@ static int compute_units() {
 // fused steps save (48^3 FP64 6.8 to 7.5 us a step in two rounds, 6.2 in
 // single passes).  Of 15 shapes swept at 16^3 to 40^3 and 10x10x50 these are
 // the fastest: 4x4x4 of 3 steps at 24^3 (3.15 us, the 2-step blocks 3.2 and
-// more), 8x4x4 of 2 at 32^3 (3.6; 4x4x8 of 3 steps 4.0), 8x8x4 at 40^3.
-BlockShape block_shape(const Lattice& L) {
-  static constexpr int kShapes[3][4] = {{3, 4, 4, 4}, {2, 8, 4, 4}, {2, 8, 8, 4}};
+// more), 8x4x4 of 2 at 32^3 (3.6; 4x4x8 of 3 steps 4.0), 8x8x4 at 40^3.  In FP32
+// two blocks of 6x6x6 share a CU (48^3 5.3 us a step in single passes, 4.7 so).
+BlockShape block_shape(const Lattice& L, int precision) {
+  // steps, cells of a block, blocks per CU
+  static constexpr int kShapes[4][5] = {{3, 4, 4, 4, 1}, {2, 8, 4, 4, 1}, {2, 8, 8, 4, 1}, {2, 6, 6, 6, 2}};
   const long long n[3] = {L.nx, L.ny, L.nz};
-  for (const int(&c)[4] : kShapes) {
+  for (const int(&c)[5] : kShapes) {
+    const long long room = (long long)c[4] * compute_units();
+    if (c[4] > 1 && precision == 0) continue;
     BlockShape b{};
     b.steps = c[0];
     long long blocks = 1;
     for (int d = 0; d < 3; ++d) {
       b.b[d] = c[1 + d];
       b.n[d] = int((n[d] + c[1 + d] - 1) / c[1 + d]);
-      blocks = blocks > compute_units() ? blocks : blocks * b.n[d];
+      blocks = blocks > room ? blocks : blocks * b.n[d];
     }
-    if (blocks <= compute_units()) return b;
+    if (blocks <= room) return b;
   }
   return BlockShape{};
 }

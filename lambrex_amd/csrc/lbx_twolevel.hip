@@ -995,7 +995,7 @@ hipError_t launch_fine_stream_zero(int precision, const void* in, void* out, con
 template <typename S>
 static hipError_t fine_step(const FineStep& a, dim3 grid, hipStream_t st) {
 #define LBX_FINE_STEP(FINEST, MIDDLE, AVG)                                                                     \
-  k_fine_step<S, FINEST, MIDDLE, MIDDLE, AVG><<<grid, fine_tile_cells(sizeof(S), FINEST), 0, st>>>(                                   \
+  k_fine_step<S, FINEST, MIDDLE, MIDDLE, AVG><<<grid, fine_tile_cells(sizeof(S), FINEST), 0, st>>>( \
       (const S*)a.now, (S*)a.next, (const S*)a.parent, a.own, a.tiles, a.ntiles, a.fill, a.strides,             \
       a.parent_stride, a.mask, a.relax, a.avg, a.avg_stride, a.spans, a.cavg, a.cavg_stride, a.contrib)
   if (a.finest)

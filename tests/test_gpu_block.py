@@ -28,6 +28,11 @@ CASES = [  # dims, periodic
     ((250, 2, 3), (1, 0, 1)),
     ((3, 2, 1000), (1, 1, 1)),
 ]
+FP32_CASES = [  # two blocks to a CU, in FP32 only
+    ((48, 48, 48), (1, 1, 1)),
+    ((47, 43, 46), (0, 1, 0)),
+    ((84, 31, 35), (1, 1, 1)),
+]
 
 
 @pytest.fixture(scope="module")
@@ -36,8 +41,9 @@ def ctx():
         yield c
 
 
-@pytest.mark.parametrize("precision", [lbx.LBX_FP64, lbx.LBX_FP32_SHIFTED])
-@pytest.mark.parametrize("dims,periodic", CASES)
+@pytest.mark.parametrize("dims,periodic,precision",
+                         [c + (p,) for c in CASES for p in (lbx.LBX_FP64, lbx.LBX_FP32_SHIFTED)]
+                         + [c + (lbx.LBX_FP32_SHIFTED,) for c in FP32_CASES])
 def test_blocks_equal_single_passes(ctx, dims, periodic, precision):
     rho, u = workloads.random_state(dims, 5, 1e-2, 0.03)
     a, b = (start(ctx, dims, periodic, precision, rho, u) for _ in range(2))
