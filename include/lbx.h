@@ -259,11 +259,11 @@ int lbx_bench_copy(lbx_ctx* ctx, size_t bytes, int reps, double* gbs);
  * (ratio 2) stepped by the Rohde cycle (src/AmrSim.cpp:430-469).
  * Single-level requests are admitted while the server's device arena has
  * room and advance together, one patch-list kernel launch per step (or per two,
- * where that is faster) over the work items of every active run; a refined run is admitted while the
- * device has memory for its levels, is held in a simulation of its own on
- * the context (one captured level-0 step per server step, on the context's
- * stream, overlapping the patch-list launches on the server's stream) and
- * is released when delivered.  Each run computes exactly what lbx_iterate
+ * where that is faster) over the work items of every active run; a refined
+ * run is admitted while the device has memory for its levels, is held in a
+ * simulation of its own on the context (one level-0 step per server step, on
+ * the context's stream, overlapping the patch-list launches on the server's
+ * stream) and is released when delivered.  Each run computes exactly what lbx_iterate
  * computes for it alone, bit for bit. */
 
 #define LBX_INIT_PLANE_PULSE 0  /* rho = 1 + amplitude on plane `plane` normal to `axis`, u = 0 */

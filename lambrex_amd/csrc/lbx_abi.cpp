@@ -1231,7 +1231,7 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
 
 // Level `level`'s mask bytes with no cell masked (a level starts unmasked;
 // on a level array they still carry the box-face bits of the coarse push).
-// The device buffer is kept if there is one, so captured steps stay valid.
+// The device buffer is kept if there is one.
 int unmask_level(lbx_sim* sim, int level) {
   lbx_ctx* ctx = sim->ctx;
   Level& C = sim->lev[level];

@@ -20,8 +20,7 @@
 //
 // A request with fine boxes is a refined run: a two-level hierarchy (ratio
 // 2, the fine-grid mask) held in a simulation of its own, made through the
-// C ABI on the server's context, whose level-0 steps (one captured Rohde
-// cycle each) go to the context's stream while the patch-list launches of
+// C ABI on the server's context, whose level-0 steps go to the context's stream while the patch-list launches of
 // the single-level runs go to the server's stream, so the two overlap on the
 // device.  It takes one coarse step per global step, is admitted against
 // the device's free memory (its levels are allocated when it is admitted
