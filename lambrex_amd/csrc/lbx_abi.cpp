@@ -1106,7 +1106,10 @@ int build_level(lbx_sim* sim, int level, const std::vector<Box>& boxes, Level& F
       for (int gy = 0; gy < P.g[1]; ++gy)
         for (int gx = 0; gx < P.g[0]; ++gx) {
           const int x = P.lo[0] - 2 + gx, y = P.lo[1] - 2 + gy, z = P.lo[2] - 2 + gz;
-          if (boxes[b].contains(x, y, z)) continue;
+          if (boxes[b].contains(x, y, z)) {  // the row's valid cells have no entry
+            gx += boxes[b].hi[0] - x;
+            continue;
+          }
           const int wx = wrap(x, fdom[0]), wy = wrap(y, fdom[1]), wz = wrap(z, fdom[2]);
           int src = -1;
           if (boxes[hint].contains(wx, wy, wz)) {

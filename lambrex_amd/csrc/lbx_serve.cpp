@@ -127,6 +127,7 @@ struct Run {
   int passes = 0;        // passes launched, of steps + 1: collide, steps - 1 fused, stream
   int cur = 0;           // buffer that holds the state after them
   short bx = 0, by = 0;  // column of cells of a work item of two passes
+  long long columns = 0, cells = 0;
   double t_admit = 0.0;
   bool launched_last = false;
   long long last_step = 0;
@@ -307,10 +308,8 @@ void pair_column(Run& r) {
       r.by = (short)((ny + ty - 1) / ty);
     }
   }
-}
-
-long long columns(const Run& r) {
-  return (long long)((r.r.req.dims[0] + r.bx - 1) / r.bx) * ((r.r.req.dims[1] + r.by - 1) / r.by);
+  r.columns = (long long)((nx + r.bx - 1) / r.bx) * ((ny + r.by - 1) / r.by);
+  r.cells = cells_of(r.r.req);
 }
 
 // Planes per work item, from the cost of a launch: rounds of items over the
@@ -325,7 +324,7 @@ int pair_depth(const lbx_server* s) {
   for (int depth = 8; depth <= 32; depth *= 2) {
     long long items = 0;
     for (const Run& r : s->active)
-      if (!r.sim && !r.launched_last) items += columns(r) * ((r.r.req.dims[2] + depth - 1) / depth);
+      if (!r.sim && !r.launched_last) items += r.columns * ((r.r.req.dims[2] + depth - 1) / depth);
     const long long cost = (items + s->cus - 1) / s->cus * (depth + 3);
     if (depth == 8 || cost < best) {
       best = cost;
@@ -339,15 +338,16 @@ int pair_depth(const lbx_server* s) {
 // (kPairCells), in lattices whose columns keep most lanes busy (a cube's do to
 // 2/3 and more; a row of cells is better off as 256 cells per item).
 bool pairs_pay(const lbx_server* s) {
-  long long cells = 0, lanes = 0, left = 0;
+  long long cells = 0, lanes = 0;
+  bool more = false;
   for (const Run& r : s->active) {
     if (r.launched_last) continue;
-    left = std::max(left, r.sim ? (long long)r.r.req.steps - r.steps_done : (long long)r.r.req.steps + 1 - r.passes);
+    more |= r.sim ? r.r.req.steps - r.steps_done > 1 : r.r.req.steps + 1 - r.passes > 1;
     if (r.sim) continue;
-    cells += cells_of(r.r.req);
-    lanes += columns(r) * lbx::kServePairCells * r.r.req.dims[2];
+    cells += r.cells;
+    lanes += r.columns * lbx::kServePairCells * r.r.req.dims[2];
   }
-  return left > 1 && cells >= kPairCells && lanes <= 2 * cells;
+  return more && cells >= kPairCells && lanes <= 2 * cells;
 }
 
 // Admission: move queued requests into the active set while they fit, in
@@ -573,20 +573,21 @@ int collect(lbx_server* s, bool wait) {
     res.t_admit = r.t_admit;
     res.t_done = now_s();
     // The run's last state is complete and stays until its arena space is
-    // released: its outputs go by a stream of their own, beside the steps
-    // already queued for the other runs.
+    // released: larger outputs go by a stream of their own, beside the steps
+    // already queued for the other runs (small ones lose 20 us by it).
+    const hipStream_t out = n * 4 * sizeof(double) >= ((size_t)2 << 20) ? s->out : s->stream;
     if (rq.out_rho || rq.out_u) {
-      SRV_HIP(s, lbx::launch_hydro(s->precision, false, fin, L, R, s->staging, s->staging + n, s->rho0, s->out));
+      SRV_HIP(s, lbx::launch_hydro(s->precision, false, fin, L, R, s->staging, s->staging + n, s->rho0, out));
       lbx::ReadBack::Part parts[2];
       int k = 0;
       if (rq.out_rho) parts[k++] = {rq.out_rho, s->staging, n * sizeof(double)};
       if (rq.out_u) parts[k++] = {rq.out_u, s->staging + n, 3 * n * sizeof(double)};
-      SRV_HIP(s, lbx::ctx_readback(s->ctx).copy(s->device, parts, k, s->out));
+      SRV_HIP(s, lbx::ctx_readback(s->ctx).copy(s->device, parts, k, out));
     }
     if (rq.out_f) {
-      SRV_HIP(s, lbx::launch_pack_f(s->precision, false, fin, L, R, s->staging, s->rho0, s->out));
+      SRV_HIP(s, lbx::launch_pack_f(s->precision, false, fin, L, R, s->staging, s->rho0, out));
       const lbx::ReadBack::Part part{rq.out_f, s->staging, lbx::NV_TOTAL * n * sizeof(double)};
-      SRV_HIP(s, lbx::ctx_readback(s->ctx).copy(s->device, &part, 1, s->out));
+      SRV_HIP(s, lbx::ctx_readback(s->ctx).copy(s->device, &part, 1, out));
     }
     s->lattice_updates += n * (int64_t)rq.steps;
     s->arena.release(r.off, r.bytes);
@@ -650,7 +651,7 @@ int launch_steps(lbx_server* s, int width) {
       d.by = r.by;
       const int chunks = (d.n[2] + depth - 1) / depth;
       d.depth = (d.n[2] + chunks - 1) / chunks;
-      items += (int)(columns(r) * ((d.n[2] + d.depth - 1) / d.depth));
+      items += (int)(r.columns * ((d.n[2] + d.depth - 1) / d.depth));
       r.passes += alone ? 1 : 2;
     } else {
       d.kind = r.passes == 0 ? lbx::STEP_COLLIDE : r.passes == last ? lbx::STEP_STREAM : lbx::STEP_FUSED;
