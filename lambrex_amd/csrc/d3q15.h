@@ -181,11 +181,12 @@ LBX_HD double third_of(double x) {
 // The relaxation of the stress modes (src/AmrSim.cpp:51-93) in the reference's
 // order.  With SHARED the divisions by the density share one reciprocal and
 // those by 3 are third_of: the same correctly rounded quotients while the
-// density and the squares stay far from the ends of the range, which is what
-// the result says; otherwise the caller takes the divisions themselves.  A
-// momentum or trace so small that its remainder underflows (2^-950) needs no
-// check: its quotient enters f in terms below 2^-700, next to a density above
-// 2^-100.
+// density, the squares and the trace, relaxed or not, stay far from the ends of
+// the range, which is what the result says (of an infinite trace, which a rate
+// without bound makes, third_of would make a NaN); otherwise the caller takes
+// the divisions themselves.  A momentum or trace so small that its remainder
+// underflows (2^-950) needs no check: its quotient enters f in terms below
+// 2^-700, next to a density above 2^-100.
 // The two-step passes are bound by FP64 issue: 96x80x72 with walls 7.44 -> 7.20
 // ms and 256^3 180.5 -> 178.9 ms for whole runs, 128^3 with a 64x256x256 level
 // 85.6 -> 84.7 ms.
@@ -220,12 +221,14 @@ LBX_HD bool relax_f64(double* mode, double omega_s, double omega_b) {
   TrS = TrS + s00;
   TrS = TrS + s11;
   TrS = TrS + s22;
-  const bool plain = density > 0x1p-100 && density < 0x1p100 && usq < 0x1p400 && TrS < 0x1p900 && TrS > -0x1p900;
+  const double trace = TrS;
   const double third_tr = SHARED ? third_of(TrS) : TrS / 3.0;
   s00 = s00 - third_tr;
   s11 = s11 - third_tr;
   s22 = s22 - third_tr;
   TrS = TrS - omega_b * (TrS - density * usq);
+  const bool plain = density > 0x1p-100 && density < 0x1p100 && usq < 0x1p400 &&
+                     __builtin_fmax(__builtin_fabs(trace), __builtin_fabs(TrS)) < 0x1p900;
   const double third_relaxed = SHARED ? third_of(TrS) : TrS / 3.0;
   // Off-diagonal: usq * DELTA = +0, and x - (+0) == x exactly.
   s00 = s00 - omega_s * (s00 - density * (v[0] * v[0] - usq * DELTA_D));
