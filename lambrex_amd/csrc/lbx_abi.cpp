@@ -223,8 +223,12 @@ hipError_t upload(T** dptr, const std::vector<T>& h, hipStream_t st) {
   hipError_t e = hipMalloc(dptr, h.size() * sizeof(T));
   if (e != hipSuccess) return e;
   e = hipMemcpyAsync(*dptr, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st);
-  if (e != hipSuccess) return e;
-  return hipStreamSynchronize(st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e != hipSuccess) {  // a table that did not arrive is not there
+    (void)hipFree(*dptr);
+    *dptr = nullptr;
+  }
+  return e;
 }
 
 void free_level(Level& L) {
@@ -1247,13 +1251,18 @@ int unmask_level(lbx_sim* sim, int level) {
 }
 
 // A level replaces any level at its index and discards the finer ones; its
-// parent starts unmasked.
+// parent starts unmasked.  Nothing is replaced before the parent has its mask:
+// a level's parent is stepped with one.
 int define_level(lbx_sim* sim, int level, const std::vector<Box>& boxes) {
   Level nf;
   if (int rc = build_level(sim, level, boxes, nf)) return rc;
+  if (int rc = unmask_level(sim, level - 1)) {
+    free_level(nf);
+    return rc;
+  }
   free_levels_from(sim, level);
   sim->lev[level] = nf;
-  return unmask_level(sim, level - 1);
+  return LBX_OK;
 }
 
 // RemakeLevel (src/AmrSim.cpp:715-744) of the finest level: a new BoxArray
