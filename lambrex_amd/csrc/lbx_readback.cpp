@@ -11,14 +11,11 @@ namespace lbx {
 
 namespace {
 
-// The ring from 2 MB on: 4 MB of fresh memory 0.41 -> 0.23 ms, but 1 MB into
-// memory already touched lost 30 us to the threads.  Larger chunks as the copy
-// grows: a chunk's fixed cost against the time until the first one has arrived
-// (16 MB: 0.61 ms in chunks of 2 MB, 0.82 in 512 KB; 512 MB: 11.8 ms in 4 MB,
-// 13.3 in 2 MB).
-constexpr size_t kFrom = (size_t)2 << 20;
+// Larger chunks as the copy grows: a chunk's fixed cost (17 us) against the
+// time until the first one has arrived (512 MB: 11.8 ms in 4 MB, 13.3 in 2 MB;
+// a served run of 60^3 with 6.9 MB of fields 1.29 ms in 1 MB, 1.78 in 512 KB).
 size_t chunk_bytes(size_t total) {
-  return total >= (size_t)64 << 20 ? (size_t)4 << 20 : total >= (size_t)8 << 20 ? (size_t)2 << 20 : (size_t)512 << 10;
+  return total >= (size_t)64 << 20 ? (size_t)4 << 20 : total >= (size_t)8 << 20 ? (size_t)2 << 20 : (size_t)1 << 20;
 }
 // Copying threads, the caller included: four fill fresh memory as fast as the
 // link (two reach 26 GB/s); for a few chunks more than two cost their start.

@@ -14,9 +14,15 @@ namespace lbx {
 // runtime's own staging (10 GB/s into fresh memory, 17 GB/s into touched
 // memory; the link moves 57 GB/s).  Here the link fills a ring of pinned
 // chunks and a few threads empty it: 512 MB of fresh memory 50.5 -> 11.8 ms,
-// 64 MB 6.4 -> 1.8 ms, 16 MB 1.6 -> 0.6 ms, 4 MB 0.41 -> 0.23 ms.
+// 64 MB 6.4 -> 1.8 ms, 16 MB 1.6 -> 0.6 ms.
 class ReadBack {
  public:
+  // The ring from 3.5 MB on: below, the threads' start costs what they bring.  Us
+  // into memory already touched, directly and so: 3.5 MB 206 and 226 (in chunks
+  // of 512 KB), 3.8 MB 221 and 190, 4.5 MB 283 and 224, 6.9 MB 390 and 288, 8.4
+  // MB 481 and 317; one served run of 48^3 with its fields (3.5 MB) 810 and 1090,
+  // of 52^3 (4.5 MB) 1100 and 989, of 60^3 (6.9 MB) 1306 and 1290.
+  static constexpr size_t kFrom = (size_t)7 << 19;
   struct Part {
     void* dst;
     const void* src;

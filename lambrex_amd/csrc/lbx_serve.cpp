@@ -575,7 +575,7 @@ int collect(lbx_server* s, bool wait) {
     // The run's last state is complete and stays until its arena space is
     // released: larger outputs go by a stream of their own, beside the steps
     // already queued for the other runs (small ones lose 20 us by it).
-    const hipStream_t out = n * 4 * sizeof(double) >= ((size_t)2 << 20) ? s->out : s->stream;
+    const hipStream_t out = n * 4 * sizeof(double) >= lbx::ReadBack::kFrom ? s->out : s->stream;
     if (rq.out_rho || rq.out_u) {
       SRV_HIP(s, lbx::launch_hydro(s->precision, false, fin, L, R, s->staging, s->staging + n, s->rho0, out));
       lbx::ReadBack::Part parts[2];

@@ -1,4 +1,4 @@
-"""The library's host code where the device runs out of memory, on a stand-in
+"""The library's host code on failing allocations and in its copies, on a stand-in
 HIP runtime (tests/cpp/fake_hip.cpp) in a process of its own: no GPU."""
 import subprocess
 import sys
@@ -52,4 +52,20 @@ def test_a_level_whose_allocation_fails_is_not_defined():
             assert fake.fake_launches(b"k_fine_step") == (4 if old else 1), failures
             sim.close()
         assert failures >= 8, failures
+    """)
+
+
+def test_small_read_backs_are_direct():
+    """A level's fields of 2.2 and 3.5 MB (41^3, 48^3) come in two copies, those of
+    4 MB and more in chunks of 1 MB: below, the threads that empty the chunks
+    cost what they bring."""
+    run("""
+    for dims, chunks in (((41, 41, 41), 2), ((48, 48, 48), 2), ((50, 50, 50), 4), ((60, 60, 60), 7), ((64, 64, 64), 4)):
+        sim = lbx.Sim(ctx, dims)
+        sim.define_level(0, [((0, 0, 0), tuple(d - 1 for d in dims))])
+        fake.fake_reset()
+        sim.hydro_level(0)
+        n = fake.fake_copies_to_host()
+        assert n == chunks, (dims, n)
+        sim.close()
     """)
