@@ -555,6 +555,13 @@ constexpr int kTagGroups = 1024;       // and the workgroups it cuts z for
 // Cells from which a tile pays: k_tag against it, 32^3 6.4 and 8.8 us (FP32
 // 6.8 and 8.2), 48^3 13.4 and 10.7 (9.7 and 8.2).
 constexpr long long kTagTiled = 64000;
+// ... and its lanes per cell, rings and idle ones counted, up to which it does.
+// Whole calls, k_tag against the tiles, in us: 192x160x128 (1.5) 2.8 times the
+// kernel's time; 64^3 (3.8) 57 and 55, 4 rows of 1000x1000 (4.6) 667 and 554
+// (FP32 499 and 460), 32x32x400 (6) 80 and 72 (61 and 62), 8x256x256 (7) 92 and
+// 91 (76 and 78), 3x600x600 (13) 209 and 275, 4x1000x1000 (10) 614 and 1350,
+// 1x256x256 (57) 35 and 59.
+constexpr int kTagLanes = 6;
 
 // ErrorEst on device data: tag[c] = 1 (c = (z*ny + y)*nx + x) where
 // CRIT 0: |grad rho|^2 > thr2, central differences with periodic wrap;
@@ -1000,14 +1007,15 @@ static void tag_launch(int criterion, const S* f, const Lattice& L, double rho0,
                 int blocks, hipStream_t st) {
   if (criterion == 1)
     return k_tag<S, 1, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
-  if ((long long)L.nx * L.ny * L.nz < kTagTiled)
-    return k_tag<S, 0, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
+  const long long cells = (long long)L.nx * L.ny * L.nz;
   const int tx = (L.nx + kTagX - 3) / (kTagX - 2), ty = (L.ny + kTagY - 3) / (kTagY - 2);
   const long long columns = (long long)tx * ty;
   const long long want = columns * L.nz / kTagGroups;  // planes per workgroup that leave kTagGroups of them
   const int depth = want < 2 ? 2 : want > 32 ? 32 : (int)want;
-  const int tz = (L.nz + depth - 1) / depth;
-  const int groups = tx * ty * tz;
+  const long long tz = (L.nz + depth - 1) / depth;
+  if (cells < kTagTiled || columns * (L.nz + 2 * tz) * (kTagX * kTagY) > kTagLanes * cells)
+    return k_tag<S, 0, PULL><<<blocks, 256, 0, st>>>(f, L, rho0, thr2, tag);
+  const int groups = int(columns * tz);
   k_tag_gradient<S, PULL><<<(groups + 7) / 8 * 8, dim3(kTagX, kTagY), 0, st>>>(f, L, rho0, thr2, tx, ty, groups, depth,
                                                                               tag);
 }
