@@ -293,12 +293,13 @@ void reject_refined(lbx_server* s, Run& r, int rc) {
 
 // Two passes at once (k_serve_pair): the column of cells of a run's work
 // items, the one that covers its x-y plane in the fewest, rows whole or in
-// pieces of whole cache lines.
+// pieces of 32 cells and more: pieces of 16 straddle the lines (33 rows of 16 on
+// 97^3 5.4 us a plane, 4 whole rows 3.1).
 void pair_column(Run& r) {
   const int nx = r.r.req.dims[0], ny = r.r.req.dims[1];
   long long best = -1;
   for (int bx = std::min(nx, 208); bx >= 1; --bx) {
-    if (bx != nx && bx % 16) continue;
+    if (bx != nx && (bx % 16 || bx < 32)) continue;
     const int rows = lbx::kServePairCells / (bx + 2) - 2;
     if (rows < 1) continue;
     const long long tx = (nx + bx - 1) / bx, ty = (ny + rows - 1) / rows;
@@ -334,20 +335,48 @@ int pair_depth(const lbx_server* s) {
   return best_depth;
 }
 
+// The time of a launch of two steps: rounds of items over the CUs x planes an
+// item walks (its own, the ring's two and one to start) x the time of a plane,
+// which is less in columns of whole rows.
+double pair_us(const lbx_server* s, int depth) {
+  long long items = 0;
+  double sum = 0.0, longest = 0.0;
+  for (const Run& r : s->active) {
+    if (r.sim || r.launched_last) continue;
+    const int nx = r.r.req.dims[0], nz = r.r.req.dims[2], chunks = (nz + depth - 1) / depth;
+    const bool whole = r.bx == nx && nx >= 32;
+    const double plane_us = s->precision == LBX_FP64 ? whole ? 4.2 : 4.8 : whole ? 2.9 : 3.4;
+    const double us = plane_us * ((nz + chunks - 1) / chunks + 3);
+    items += r.columns * chunks;
+    sum += us * double(r.columns * chunks);
+    longest = std::max(longest, us);
+  }
+  return items ? std::max(longest, double((items + s->cus - 1) / s->cus) * sum / double(items)) : 0.0;
+}
+
 // Whether the next launch advances the active runs by two steps: enough cells
-// (kPairCells), in lattices whose columns keep most lanes busy (a cube's do to
-// 2/3 and more; a row of cells is better off as 256 cells per item).
+// (kPairCells), and a shorter time than two launches of one step, which take 7
+// us and the state at 5.4 TB/s (FP32 5.0; 4.7 and 4.5 with rows that are no
+// multiple of 4 cells).  The constants are fitted to batches of 1 to 44 runs of
+// 44 shapes, 0.7 to 8.6 M cells: of 230 the rule takes the slower of the two for
+// 8, by 9 % at most.  Us per step, one and two at a time: FP32 97^3 27.4 and
+// 24.4, 2 of 80^3 28.6 and 31.5, 5 of 80^3 61 and 58, 23 of 300x300x4 189 and
+// 220; FP64 2 of 80^3 47.8 and 47.9, 3 of 200x200x8 46.0 and 49.7, 25 of them 355
+// and 287.
 bool pairs_pay(const lbx_server* s) {
-  long long cells = 0, lanes = 0;
+  long long cells = 0;
+  double single_us = 7.0;
   bool more = false;
   for (const Run& r : s->active) {
     if (r.launched_last) continue;
     more |= r.sim ? r.r.req.steps - r.steps_done > 1 : r.r.req.steps + 1 - r.passes > 1;
     if (r.sim) continue;
     cells += r.cells;
-    lanes += r.columns * lbx::kServePairCells * r.r.req.dims[2];
+    const bool even = r.r.req.dims[0] % 4 == 0;
+    const double tbs = s->precision == LBX_FP64 ? even ? 5.4 : 4.7 : even ? 5.0 : 4.5;
+    single_us += double(r.cells) * 2 * lbx::NV_TOTAL * (double)esize(s->precision) / (tbs * 1e6);
   }
-  return more && cells >= kPairCells && lanes <= 2 * cells;
+  return more && cells >= kPairCells && pair_us(s, pair_depth(s)) < 2 * single_us;
 }
 
 // Admission: move queued requests into the active set while they fit, in

@@ -1,4 +1,4 @@
-"""The library's host code on failing allocations and in its copies, on a stand-in
+"""The library's host code on failing allocations, its copies and launches, on a stand-in
 HIP runtime (tests/cpp/fake_hip.cpp) in a process of its own: no GPU."""
 import subprocess
 import sys
@@ -68,4 +68,26 @@ def test_small_read_backs_are_direct():
         n = fake.fake_copies_to_host()
         assert n == chunks, (dims, n)
         sim.close()
+    """)
+
+
+def test_served_batches_take_the_faster_launch():
+    """Batches of served runs for which two launches of one step are the faster
+    take no launch of two, and the other way round."""
+    run("""
+    cases = [(lbx.LBX_FP32_SHIFTED, (80, 80, 80), 2, False), (lbx.LBX_FP32_SHIFTED, (200, 200, 8), 3, False),
+             (lbx.LBX_FP32_SHIFTED, (300, 300, 4), 23, False), (lbx.LBX_FP64, (200, 200, 8), 3, False),
+             (lbx.LBX_FP64, (8, 8, 3000), 14, False), (lbx.LBX_FP32_SHIFTED, (97, 97, 97), 1, True),
+             (lbx.LBX_FP32_SHIFTED, (130, 130, 30), 5, True), (lbx.LBX_FP64, (200, 200, 8), 25, True),
+             (lbx.LBX_FP64, (161, 33, 47), 11, True), (lbx.LBX_FP32_SHIFTED, (32, 32, 32), 30, True)]
+    for precision, dims, runs, pairs in cases:
+        srv = lbx.Server(ctx, precision=precision, arena_bytes=3 << 30)
+        for _ in range(runs):
+            srv.submit(dims, 5, 0.7)
+        fake.fake_reset()
+        srv.drain()
+        assert len(srv.poll()) == runs
+        srv.close()
+        assert (fake.fake_launches(b"k_serve_pair") > 0) == pairs, (precision, dims, runs)
+        assert fake.fake_launches(b"k_serve_step") == (0 if pairs else 6), (precision, dims, runs)
     """)
