@@ -100,6 +100,7 @@ struct Level {
   std::vector<std::pair<int, int>> groups;  // (first position in gdesc, count)
   lbx::FineTile* d_tiles[2] = {nullptr, nullptr};  // as the finest level; with a finer one, planned with that
   int ntiles[2] = {0, 0};
+  int tile_cells[2] = {0, 0};
   double* d_avg = nullptr;       // 15 planes of avg_stride 2x2x2 block averages
   long long avg_stride = 0;
   int max_blocks = 0;            // largest (g/2)^3 of a patch
@@ -516,6 +517,7 @@ lbx::FineStep fine_step_args(const lbx_sim* sim, int l, bool finest, bool averag
   a.own = L.d_gdesc;
   a.tiles = L.d_tiles[finest ? 0 : 1];
   a.ntiles = L.ntiles[finest ? 0 : 1];
+  a.cells = L.tile_cells[finest ? 0 : 1];
   a.fill = (const unsigned long long*)L.d_fill;
   a.strides = L.d_strides;
   a.parent_stride = P.patched ? P.gdesc[0].qs : P.lat.ps;
@@ -863,19 +865,17 @@ std::vector<unsigned char> patch_mask(const Level& C, const std::vector<Box>& ma
 // The k-th of n even-aligned parts of [0, g) (g even), as even as they can be.
 int part_begin(int g, int n, int k) { return 2 * (int)((long long)(g / 2) * k / n); }
 
-// Cuts patches into tiles for launch_fine_step.  Every patch is cut into parts
-// of at most `want` cells per direction (4 or more, in z 2: on a small level the
-// planes a workgroup walks are all the time, 24^3 with a 16-wide level 42 -> 37
-// us a step); the target that costs least is taken:
-// rounds of workgroups over the CUs x planes a workgroup walks (its own and
-// up to 4 around them, and 2 of the pipeline) x time of a plane (2.5 us + 0.4
-// us, in FP32 0.2, per wave of its A plane).  The model only ranks the targets:
-// of a sweep that forced each of them on 36^3 and 28^3 patches in FP64, none was
-// faster than the one it takes by more than the runs differed; in FP32 0.4 a
-// wave takes smaller tiles and is slower (64^3 with a 32x128x128 level 72 us a
-// step, 68 so; three levels over 32^3 152 and 138).
-std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int elem_bytes, bool finest) {
-  const int room = lbx::fine_tile_cells(elem_bytes, finest);
+// Cuts patches into tiles for launch_fine_step, and says in *room which of its
+// kernels they are for (FineStep::cells).  Every patch is cut into parts of at
+// most `want` cells per direction (4 or more, in z 2: on a small level the planes
+// a workgroup walks are all the time, 24^3 with a 16-wide level 42 -> 37 us a
+// step); the target and kernel that cost least are taken: rounds of workgroups
+// over the CUs x planes a workgroup walks (its own and up to 4 around them, and 2
+// of the pipeline) x relative time of a plane (plane_time).  The model only ranks
+// them.  Of all the targets and both kernels forced on levels of 16x16x16,
+// 32x64x64 and 64x128x128 in boxes of 2 to 32 as the finest, none was faster than
+// the one it takes by more than 4 % in FP64 and 1 % in FP32.
+std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int elem_bytes, bool finest, int* room) {
   std::map<std::tuple<int, int, int>, int> shapes;  // grown extents -> patches
   int gmax[3] = {2, 2, 2};
   for (const PatchDesc& p : patches) {
@@ -894,15 +894,27 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   int best[3] = {4, 4, gmax[2]};
-  double best_us = 1e300;
-  auto targets = [](int g, int least) {
+  double least = 1e300;
+  const int large = lbx::fine_tile_cells(elem_bytes, finest);
+  std::vector<int> rooms{lbx::kFineSmall};
+  if (large > lbx::kFineSmall) rooms.push_back(large);
+  *room = lbx::kFineSmall;
+  // of `waves` waves of the kernel with r cells, `resident` workgroups to a CU
+  auto plane_time = [&](int r, int waves, long long resident) {
+    if (!finest && elem_bytes == 8) return 1.0 + 0.16 * waves;
+    const double alone = 1.0 + (finest ? 0.04 : 0.02) * waves;
+    if (r > lbx::kFineSmall) return alone * (finest ? 1.1 : 1.0);
+    return alone * (1.0 + (finest ? 0.3 : 0.15) * double(resident - 1) /
+                              (lbx::fine_tile_groups(elem_bytes, finest, r) - 1));
+  };
+  auto targets = [](int g, int fewest) {
     std::vector<int> t;
     for (int n = 1; n <= 64; ++n) {
       const int want = ((g + n - 1) / n + 1) / 2 * 2;
-      if (want >= least && (t.empty() || t.back() != want)) t.push_back(want);
+      if (want >= fewest && (t.empty() || t.back() != want)) t.push_back(want);
     }
     if (t.empty()) t.push_back(g);
-    if (t.back() > least) t.push_back(least);
+    if (t.back() > fewest) t.push_back(fewest);
     return t;
   };
   const std::vector<int> tx = targets(gmax[0], 4), ty = targets(gmax[1], 4), tz = targets(gmax[2], 2);
@@ -916,8 +928,7 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
         cells = std::max(cells, widest(gx, nx) * widest(gy, ny));
         columns += (long long)nx * ny * s.second;
       }
-      if (cells > room || columns > (1 << 24)) continue;
-      const double plane_us = 2.5 + (elem_bytes == 8 ? 0.4 : 0.2) * ((cells + 63) / 64);
+      if (cells > rooms.back() || columns > (1 << 24)) continue;
       for (int wz : tz) {
         long long n = 0;
         int planes = 0;
@@ -926,13 +937,19 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
           n += (long long)parts(std::get<0>(s.first), wx) * parts(std::get<1>(s.first), wy) * nz * s.second;
           planes = std::max(planes, widest(gz, nz) + 2);
         }
-        const long long slots = room <= 256 ? 2 * cus : cus;  // workgroups of 4 waves: two to a CU
-        const double us = (double)((n + slots - 1) / slots) * planes * plane_us;
-        if (n < (1 << 24) && us < best_us) {
-          best_us = us;
-          best[0] = wx;
-          best[1] = wy;
-          best[2] = wz;
+        for (int r : rooms) {
+          if (cells > r || n >= (1 << 24)) continue;
+          const long long groups = lbx::fine_tile_groups(elem_bytes, finest, r), slots = groups * cus;
+          const double cost = (double)((n + slots - 1) / slots) * planes *
+                              plane_time(r, (cells + 63) / 64, std::min(groups, (n + cus - 1) / cus));
+          // of equal ones the shorter walk
+          if (cost < least || (cost == least && r == *room && wx == best[0] && wy == best[1])) {
+            least = cost;
+            best[0] = wx;
+            best[1] = wy;
+            best[2] = wz;
+            *room = r;
+          }
         }
       }
     }
@@ -960,7 +977,8 @@ std::vector<lbx::FineTile> plan_tiles(const std::vector<PatchDesc>& patches, int
 // Plans and uploads a level's tiles for its steps as the finest or a middle
 // level; returns when they have arrived.
 hipError_t set_tiles(lbx_sim* sim, Level& L, bool finest) {
-  const std::vector<lbx::FineTile> t = plan_tiles(L.gdesc, (int)elem_size(sim->precision), finest);
+  int* cells = &L.tile_cells[finest ? 0 : 1];
+  const std::vector<lbx::FineTile> t = plan_tiles(L.gdesc, (int)elem_size(sim->precision), finest, cells);
   L.ntiles[finest ? 0 : 1] = (int)t.size();
   return upload(&L.d_tiles[finest ? 0 : 1], t, sim->ctx->stream);
 }

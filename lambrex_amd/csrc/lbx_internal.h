@@ -229,9 +229,18 @@ struct FineTile {
 // 2294; the finest level loses by it, 549 -> 639 us for 128^3 with a 64x256x256
 // level).  In FP32 the finest level does with 168 and so takes 12 waves (360 ->
 // 306 us for that hierarchy); a middle level spills there, and two workgroups
-// of 4 are slower (370 -> 398 us for three levels over 64^3).
+// of 4 are slower (370 -> 398 us for three levels over 64^3).  Small patches
+// leave most of so many lanes idle: a level cut into tiles of at most kFineSmall
+// cells may run workgroups of that many lanes, several to a CU.  Us per step of a
+// 64x128x128 level in boxes of 8, large and small: FP64 378 and 266, FP32 315 and
+// 166; a 32x64x64 level in boxes of 4 200 and 117, 183 and 87.
+constexpr int kFineSmall = 256;
 constexpr int fine_tile_cells(int elem_bytes, bool finest) {
-  return elem_bytes == 8 ? finest ? 512 : 256 : finest ? 768 : 512;
+  return elem_bytes == 8 ? finest ? 512 : kFineSmall : finest ? 768 : 512;
+}
+// Workgroups of `cells` cells to a CU.
+constexpr int fine_tile_groups(int elem_bytes, bool finest, int cells) {
+  return cells > kFineSmall ? 1 : elem_bytes == 4 && finest ? 3 : 2;
 }
 
 constexpr unsigned long long kFillParent = 1ull << 63, kFillElement = (1ull << 40) - 1;
@@ -249,6 +258,7 @@ struct FineStep {
   const PatchDesc* own;        // the level's patches in launch order
   const FineTile* tiles;
   int ntiles;
+  int cells;                   // of a tile's plane at most: kFineSmall or fine_tile_cells
   // Per ghost cell of the level: the element of population 0 of its source,
   // in the parent's state with kFillParent, else in the level's; the source's
   // population stride is strides[bits from kFillStrideShift], or with strides

@@ -366,8 +366,8 @@ __device__ constexpr int lateral(int q) { return (kC[q][1] + 1) * 3 + kC[q][0] +
 // First of the populations that share (c_x, c_y): 1 to 4, then 5, 7, 9, 11, 13.
 __device__ constexpr int pull_first(int c) { return c < 4 ? c + 1 : 2 * c - 3; }
 
-template <typename S, bool FINEST, bool MASK, bool SUM, bool AVG>
-__global__ __launch_bounds__(fine_tile_cells(sizeof(S), FINEST)) void k_fine_step(
+template <typename S, bool FINEST, bool MASK, bool SUM, bool AVG, int CELLS>
+__global__ __launch_bounds__(CELLS) void k_fine_step(
     const S* __restrict__ fnow, S* __restrict__ fnext, const S* __restrict__ cnow,
     const PatchDesc* __restrict__ own, const FineTile* __restrict__ tiles, int ntiles,
     const unsigned long long* __restrict__ fill, const unsigned* __restrict__ strides, long long parent_stride,
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(fine_tile_cells(sizeof(S), FINEST)) void k_fine_ste
     const int* __restrict__ contrib) {
   // plane A of population q, then plane B of it
   constexpr int kSets = FINEST ? 2 : 1;
-  constexpr int kFineCells = fine_tile_cells(sizeof(S), FINEST);
+  constexpr int kFineCells = CELLS;
   __shared__ S planes[NV - 1][kSets][kFineCells];
   constexpr int kB = kSets - 1;
   constexpr int kCut1 = 5, kCut2 = 10;
@@ -992,25 +992,29 @@ hipError_t launch_fine_stream_zero(int precision, const void* in, void* out, con
   return hipGetLastError();
 }
 
-template <typename S>
-static hipError_t fine_step(const FineStep& a, dim3 grid, hipStream_t st) {
-#define LBX_FINE_STEP(FINEST, MIDDLE, AVG)                                                                     \
-  k_fine_step<S, FINEST, MIDDLE, MIDDLE, AVG><<<grid, fine_tile_cells(sizeof(S), FINEST), 0, st>>>( \
-      (const S*)a.now, (S*)a.next, (const S*)a.parent, a.own, a.tiles, a.ntiles, a.fill, a.strides,             \
-      a.parent_stride, a.mask, a.relax, a.avg, a.avg_stride, a.spans, a.cavg, a.cavg_stride, a.contrib)
-  if (a.finest)
-    LBX_FINE_STEP(true, false, true);
-  else if (a.avg)
-    LBX_FINE_STEP(false, true, true);
-  else
-    LBX_FINE_STEP(false, true, false);
-#undef LBX_FINE_STEP
+template <typename S, bool FINEST, bool AVG, int CELLS>
+static hipError_t fine_step(const FineStep& a, hipStream_t st) {
+  k_fine_step<S, FINEST, !FINEST, !FINEST, AVG, CELLS><<<(a.ntiles + 7) / 8 * 8, CELLS, 0, st>>>(
+      (const S*)a.now, (S*)a.next, (const S*)a.parent, a.own, a.tiles, a.ntiles, a.fill, a.strides, a.parent_stride,
+      a.mask, a.relax, a.avg, a.avg_stride, a.spans, a.cavg, a.cavg_stride, a.contrib);
   return hipGetLastError();
 }
 
+template <typename S, int CELLS>
+static hipError_t fine_step(const FineStep& a, hipStream_t st) {
+  if (a.finest) return fine_step<S, true, true, CELLS>(a, st);
+  return a.avg ? fine_step<S, false, true, CELLS>(a, st) : fine_step<S, false, false, CELLS>(a, st);
+}
+
 hipError_t launch_fine_step(int precision, const FineStep& a, hipStream_t st) {
-  const dim3 grid((a.ntiles + 7) / 8 * 8);
-  return precision == 0 ? fine_step<double>(a, grid, st) : fine_step<float>(a, grid, st);
+  if (a.cells == kFineSmall)
+    return precision == 0 ? fine_step<double, kFineSmall>(a, st) : fine_step<float, kFineSmall>(a, st);
+  if (a.finest)
+    return precision == 0 ? fine_step<double, true, true, fine_tile_cells(8, true)>(a, st)
+                          : fine_step<float, true, true, fine_tile_cells(4, true)>(a, st);
+  if (precision == 0) return hipErrorInvalidValue;
+  return a.avg ? fine_step<float, false, true, fine_tile_cells(4, false)>(a, st)
+               : fine_step<float, false, false, fine_tile_cells(4, false)>(a, st);
 }
 
 hipError_t launch_fine_stream_collide(int precision, const void* in, void* out,

@@ -91,3 +91,30 @@ def test_served_batches_take_the_faster_launch():
         assert (fake.fake_launches(b"k_serve_pair") > 0) == pairs, (precision, dims, runs)
         assert fake.fake_launches(b"k_serve_step") == (0 if pairs else 6), (precision, dims, runs)
     """)
+
+
+def test_refined_levels_take_the_kernel_for_their_boxes():
+    """Small boxes run workgroups of 256 lanes, several to a CU, where the large
+    kernels would leave most of their lanes idle."""
+    run(f"""
+    sys.path.insert(0, {str(ROOT / 'tests')!r})
+    from fine_kernels import CASES
+    from lambrex_amd import workloads
+    for name, (dims, refined, lanes) in CASES.items():
+        for precision, letter in ((lbx.LBX_FP64, "d"), (lbx.LBX_FP32_SHIFTED, "f")):
+            sim = lbx.Sim(ctx, dims, precision=precision)
+            sim.define_level(0, workloads.chop(dims, 32))
+            for l, boxes in enumerate(refined):
+                sim.define_level(l + 1, boxes)
+            for l in range(len(refined) + 1):
+                sim.set_tau(l, 0.8)
+            fake.fake_reset()
+            sim.iterate(1)
+            for role, flag in (("finest", 1), ("middle", 0)):
+                for n in (256, 512, 768):
+                    ran = sum(fake.fake_launches(f"k_fine_stepI{{letter}}Lb{{flag}}{{m}}Lb{{avg}}ELi{{n}}E".encode())
+                              for m in ("ELb0ELb0E", "ELb1ELb1E") for avg in (0, 1))
+                    want = role in lanes and lanes[role][precision] == n
+                    assert (ran > 0) == want, (name, letter, role, n, ran)
+            sim.close()
+    """)
