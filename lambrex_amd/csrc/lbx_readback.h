@@ -17,12 +17,11 @@ namespace lbx {
 // 64 MB 6.4 -> 1.8 ms, 16 MB 1.6 -> 0.6 ms.
 class ReadBack {
  public:
-  // The ring from 3.5 MB on: below, the threads' start costs what they bring.  Us
-  // into memory already touched, directly and so: 3.5 MB 206 and 226 (in chunks
-  // of 512 KB), 3.8 MB 221 and 190, 4.5 MB 283 and 224, 6.9 MB 390 and 288, 8.4
-  // MB 481 and 317; one served run of 48^3 with its fields (3.5 MB) 810 and 1090,
-  // of 52^3 (4.5 MB) 1100 and 989, of 60^3 (6.9 MB) 1306 and 1290.
-  static constexpr size_t kFrom = (size_t)7 << 19;
+  // The ring from 2 MB on: below, the threads' start costs what they bring.  Us
+  // into memory already touched, directly and so: 2.2 MB 142 and 120, 3.5 MB 219
+  // and 194, 4.5 MB 282 and 235, 6.9 MB 405 and 289, 8.4 MB 481 and 317; 1 MB
+  // would lose 30.
+  static constexpr size_t kFrom = (size_t)2 << 20;
   struct Part {
     void* dst;
     const void* src;

@@ -55,12 +55,12 @@ def test_a_level_whose_allocation_fails_is_not_defined():
     """)
 
 
-def test_small_read_backs_are_direct():
-    """A level's fields of 2.2 and 3.5 MB (41^3, 48^3) come in two copies, those of
-    4 MB and more in chunks of 1 MB: below, the threads that empty the chunks
-    cost what they bring."""
+def test_read_backs_come_in_few_chunks():
+    """A level's fields below 2 MB (40^3) come in two copies, above in chunks of 1
+    MB and from 8 MB on (64^3) of 2 MB: smaller ones leave the threads that empty
+    them waiting for the next."""
     run("""
-    for dims, chunks in (((41, 41, 41), 2), ((48, 48, 48), 2), ((50, 50, 50), 4), ((60, 60, 60), 7), ((64, 64, 64), 4)):
+    for dims, chunks in (((40, 40, 40), 2), ((41, 41, 41), 3), ((48, 48, 48), 4), ((60, 60, 60), 7), ((64, 64, 64), 4)):
         sim = lbx.Sim(ctx, dims)
         sim.define_level(0, [((0, 0, 0), tuple(d - 1 for d in dims))])
         fake.fake_reset()
