@@ -823,14 +823,20 @@ static int compute_units() {
 // single passes).  Of 15 shapes swept at 16^3 to 40^3 and 10x10x50 these are
 // the fastest: 4x4x4 of 3 steps at 24^3 (3.15 us, the 2-step blocks 3.2 and
 // more), 8x4x4 of 2 at 32^3 (3.6; 4x4x8 of 3 steps 4.0), 8x8x4 at 40^3.  In FP32
-// two blocks of 6x6x6 share a CU (48^3 5.3 us a step in single passes, 4.7 so).
+// two blocks of 6x6x6 may share a CU, which then takes 4.7 us a step whatever the
+// lattice, and 0.5 more with walls: from 90000 cells on less than single passes or
+// the same (48^3 5.1 and 4.7 us, with walls 5.2 and 5.2, 36x36x72 5.0 and 4.6,
+// 60x60x30 4.9 and 5.0), below more (64x36x36 4.5 and 4.9, 199x15x30 4.8 and 5.4,
+// 90x15x63 between walls 4.9 and 5.4).  One to a CU 103x10x41 4.2 and 4.1,
+// 11x369x11 4.2 and 3.6.
+constexpr long long kBlockShared = 90000;
 BlockShape block_shape(const Lattice& L, int precision) {
-  // steps, cells of a block, blocks per CU
+  // steps, cells of a block, blocks per CU at most
   static constexpr int kShapes[4][5] = {{3, 4, 4, 4, 1}, {2, 8, 4, 4, 1}, {2, 8, 8, 4, 1}, {2, 6, 6, 6, 2}};
   const long long n[3] = {L.nx, L.ny, L.nz};
   for (const int(&c)[5] : kShapes) {
-    const long long room = (long long)c[4] * compute_units();
     if (c[4] > 1 && precision == 0) continue;
+    const long long room = (n[0] * n[1] * n[2] < kBlockShared ? 1 : c[4]) * (long long)compute_units();
     BlockShape b{};
     b.steps = c[0];
     long long blocks = 1;

@@ -118,3 +118,21 @@ def test_refined_levels_take_the_kernel_for_their_boxes():
                     assert (ran > 0) == want, (name, letter, role, n, ran)
             sim.close()
     """)
+
+
+def test_small_fp32_lattices_take_the_faster_pass():
+    """Blocks of 6x6x6 cells, two to a CU, only where single passes take longer."""
+    run("""
+    cases = [((90, 15, 63), (1, 1, 0), False), ((494, 25, 5), (0, 1, 1), False), ((199, 15, 30), (1, 1, 1), False),
+             ((64, 36, 36), (1, 1, 1), False), ((48, 48, 48), (0, 0, 0), True), ((48, 48, 48), (1, 1, 1), True),
+             ((36, 36, 72), (1, 1, 1), True), ((11, 369, 11), (1, 1, 1), True), ((257, 28, 5), (0, 0, 0), True)]
+    for dims, periodic, blocks in cases:
+        sim = lbx.Sim(ctx, dims, precision=lbx.LBX_FP32_SHIFTED, periodic=periodic)
+        sim.define_level(0, [((0, 0, 0), tuple(d - 1 for d in dims))])
+        sim.set_tau(0, 0.8)
+        sim.iterate(1)
+        fake.fake_reset()
+        sim.iterate(6)
+        assert fake.fake_launches(b"k_step_block") == (3 if blocks else 0), (dims, periodic)
+        sim.close()
+    """)
