@@ -136,3 +136,23 @@ def test_small_fp32_lattices_take_the_faster_pass():
         assert fake.fake_launches(b"k_step_block") == (3 if blocks else 0), (dims, periodic)
         sim.close()
     """)
+
+
+def test_lattices_run_each_two_step_kernel():
+    """The lattices of tests/pair_paths.py take the kernels they are listed for."""
+    run(f"""
+    sys.path.insert(0, {str(ROOT / 'tests')!r})
+    from pair_paths import CASES
+    for dims, periodic, precision, column in CASES:
+        sim = lbx.Sim(ctx, dims, precision=precision, periodic=periodic)
+        sim.define_level(0, [((0, 0, 0), tuple(d - 1 for d in dims))])
+        sim.set_tau(0, 0.8)
+        sim.iterate(1)
+        fake.fake_reset()
+        sim.iterate(4)
+        walls = 0 if all(periodic) else 1
+        for b in (0, 32, 64):
+            part = f"k_step_pairI{{'df'[precision]}}Li{{b}}ELi{{(0, 16, 8)[(0, 32, 64).index(b)]}}ELb{{walls}}E"
+            assert fake.fake_launches(part.encode()) == (2 if b == column else 0), (dims, precision, b)
+        sim.close()
+    """)
