@@ -103,7 +103,9 @@ def measure(ctx, dims, mgs, tau, rho, u, precision, steps, warmup, keep_fields=F
     storage = "double" if precision == lbx.LBX_FP64 else "float"
     wall_arg = "" if all(periodic) else ", walls"
     if launches and 2 * launches <= steps + 1 and steps > 1:
-        name = "k_step_block" if cells <= 110592 else "k_step_pair"  # blocks of at most 432 cells per CU
+        # several steps per launch: three only in blocks, and no lattice of more than 432 cells per CU in blocks
+        name = ("k_step_block" if 5 * launches < 2 * steps else
+                "k_step_pair" if cells > 110592 else "k_step_block or k_step_pair")
         kernel = f"{name}<{storage}{wall_arg}>"
     else:
         kernel = f"k_step_{'f64' if precision == lbx.LBX_FP64 else 'f32s'}<STEP_FUSED{wall_arg}>"
@@ -468,7 +470,8 @@ def main():
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--no-copy", action="store_true", help="skip the copy-bandwidth ceiling")
     ap.add_argument("--autotune", action="store_true",
-                    help="time every workgroup shape first and use the fastest (default: the default shape)")
+                    help="time every workgroup shape of one-step launches first and use the fastest "
+                         "(default: the default shape)")
     ap.add_argument("--copy-only", action="store_true",
                     help="only run the copy kernel (counter calibration)")
     ap.add_argument("--clock-warmup-ms", type=float, default=CLOCK_WARMUP_MS,
@@ -651,7 +654,7 @@ def main():
         "config": {"workload": workload, "cells": cells, "boxes": r64["boxes"], "tau": tau,
                    "seed": seed, "precision": "FP64",
                    "workgroup": {"bx": shape64[0], "by": shape64[1], "max_workgroups_per_cu": shape64[2],
-                                 "autotuned": bool(args.autotune)}},
+                                 "autotuned": bool(args.autotune), "applies_to": "launches of one step"}},
         "roofline": {
             "bound": "hbm",
             "achieved": round(r64["kernel_gbs"], 1),
@@ -680,7 +683,8 @@ def main():
                          "kernel": r32["kernel"], "updates_per_launch": r32["updates_per_launch"],
                          "kernel_avg_ms": round(r32["kernel_avg_ms"], 5),
                          "algorithmic_bytes_per_launch": BYTES_PER_LU[lbx.LBX_FP32_SHIFTED] * cells},
-            "workgroup": {"bx": shape32[0], "by": shape32[1], "max_workgroups_per_cu": shape32[2]},
+            "workgroup": {"bx": shape32[0], "by": shape32[1], "max_workgroups_per_cu": shape32[2],
+                          "applies_to": "launches of one step"},
             "max_rel_rho_err_vs_fp64": r32["max_rel_rho_err_vs_fp64"],
             "max_du_over_max_u_vs_fp64": r32["max_du_over_max_u_vs_fp64"],
         }

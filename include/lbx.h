@@ -234,11 +234,14 @@ int lbx_profile_read(lbx_ctx* ctx, double* ms, int64_t* launches);
  * (0 = none, else 1 to 6; enforced by reserving LDS the kernel does not use).
  * While enabled, the first launch for a new (nx, ny, precision) times every
  * candidate on a small proxy lattice with the same rows and keeps the
- * fastest for the context's lifetime; shapes never change results.  Passes
- * that advance several steps in one launch have a shape of their own.  No
- * reference counterpart.  lbx_tuned_shape reports the shape launches of
- * that geometry use: the tuned choice and its time per proxy launch, or the
- * default shape (time 0) if the geometry was never tuned. */
+ * fastest for the context's lifetime; shapes never change results.  It is the
+ * shape of the passes of one step: most lattices advance by launches of two
+ * or three steps, whose columns or blocks the library picks and no tuning
+ * changes, so there it holds for the collide-only pass of a new state and for
+ * the step that an odd count leaves.  No reference counterpart.
+ * lbx_tuned_shape reports the shape one-step launches of that geometry use:
+ * the tuned choice and its time per proxy launch, or the default shape (time
+ * 0) if the geometry was never tuned. */
 int lbx_set_autotune(lbx_ctx* ctx, int enable);
 int lbx_tuned_shape(lbx_ctx* ctx, int nx, int ny, int precision, int32_t* bx, int32_t* by,
                     int32_t* wg_per_cu, float* ms_per_launch);

@@ -346,7 +346,8 @@ struct ProfileScope {
 // a proxy lattice with the same rows (nx, ny) and a few z-planes; the
 // fastest is kept for that (nx, ny, precision).  Shapes change only which
 // lanes compute which cells, never the arithmetic, so results do not depend
-// on the choice.
+// on the choice.  Launches of several steps (pair_shape, block_shape) have
+// shapes of their own.
 std::vector<LaunchShape> shape_candidates(const Lattice& L) {
   std::vector<LaunchShape> c;
   for (int lanes : {256, 512}) {

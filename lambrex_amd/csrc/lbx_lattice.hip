@@ -69,8 +69,7 @@ __device__ constexpr int opposite(int q) {
 // Pull with halfway bounce-back: population q of cell (x, y, z) comes from
 // x - c_q, unless that crosses a wall face (an axis with its bit in
 // L.walls), where the cell's own opposite population, which left towards
-// the wall, returns instead.  Periodic axes wrap as in load_cell.  ONCE: no
-// other workgroup reads the same elements (non-temporal loads).
+// the wall, returns instead.  Periodic axes wrap as in load_cell.
 template <typename S>
 __device__ __forceinline__ void load_cell_walls(const S* __restrict__ src, const Lattice& L, int x, int y,
                                                 int z, long long selfz, int selfp, const Upstream& u, S* f) {
@@ -165,9 +164,9 @@ __global__ __launch_bounds__(512) void k_step_f32s(const float* __restrict__ src
 // a contiguous range of columns) and, with one workgroup of 11 waves per CU
 // (LDS, and ~150 VGPRs in FP64), the part of the collisions that the loads
 // do not cover; in FP32 the vector units are busy 90 % of the time.
-// Measured (us per step, single pass -> pair): 256^3 FP64 652 -> 397, FP32
-// 328 -> 208 (5.2 and 5.0 TB/s, of a copy's 6.5); 128^3 FP64 88 -> 57, FP32
-// 42.5 -> 30.  FP64 409 and FP32 219 with the next plane's loads waited for
+// Measured (us per step, single pass -> pair): 256^3 FP64 652 -> 389, FP32
+// 328 -> 206 (5.2 and 4.9 TB/s, of a copy's 6.5); 128^3 FP64 88 -> 57, FP32
+// 42.5 -> 29.  FP64 408 and FP32 216 with the next plane's loads waited for
 // before the second step.  Slower: 32 x 8 and 64 x 4 columns with two
 // workgroups per CU, separate waves for the two steps, non-temporal loads (the
 // ring misses L2); in FP32 32 x 16 (221), 64 x 12 (229), 128 x 5 (226) and 64 x
@@ -853,9 +852,12 @@ BlockShape block_shape(const Lattice& L, int precision) {
 // Shape of the two-step pass for a lattice, or none (tx = 0) where two single
 // passes are the faster.  Every workgroup count that fills the device for one
 // or more rounds is a candidate: rounds x (planes of a workgroup + 2 of the
-// ring + 1 to start) x the time of a plane, measured as 6.8 us (FP64) and 4.1
-// us (FP32) at 256^3 and 4.4 and 2.8 us where both buffers stay in the 256 MB
-// MALL.  A single pass is taken at 5.3 TB/s.  At 64^3 the rule takes the pair
+// ring + 1 to start) x the time of a plane, taken as 6.8 us (FP64) and 4.1 us
+// (FP32), and 4.4 and 2.8 us where both buffers stay in the 256 MB MALL.  A
+// single pass is taken at 5.3 TB/s.  These place the line between the two and
+// are no figures of the kernel, which takes 5.9 and 3.1 us a plane at 256^3 and
+// 128^3 alike: of 150 drawn lattices of each type none that takes the pair is
+// the slower for it.  At 64^3 the rule takes the pair
 // in FP64 (10.2 against 12.4 us a step) and not in FP32 (6.9 against 5.9); at
 // 48^3 in neither (7.1 against 6.4, 5.6 against 4.7); at 96x80x72 in both (18.5
 // against 25.7, 12.2 against 12.9).

@@ -200,7 +200,8 @@ long long cells_of(const lbx_request& q) { return (long long)q.dims[0] * q.dims[
 // and their flag bytes, four buffers of grown fine patches (2 ghost layers,
 // population stride rounded to 64) with their fill table, mask bytes and
 // block averages, and the parent's touched-cell slots; 1/8 more for the
-// smaller tables.
+// smaller tables.  A level holds less: three such buffers above ratio 2, two of
+// valid cells alone at ratio 2.
 size_t refined_bytes_estimate(const Request& q, int precision) {
   const lbx::Lattice L = lbx::make_lattice(q.req.dims[0], q.req.dims[1], q.req.dims[2], (int)esize(precision));
   const long long coarse_cells = (long long)L.nx * L.ny * L.nz;

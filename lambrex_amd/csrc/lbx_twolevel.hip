@@ -883,11 +883,11 @@ __global__ __launch_bounds__(256) void k_fine_remake(S* __restrict__ fnew, const
   for (int q = 0; q < NV; ++q) fnew[to + q * P.qs] = from[q * stride];
 }
 
-// Valid cells of one patch <-> packed FP64 f [15][nz][ny][nx]; hydro of one
-// patch.
-template <int OP, typename S>  // 0 pack, 1 unpack, 2 hydro
+// Valid cells of one patch <-> packed FP64 f [15][nz][ny][nx].
+template <int OP, typename S>  // 0 pack, 1 unpack
 __global__ __launch_bounds__(256) void k_patch_io(S* __restrict__ f, const PatchDesc* __restrict__ patches, int b,
                                                   double* __restrict__ a, double rho0) {
+  static_assert(OP == 0 || OP == 1);
   const PatchDesc P = patches[b];
   const int nx = P.hi[0] - P.lo[0] + 1, ny = P.hi[1] - P.lo[1] + 1, nz = P.hi[2] - P.lo[2] + 1;
   const int n = nx * ny * nz;

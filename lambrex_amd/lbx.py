@@ -177,8 +177,8 @@ class Context:
         self.check(self._lib.lbx_set_autotune(self.h, 1 if on else 0))
 
     def tuned_shape(self, nx, ny, precision=LBX_FP64):
-        """((bx, by, workgroups_per_cu_cap), ms per proxy launch) that launches over
-        rows of nx x ny use: the autotuner's choice, or the default shape (ms 0)
+        """((bx, by, workgroups_per_cu_cap), ms per proxy launch) that one-step launches
+        over rows of nx x ny use: the autotuner's choice, or the default shape (ms 0)
         if that geometry was never tuned."""
         bx, by, occ, ms = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32(), ctypes.c_float()
         self.check(self._lib.lbx_tuned_shape(self.h, int(nx), int(ny), int(precision), ctypes.byref(bx),
